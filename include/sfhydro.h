@@ -164,7 +164,8 @@ int sfh_correct(sfh_ocean ocean, double Fdq[3], double Tdq[3], double Fdf[3], do
  * GPU (held until the process ends), sized for meshes of at most 524,288
  * faces; a larger mesh returns SFH_ERR_SIZE.  It calls
  * no hipMalloc, hipFree or allocating routine.  Every call on one GPU shares
- * that array: calls that overlap on one GPU (several streams or threads)
+ * that array (a chunk counter, zero between calls, and the chunks' partial
+ * sums): calls that overlap on one GPU (several streams or threads)
  * race, so the caller orders them.  mesh must not be NULL. */
 int sfh_forces_noalloc(const sfh_settings* settings, int mode, sfh_mesh mesh, sfh_ocean ocean,
                        const double* d_state, double* d_out, void* stream);
@@ -201,6 +202,11 @@ typedef struct {
     uint32_t split_passes;    /* 0: one face launch runs the submerged and the crossing
                                  chunks; 1: a launch for each, each at its own occupancy */
 } sfh_batch_opts;
+/* With split_passes 0 a batch of at most 1,024 chunks (of bodies that all have
+ * faces, 8 or 16 faces per lane, not compounds) runs its whole step in one
+ * launch, a workgroup per chunk; `waves` then has no effect, and both times of
+ * sfh_batch_kernel_ms are that launch's.  The rows are the same bits either
+ * way. */
 
 /* Replaces the per-body pool fan-out of SimulationManager::SimulationTickCallback
  * (SimulationManager.cpp:1619-1655) + Ocean::ApplyFluidForces (Ocean.cpp:219-268)

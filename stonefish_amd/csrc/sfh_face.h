@@ -169,22 +169,11 @@ SFH_HD void face_submerged(const FaceBody& B, f3 p1, f3 p2, f3 p3, AccT& acc)
 // quadratic-drag slot; there is no skin friction.  The wind (the atmosphere's
 // velocity fields) is sampled at the centroid as for the currents.
 #define SFH_GLM_VEC3_LENGTH 3.0f
-template <class Flow, class AccT>
-SFH_HD void face_aero(const FaceBody& B, f3 p1, f3 p2, f3 p3, const Flow& flow, AccT& acc)
+template <bool ON, class AccT>
+SFH_HD void aero_drag(const FaceBody& B, f3 c, f3 n1, float A, f3 uf, AccT& acc)
 {
-    f3 e1 = p2 - p1, e2 = p3 - p1;
-    f3 n = cross(e1, e2);
-    float n2 = dot(n, n);
-    if (n2 < SFH_DEGENERATE_N2) return;
-    float inv = frsq(n2);
-    f3 n1 = n * inv;
-    float A = 0.5f * (n2 * inv);
-    f3 c = p1 + (e1 + e2) * (1.0f / 3.0f);
     f3 vm = B.vb + cross(B.w, c);
-    if (Flow::on)
-        vm = vm - flow(((double)p1.x + (double)p2.x + (double)p3.x) / 3.0,
-                       ((double)p1.y + (double)p2.y + (double)p3.y) / 3.0,
-                       ((double)p1.z + (double)p2.z + (double)p3.z) / 3.0);
+    if (ON) vm = vm - uf;
     float s = dot(vm, n1);
     if (s > -SFH_APPROACH_VN) {
         f3 q = n1 * (-(s * SFH_GLM_VEC3_LENGTH * A));
@@ -193,11 +182,29 @@ SFH_HD void face_aero(const FaceBody& B, f3 p1, f3 p2, f3 p3, const Flow& flow, 
     }
 }
 
+template <class Flow, class AccT>
+SFH_HD void face_aero(const FaceBody& B, f3 p1, f3 p2, f3 p3, const Flow& flow, AccT& acc)
+{
+    f3 e1 = p2 - p1, e2 = p3 - p1;
+    f3 n = cross(e1, e2);
+    float n2 = dot(n, n);
+    if (n2 < SFH_DEGENERATE_N2) return;
+    float inv = frsq(n2);
+    f3 c = p1 + (e1 + e2) * (1.0f / 3.0f);
+    f3 uf = mk3(0.f, 0.f, 0.f);
+    if (Flow::on)
+        uf = flow(((double)p1.x + (double)p2.x + (double)p3.x) / 3.0, ((double)p1.y + (double)p2.y + (double)p3.y) / 3.0,
+                  ((double)p1.z + (double)p2.z + (double)p3.z) / 3.0);
+    aero_drag<Flow::on>(B, c, n * inv, 0.5f * (n2 * inv), uf, acc);
+}
+
 // Result of clipping one face against the waterline: the wet polygon as a
 // base vertex plus an offset to its centroid, its unit normal and area, and
 // whether the face contributes.
 struct Wet {
     f3 base, off;   // centroid = base + off
+    f3 cs;          // off = cs * ck: the sum of the polygon's offsets from base, one over their number
+    float ck;
     f3 n1;
     float A;
     bool ok;
@@ -326,10 +333,13 @@ SFH_HD Wet face_clip(const FaceBody& B, f3 p1, f3 p2, f3 p3, float d0, float d1,
         f3 n34 = cross(fv3, fv4);
         r.A = 0.5f * (len + fsqrt(dot(n34, n34)));
         r.off = csum * 0.25f;
+        r.ck = 0.25f;
     } else {
         r.A = 0.5f * len;
         r.off = csum * (1.0f / 3.0f);
+        r.ck = 1.0f / 3.0f;
     }
+    r.cs = csum;
     r.ok = true;
     return r;
 }
@@ -355,6 +365,8 @@ SFH_HD Wet face_allwet(const FaceBody& B, f3 p1, f3 p2, f3 p3, Acc<T>& acc)
     r.base = base;
     r.A = 0.5f * len;
     r.off = csum * (1.0f / 3.0f);
+    r.cs = csum;
+    r.ck = 1.0f / 3.0f;
     r.ok = true;
     return r;
 }

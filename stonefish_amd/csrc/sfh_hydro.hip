@@ -2,8 +2,9 @@
 // hydrodynamics (SolidEntity.cpp:1239-1850, Ocean.cpp:149-201,
 // OpenGLRealOcean.cpp:280-331, Compound-free body path).
 //
-// One evaluation pass over a batch of bodies is three launches on one stream
-// (four for compounds):
+// One evaluation pass over a small batch of bodies, or of one body, is one
+// launch (k_step, k_step_one); over a larger batch it is three launches on one
+// stream (four for compounds):
 //   k_prologue  eight lanes per body, FP64: C transform, body/fluid
 //               classification (8 AABB corners against the surface), per-body
 //               FP32 constants of the face loop in the mesh frame, FP64
@@ -462,32 +463,21 @@ static constexpr int kPrologueLanes = 8;
 __device__ void epilogue_finish(const BodyStatic& S, const BodyDyn& D, const OceanK& oc, const double* P,
                                 double* __restrict__ o);
 
-// Body b on its group of kPrologueLanes lanes (`sub` is the lane's index in
-// the group); returns the body's position for this step (-2: left out).
-__device__ __forceinline__ int prologue_body(const BodyStatic* __restrict__ st, const double* __restrict__ states,
-                                             int state_kind, const OceanK& oc, const uint8_t* __restrict__ active,
-                                             const uint32_t* __restrict__ sidx, BodyDyn* __restrict__ dyn,
-                                             int8_t* __restrict__ bpos, double* __restrict__ out, uint32_t b, int sub)
+// One body on a group of kPrologueLanes lanes (`sub` is the lane's index in the
+// group): its record dd for this step and, with `rows`, the row o of a body
+// without face work.  s: the body's state (its row of the state array).
+// Returns the body's position for this step.
+__device__ __forceinline__ int prologue_body(const BodyStatic& S, const double* s, int state_kind, const OceanK& oc,
+                                             BodyDyn* __restrict__ dd, bool rows, double* __restrict__ o, int sub)
 {
-    const BodyStatic& S = st[b];
-    // A body the step skips is marked in bpos only: its static record and its
-    // BodyDyn row are not touched (the later passes test bpos, and the
-    // compound pass returns first for an inactive compound, whose parts share
-    // its activity).
-    if (active && !active[sidx[b]]) {
-        if (sub == 0) bpos[b] = -2;
-        return -2;
-    }
     // The body's BodyDyn record is written by the group's lane 0 as its parts
     // are computed (a record held whole until one store at the end keeps ~1 KB
     // live in registers); the wave layers below nlayers, and the currents'
     // table only when there are varying currents (cur.n says how many), so a
     // body on one layer without jets or pipes writes 360 of its 944 bytes.
     // D keeps what the finish of a body without faces reads.
-    BodyDyn* __restrict__ dd = dyn + b;
     const bool w0 = sub == 0;
     BodyDyn D;
-    const double* s = states + (size_t)S.sidx * (state_kind ? 38 : 22);
     double Rcg[9], tcg[3], R[9], tc[3];
     gl_basis(s, Rcg);
     tcg[0] = s[12]; tcg[1] = s[13]; tcg[2] = s[14];
@@ -533,7 +523,6 @@ __device__ __forceinline__ int prologue_body(const BodyStatic* __restrict__ st, 
     D.pos = pos;
     D.flags = flags;
     if (w0) {
-        bpos[b] = (int8_t)pos;
         dd->pos = pos;
         dd->flags = flags;
         dd->cpos = D.cpos;
@@ -601,7 +590,7 @@ __device__ __forceinline__ int prologue_body(const BodyStatic* __restrict__ st, 
         for (int i = 0; i < 3; ++i) dd->tcg[i] = tcg[i];
     }
 
-    double* o = out + (size_t)b * SFH_OUT_DOUBLES;
+    if (!rows) return pos;
     if (pos == -1) {          // not a hydrodynamic body: nothing assigned
         if (sub == 0) { o[20] = 0.0; o[21] = -1.0; }
     } else if (pos == 0) {    // OUTSIDE: everything zero (SolidEntity.cpp:1810-1821)
@@ -674,21 +663,32 @@ __device__ __forceinline__ void list_append(uint32_t* __restrict__ list, uint32_
 
 // Every lane of the grid reaches the list build (lanes past the last body
 // contribute nothing), so the scans see whole wavefronts and workgroups.
-// The prologue of the bodies of one workgroup of BLOCK threads (gt: the
-// thread's index in the grid); every thread of the workgroup calls it (the
-// list build's barriers).
 template <int BLOCK>
-__device__ __forceinline__ void prologue_group(const BodyStatic* __restrict__ st, const double* __restrict__ states,
-                                               int state_kind, uint32_t n, const OceanK& oc,
-                                               const uint8_t* __restrict__ active, const uint32_t* __restrict__ sidx,
-                                               BodyDyn* __restrict__ dyn, int8_t* __restrict__ bpos,
-                                               double* __restrict__ out, uint32_t* __restrict__ list, uint32_t nc,
-                                               uint32_t* __restrict__ counts, uint32_t gt)
+__global__ __launch_bounds__(BLOCK) void k_prologue(const BodyStatic* __restrict__ st,
+                                                    const double* __restrict__ states, uint32_t n, OceanK oc,
+                                                    const uint8_t* __restrict__ active,
+                                                    const uint32_t* __restrict__ sidx, BodyDyn* __restrict__ dyn,
+                                                    int8_t* __restrict__ bpos, double* __restrict__ out,
+                                                    uint32_t* __restrict__ list, uint32_t nc,
+                                                    uint32_t* __restrict__ counts)
 {
+    const uint32_t gt = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t b = gt / kPrologueLanes;
     const int sub = (int)(gt % kPrologueLanes);
     int pos = -3;
-    if (b < n) pos = prologue_body(st, states, state_kind, oc, active, sidx, dyn, bpos, out, b, sub);
+    // A body the step skips is marked in bpos only: its static record and its
+    // BodyDyn row are not touched (the later passes test bpos, and the
+    // compound pass returns first for an inactive compound, whose parts share
+    // its activity).
+    if (b < n) {
+        pos = -2;
+        if (!active || active[sidx[b]]) {
+            const BodyStatic& S = st[b];
+            pos = prologue_body(S, states + (size_t)S.sidx * SFH_STATE_DOUBLES, 0, oc, dyn + b, true,
+                                out + (size_t)b * SFH_OUT_DOUBLES, sub);
+        }
+        if (sub == 0) bpos[b] = (int8_t)pos;
+    }
     uint32_t c_sub = 0, c_cross = 0, chunk0 = 0;
     if (pos == 1 || pos == 2) {
         chunk0 = st[b].chunk0;
@@ -696,17 +696,6 @@ __device__ __forceinline__ void prologue_group(const BodyStatic* __restrict__ st
         else c_cross = st[b].nchunks;
     }
     list_append<BLOCK>(list, counts, nc, c_sub, c_cross, chunk0, sub);
-}
-
-template <int BLOCK>
-__global__ __launch_bounds__(BLOCK) void k_prologue(const BodyStatic* __restrict__ st, const double* __restrict__ states, int state_kind,
-                           uint32_t n, OceanK oc, const uint8_t* __restrict__ active,
-                           const uint32_t* __restrict__ sidx, BodyDyn* __restrict__ dyn,
-                           int8_t* __restrict__ bpos, double* __restrict__ out, uint32_t* __restrict__ list,
-                           uint32_t nc, uint32_t* __restrict__ counts)
-{
-    prologue_group<BLOCK>(st, states, state_kind, n, oc, active, sidx, dyn, bpos, out, list, nc, counts,
-                          blockIdx.x * blockDim.x + threadIdx.x);
 }
 
 // Jets and pipes at a mesh-frame point (Jet.cpp:54-75, Pipe.cpp:57-78): the
@@ -757,7 +746,8 @@ struct CurFlow {
 struct Chunk {
     uint32_t body, first, count;
     uint32_t vlo, vn;
-    uint32_t pad[3];
+    uint32_t sidx;      // BodyStatic::sidx of the body
+    uint32_t pad[2];
 };
 
 // Vertex-window capacity (vertices) of a crossing-pass wavefront for chunks
@@ -1081,35 +1071,44 @@ __device__ __forceinline__ void cross_chunk(uint32_t c, uint32_t f0, uint32_t nf
 
 // CorrectHydrodynamicForces (SolidEntity.cpp:1263-1287): M = inverse(basis of
 // T_O) by cofactors (btMatrix3x3.h:1093-1103); safeNormalize (btVector3.h:286-299).
-__device__ void correct64(double rho, const double* BO, const double* Cd, const double* Cf,
-                          double* Fdq, double* Tdq, double* Fdf, double* Tdf)
+__device__ __forceinline__ void correct_inverse(const double* BO, double* M)
 {
 #pragma clang fp contract(on)   // FMAs only within an expression: the same rounding wherever this is inlined
 #define CF(r1, c1, r2, c2) (BO[3 * (r1) + (c1)] * BO[3 * (r2) + (c2)] - BO[3 * (r1) + (c2)] * BO[3 * (r2) + (c1)])
     double co0 = CF(1, 1, 2, 2), co1 = CF(1, 2, 2, 0), co2 = CF(1, 0, 2, 1);
     double det = BO[0] * co0 + BO[1] * co1 + BO[2] * co2;
     double s = 1.0 / det;
-    double M[9] = {co0 * s, CF(0, 2, 2, 1) * s, CF(0, 1, 1, 2) * s,
-                   co1 * s, CF(0, 0, 2, 2) * s, CF(0, 2, 1, 0) * s,
-                   co2 * s, CF(0, 1, 2, 0) * s, CF(0, 0, 1, 1) * s};
+    M[0] = co0 * s; M[1] = CF(0, 2, 2, 1) * s; M[2] = CF(0, 1, 1, 2) * s;
+    M[3] = co1 * s; M[4] = CF(0, 0, 2, 2) * s; M[5] = CF(0, 2, 1, 0) * s;
+    M[6] = co2 * s; M[7] = CF(0, 1, 2, 0) * s; M[8] = CF(0, 0, 1, 1) * s;
 #undef CF
-    double* vecs[4] = {Fdq, Tdq, Fdf, Tdf};
-    for (int q = 0; q < 4; ++q) {
-        double* x = vecs[q];
-        double d[3];
-        mat_vec(M, x, d);
-        double l2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
-        if (l2 >= 2.220446049250313e-16 * 2.220446049250313e-16) {
-            double inv = 1.0 / sqrt(l2);   // btVector3::operator/= multiplies by the reciprocal
-            d[0] *= inv; d[1] *= inv; d[2] *= inv;
-        } else {
-            d[0] = 1.0; d[1] = 0.0; d[2] = 0.0;
-        }
-        const double* C = (q < 2) ? Cd : Cf;
-        double c = fabs(d[0]) * C[0] + fabs(d[1]) * C[1] + fabs(d[2]) * C[2];
-        double k = (q < 2) ? 0.5 * rho * c : rho * c;
-        x[0] *= k; x[1] *= k; x[2] *= k;
+}
+
+// One vector of the correction: quadratic drag with C = Cd, skin friction with C = Cf.
+__device__ __forceinline__ void correct_vector(double rho, const double* M, const double* C, bool quadratic, double* x)
+{
+#pragma clang fp contract(on)   // FMAs only within an expression: the same rounding wherever this is inlined
+    double d[3];
+    mat_vec(M, x, d);
+    double l2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
+    if (l2 >= 2.220446049250313e-16 * 2.220446049250313e-16) {
+        double inv = 1.0 / sqrt(l2);   // btVector3::operator/= multiplies by the reciprocal
+        d[0] *= inv; d[1] *= inv; d[2] *= inv;
+    } else {
+        d[0] = 1.0; d[1] = 0.0; d[2] = 0.0;
     }
+    double c = fabs(d[0]) * C[0] + fabs(d[1]) * C[1] + fabs(d[2]) * C[2];
+    double k = quadratic ? 0.5 * rho * c : rho * c;
+    x[0] *= k; x[1] *= k; x[2] *= k;
+}
+
+__device__ void correct64(double rho, const double* BO, const double* Cd, const double* Cf,
+                          double* Fdq, double* Tdq, double* Fdf, double* Tdf)
+{
+    double M[9];
+    correct_inverse(BO, M);
+    double* vecs[4] = {Fdq, Tdq, Fdf, Tdf};
+    for (int q = 0; q < 4; ++q) correct_vector(rho, M, (q < 2) ? Cd : Cf, q < 2, vecs[q]);
 }
 
 // CorrectAerodynamicForces (SolidEntity.cpp:1925-1948): d = safeNormalize(
@@ -1140,52 +1139,44 @@ __device__ void correct_aero64(uint32_t type, const double* params, const double
     for (int k = 0; k < 3; ++k) { F[k] *= cor; T[k] *= cor; }
 }
 
-// Finishes the row o of a body in position 1 or 2 from the sums P of its
-// chunk partials (one lane): drag in world axes with moments about the CoG,
-// buoyancy, CorrectHydrodynamicForces, the write mask.
-__device__ void epilogue_finish(const BodyStatic& S, const BodyDyn& D, const OceanK& oc, const double* P,
-                                double* __restrict__ o)
+// The parts of a row's finish (epilogue_finish on one lane, finish_lanes on
+// several).  Drag vector q (Fdq Tdq Fdf Tdf): world = R * F_local; torque =
+// R * (M_local + dt x F_local).
+__device__ __forceinline__ void finish_drag(const BodyDyn& D, const double* P, int q, double* x)
 {
 #pragma clang fp contract(on)   // FMAs only within an expression: the same rounding wherever this is inlined
-    const int pos = D.pos;
+    const double* F = P + 6 * (q >> 1);
+    const double* M = F + 3;
+    double t[3], m[3];
+    cross64(D.dt, F, t);
+    for (int k = 0; k < 3; ++k) m[k] = (q & 1) ? M[k] + t[k] : F[k];
+    mat_vec(D.R, m, x);
+}
+
+// Basis of T_O.
+__device__ __forceinline__ void finish_basis(const BodyStatic& S, const BodyDyn& D, double* BO)
+{
+#pragma clang fp contract(on)   // FMAs only within an expression: the same rounding wherever this is inlined
+    for (int i = 0; i < 3; ++i)
+        for (int j = 0; j < 3; ++j)
+            BO[3 * i + j] = D.Rcg[3 * i] * S.cg2o[j] + D.Rcg[3 * i + 1] * S.cg2o[3 + j] + D.Rcg[3 * i + 2] * S.cg2o[6 + j];
+}
+
+// Buoyancy, wetted area and submerged volume; returns the write mask.
+__device__ __forceinline__ uint32_t finish_buoyancy(const BodyStatic& S, const BodyDyn& D, const OceanK& oc,
+                                                    const double* P, double* Fb, double* Tb, double& Swet,
+                                                    double& Vsub)
+{
+#pragma clang fp contract(on)   // FMAs only within an expression: the same rounding wherever this is inlined
     const uint32_t flags = D.flags;
     const bool body_level = !(flags & (BF_MODE_SURF | BF_MODE_SUBM | BF_MODE_AERO));
     const bool damping = flags & BF_DAMPING;
     const bool buoyant = flags & BF_BUOYANT;
     uint32_t written = 0;
-    // drag: world = R * F_local; torque = R * (M_local + dt x F_local)
-    double drag[12];
-    for (int q = 0; q < 2; ++q) {
-        const double* F = P + 6 * q;
-        const double* M = P + 6 * q + 3;
-        double t[3], m[3];
-        cross64(D.dt, F, t);
-        for (int k = 0; k < 3; ++k) m[k] = M[k] + t[k];
-        mat_vec(D.R, F, drag + 6 * q);
-        mat_vec(D.R, m, drag + 6 * q + 3);
-    }
-    double* Fdq = drag;
-    double* Tdq = drag + 3;
-    double* Fdf = drag + 6;
-    double* Tdf = drag + 9;
-    if (flags & BF_MODE_AERO) {   // Fda, Tda = 0.5 rho_gas times the sums (SolidEntity.cpp:1915-1917)
-        double Fa[3], Ta[3];
-        for (int k = 0; k < 3; ++k) {
-            Fa[k] = 0.5 * oc.rho * Fdq[k];
-            Ta[k] = 0.5 * oc.rho * Tdq[k];
-        }
-        if (flags & BF_AERO_CORRECT) correct_aero64((flags >> BF_APPROX_SHIFT) & 3u, S.Cd, S.cg2o, Fa, Ta);
-        for (int k = 0; k < 3; ++k) {
-            o[6 + k] = Fa[k];
-            o[9 + k] = Ta[k];
-        }
-        o[20] = (double)(4u | 8u);   // written: the quadratic-drag slots
-        o[21] = (double)pos;
-        return;
-    }
-    double Fb[3] = {0, 0, 0}, Tb[3] = {0, 0, 0};
-    double Swet = 0.0, Vsub = 0.0;
-    if (pos == 1) {
+    for (int k = 0; k < 3; ++k) Fb[k] = Tb[k] = 0.0;
+    Swet = 0.0;
+    Vsub = 0.0;
+    if (D.pos == 1) {
         if (body_level && !(flags & BF_PART)) {
             if (buoyant) {   // analytic buoyancy of a submerged body (1828-1836)
                 double cb[3];
@@ -1225,11 +1216,46 @@ __device__ void epilogue_finish(const BodyStatic& S, const BodyDyn& D, const Oce
         Swet = P[22];
         written |= 64u;
     }
+    return written;
+}
+
+// Finishes the row o of a body in position 1 or 2 from the sums P of its
+// chunk partials (one lane): drag in world axes with moments about the CoG,
+// buoyancy, CorrectHydrodynamicForces, the write mask.
+__device__ void epilogue_finish(const BodyStatic& S, const BodyDyn& D, const OceanK& oc, const double* P,
+                                double* __restrict__ o)
+{
+#pragma clang fp contract(on)   // FMAs only within an expression: the same rounding wherever this is inlined
+    const int pos = D.pos;
+    const uint32_t flags = D.flags;
+    const bool body_level = !(flags & (BF_MODE_SURF | BF_MODE_SUBM | BF_MODE_AERO));
+    const bool damping = flags & BF_DAMPING;
+    double drag[12];
+    for (int q = 0; q < 4; ++q) finish_drag(D, P, q, drag + 3 * q);
+    double* Fdq = drag;
+    double* Tdq = drag + 3;
+    double* Fdf = drag + 6;
+    double* Tdf = drag + 9;
+    if (flags & BF_MODE_AERO) {   // Fda, Tda = 0.5 rho_gas times the sums (SolidEntity.cpp:1915-1917)
+        double Fa[3], Ta[3];
+        for (int k = 0; k < 3; ++k) {
+            Fa[k] = 0.5 * oc.rho * Fdq[k];
+            Ta[k] = 0.5 * oc.rho * Tdq[k];
+        }
+        if (flags & BF_AERO_CORRECT) correct_aero64((flags >> BF_APPROX_SHIFT) & 3u, S.Cd, S.cg2o, Fa, Ta);
+        for (int k = 0; k < 3; ++k) {
+            o[6 + k] = Fa[k];
+            o[9 + k] = Ta[k];
+        }
+        o[20] = (double)(4u | 8u);   // written: the quadratic-drag slots
+        o[21] = (double)pos;
+        return;
+    }
+    double Fb[3], Tb[3], Swet, Vsub;
+    const uint32_t written = finish_buoyancy(S, D, oc, P, Fb, Tb, Swet, Vsub);
     if (body_level && damping) {
         double BO[9];
-        for (int i = 0; i < 3; ++i)
-            for (int j = 0; j < 3; ++j)
-                BO[3 * i + j] = D.Rcg[3 * i] * S.cg2o[j] + D.Rcg[3 * i + 1] * S.cg2o[3 + j] + D.Rcg[3 * i + 2] * S.cg2o[6 + j];
+        finish_basis(S, D, BO);
         correct64(oc.rho, BO, S.Cd, S.Cf, Fdq, Tdq, Fdf, Tdf);
     }
     if (written & 1u) for (int k = 0; k < 3; ++k) o[k] = Fb[k];
@@ -1248,16 +1274,25 @@ __device__ void epilogue_finish(const BodyStatic& S, const BodyDyn& D, const Oce
 // the body's chunks, a transposed reduction across the wavefront (a fixed
 // order, so the sums do not depend on which wavefront runs this) leaves the
 // 23 totals on 23 lanes, which store them to `ps` (24 doubles of LDS).
+// AGENT: the partials were written in this launch (k_step): agent-scope loads.
+template <bool AGENT>
 __device__ void epilogue_sums(const BodyStatic& S, const double* partials, double* ps, int lane)
 {
     double v[24];
 #pragma unroll
     for (int k = 0; k < 24; ++k) v[k] = 0.0;
     for (uint32_t c = lane; c < S.nchunks; c += 64) {
-        const double2* p = (const double2*)(partials + (size_t)(S.chunk0 + c) * kChunkDoubles);
+        const double* q = partials + (size_t)(S.chunk0 + c) * kChunkDoubles;
+        const double2* p = (const double2*)q;
 #pragma unroll
         for (int k = 0; k < 12; ++k) {
-            const double2 x = p[k];
+            double2 x;
+            if (AGENT) {
+                x.x = __hip_atomic_load(q + 2 * k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                x.y = __hip_atomic_load(q + 2 * k + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            } else {
+                x = p[k];
+            }
             v[2 * k] += x.x;
             v[2 * k + 1] += x.y;
         }
@@ -1328,7 +1363,7 @@ __global__ __launch_bounds__(64 * kEpilogueWaves, 4) void k_epilogue(
             const uint32_t k = (uint32_t)__builtin_ctzll(m);
             m &= m - 1ull;
             const uint32_t b = base + k * W;
-            epilogue_sums(st[b], partials, ps[wl][nb], lane);
+            epilogue_sums<false>(st[b], partials, ps[wl][nb], lane);
             if (nb == 0) first = b;
             if (lane == nb) mine = b;
             if (++nb == kEpilogueBatch || !m) {
@@ -1407,6 +1442,530 @@ __global__ __launch_bounds__(256, NU ? 1 : ((PASS & kPassCross) ? 5 : 8)) void k
                 cross_chunk<K, NU, NL, false>(c, f0, nfc, vlo, vn, S, D, oc, wq, ldep[wl], cutq[wl], partials, lane);
         }
     }
+}
+
+// ---------------------------------------------------------------------------
+// k_step: the whole step of a small batch (or of one body) in one launch
+// ---------------------------------------------------------------------------
+
+// A step of few chunks is bound by latency: the launches it waits for (three,
+// each with its start and drain) and, inside the face pass, one wavefront's
+// serial walk over its chunk with nothing beside it to hide a load.  Here a
+// workgroup of four wavefronts takes one chunk from the body's state to its
+// partial, and the workgroup that finishes a body's last chunk finishes its
+// row:
+//   1. the body's record and state into LDS;
+//   2. wavefront 0 runs the body's prologue (every chunk's workgroup its own;
+//      the record stays in LDS) while the others stage the chunk's vertices
+//      and its faces' window-relative vertex numbers in LDS and form every
+//      face's unit normal, area and centroid, which need no state;
+//   3. crossing chunks: the FP64 depths of the window, then per face whether
+//      it is wet, its tetra volume and its centroid's depth, over all four
+//      wavefronts;
+//   4. the sums, divided over the wavefronts by quantity (quadratic drag,
+//      skin friction, pressure buoyancy, volume and wetted area): lane l of
+//      each adds the faces l, l + 64, ... and then its cut faces in the order
+//      of k_faces from the staged terms, and the reduction over the lanes has
+//      the same tree, so the partials are those of k_faces bit for bit;
+//   5. a body of one chunk is finished at once; otherwise the chunk's partial
+//      goes to memory past the caches (agent-scope stores, waited for), the
+//      workgroup counts itself done on the body's counter, and the one that
+//      counts last sums the partials in chunk order and finishes the row.
+//      It also zeroes the counter for the next step.
+// Measured: a tick of 203 bodies (576 chunks, 60 % overlapped, two wave
+// layers) 39.4 -> 18.3 us, an aerodynamic batch of 300 bodies 16.5 -> 10.8 us,
+// the per-body calls 38 -> 32 us (2,070 faces, submerged) and 52 -> 43 us
+// (12,000 faces, surface), 13 us of which are the caller's Python.  Of the
+// tick's kernel 1.0 us are its loads, 2.9 the prologue, 4.3 the depths and the
+// wet faces' terms, 2.9 the sums and up to 2 the cut faces, 2.2 the partials'
+// way through memory, 1.5 the finish: chains of dependent loads and FP64
+// operations on one wavefront per SIMD.
+struct StepArgs {
+    const BodyStatic* st;
+    const Chunk* chunks;
+    const double* states;      // rows of 22 (kind 0) or 38 doubles (kind 1)
+    const uint8_t* active;     // per state row, or null
+    double* out;
+    double* applied;           // the tick driver's force and torque per row, or null
+    double* partials;
+    uint32_t* done;            // per body: chunks finished in this step
+    int kind;
+};
+
+__device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlane(x); }
+__device__ __forceinline__ float uni(float x) { return __int_as_float(uni(__float_as_int(x))); }
+__device__ __forceinline__ double uni(double x)
+{
+    return __hiloint2double(uni(__double2hiint(x)), uni(__double2loint(x)));
+}
+__device__ __forceinline__ f3 uni(f3 v) { return mk3(uni(v.x), uni(v.y), uni(v.z)); }
+
+template <int K, bool NU, bool AERO>
+struct StepShared {
+    // the vertex window (x, y, z, depth) and the faces' vertex numbers in it
+    float4 sv[AERO ? 1 : win_cap(K)];
+    ushort4 sf[AERO ? 1 : 64 * K];
+    float4 r0[64 * K];         // per face: unit normal, area (negative: the face adds nothing)
+    float4 r1[64 * K];         // per face: centroid, its depth
+    float v6[AERO ? 1 : 64 * K];
+    float uf[NU ? 3 : 1][NU ? 64 * K : 1];   // jets' and pipes' velocity at the centroid
+    uint16_t cutq[AERO ? 1 : 64 * K];
+    uint64_t cut[K];           // per row of 64 faces: the cut ones
+    BodyStatic S;
+    BodyDyn D;
+    double state[38];
+    double P[24];
+    int pos, wet;
+};
+
+// A chunk's faces: vertices (and depths) from the staged window, or from
+// memory for a chunk whose window is too large (whose crossing faces take
+// their vertices' depths one by one).
+struct StepFace {
+    f3 p1, p2, p3;
+    float d0, d1, d2;
+};
+
+template <int K, bool NU, int NL, bool AERO>
+struct StepFaces {
+    const StepShared<K, NU, AERO>& sh;
+    const SFH_GLOBAL float* verts;
+    const SFH_GLOBAL uint32_t* faces;
+    bool win;
+
+    __device__ __forceinline__ StepFace points(uint32_t f) const
+    {
+        StepFace q;
+        if (!AERO && win) {
+            const ushort4 k = sh.sf[f];
+            const float4 a = sh.sv[k.x], b = sh.sv[k.y], c = sh.sv[k.z];
+            q.p1 = mk3(a.x, a.y, a.z); q.p2 = mk3(b.x, b.y, b.z); q.p3 = mk3(c.x, c.y, c.z);
+            q.d0 = a.w; q.d1 = b.w; q.d2 = c.w;
+        } else {
+            const SFH_GLOBAL uint32_t* i = faces + 3 * (size_t)f;
+            q.p1 = vert(verts, i[0]); q.p2 = vert(verts, i[1]); q.p3 = vert(verts, i[2]);
+            q.d0 = q.d1 = q.d2 = 0.f;
+        }
+        return q;
+    }
+
+    __device__ __forceinline__ StepFace crossing(uint32_t f, const WaveQ<NL>& wq) const
+    {
+        StepFace q = points(f);
+        if (!win) {
+            const f3 zero = mk3(0.f, 0.f, 0.f);
+            q.d0 = (float)wq.depth(q.p1, zero);
+            q.d1 = (float)wq.depth(q.p2, zero);
+            q.d2 = (float)wq.depth(q.p3, zero);
+        }
+        return q;
+    }
+};
+
+// A wet polygon's centroid, rounded once (fused) or after the offset.
+template <bool FUSED>
+__device__ __forceinline__ f3 step_centroid(f3 base, f3 cs, float ck)
+{
+#pragma clang fp contract(off)
+    if (FUSED)
+        return mk3(__builtin_fmaf(cs.x, ck, base.x), __builtin_fmaf(cs.y, ck, base.y), __builtin_fmaf(cs.z, ck, base.z));
+    const float x = cs.x * ck, y = cs.y * ck, z = cs.z * ck;
+    return mk3(base.x + x, base.y + y, base.z + z);
+}
+
+// Transposed FP64 reduction of 6 per-lane values over the wavefront's lanes
+// (the tree of xreduce24): lane l with (2 b4 + b3) != 3 and b2 = b1 = b0 = 0
+// holds the total of quantity 3 b5 + 2 b4 + b3 in v[0].
+__device__ __forceinline__ void xreduce6(double (&v)[6], int lane)
+{
+    bool hi = lane & 32;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        double send = hi ? v[i] : v[i + 3], keep = hi ? v[i + 3] : v[i];
+        v[i] = keep + __shfl_xor(send, 32, 64);
+    }
+    v[3] = 0.0;
+    hi = lane & 16;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        double send = hi ? v[i] : v[i + 2], keep = hi ? v[i + 2] : v[i];
+        v[i] = keep + __shfl_xor(send, 16, 64);
+    }
+    hi = lane & 8;
+    {
+        double send = hi ? v[0] : v[1], keep = hi ? v[1] : v[0];
+        v[0] = keep + __shfl_xor(send, 8, 64);
+    }
+    v[0] += __shfl_xor(v[0], 4, 64);
+    v[0] += __shfl_xor(v[0], 2, 64);
+    v[0] += __shfl_xor(v[0], 1, 64);
+}
+
+__device__ __forceinline__ int xreduce6_slot(int lane)
+{
+    const int g = ((lane >> 3) & 1) + 2 * ((lane >> 4) & 1);
+    return (g == 3 || (lane & 7)) ? -1 : 3 * ((lane >> 5) & 1) + g;
+}
+
+// The sums of quantity group PART (0 quadratic or aerodynamic drag, 1 skin
+// friction, 2 pressure buoyancy, 3 volume and wetted area) over a chunk's
+// faces, on one wavefront.
+template <int K, bool NU, int NL, bool AERO, int PART>
+__device__ __forceinline__ void step_sums(const StepShared<K, NU, AERO>& sh, const StepFaces<K, NU, NL, AERO>& sf,
+                                          uint32_t nfc, const FaceBody& fb, const WaveQ<NL>& wq, bool crossing,
+                                          bool wave_buoy, bool damping, uint32_t ncut, int lane, double (&v)[6])
+{
+    constexpr bool CBON = NL <= 0;   // the volume's centroid is wanted on a flat surface only
+    const CurFlow flow{&sh.D.cur};
+    const f3 none = mk3(0.f, 0.f, 0.f);
+    Acc<float> acc;
+    acc_zero(acc);
+    if (PART < 2 ? damping : PART == 2 ? wave_buoy : crossing) {
+        const uint32_t flast = nfc - 1;
+        uint32_t f = min((uint32_t)lane, flast);
+        float4 a = sh.r0[f], b = sh.r1[f];
+        float v6 = PART == 3 ? sh.v6[AERO ? 0 : f] : 0.f;
+#pragma unroll 4
+        for (int j = 0; j < K; ++j) {
+            const uint32_t fn = min(64u * (j + 1) + lane, flast);
+            const float4 an = sh.r0[fn], bn = sh.r1[fn];
+            const float v6n = PART == 3 ? sh.v6[AERO ? 0 : fn] : 0.f;
+            if (64u * j + lane < nfc) {
+                const f3 n1 = mk3(a.x, a.y, a.z), c = mk3(b.x, b.y, b.z);
+                const float A = a.w;
+                if (PART == 3 && !CBON) acc.V6 += v6;
+                if (PART == 3 && CBON && v6 != 0.f) {   // marks the wet faces
+                    const StepFace q = sf.points(f);
+                    face_allwet<float, true>(fb, q.p1, q.p2, q.p3, acc);
+                }
+                if (A >= 0.f) {
+                    if (PART < 2) {
+                        const f3 uf = NU ? mk3(sh.uf[0][f], sh.uf[NU ? 1 : 0][f], sh.uf[NU ? 2 : 0][f]) : none;
+                        if (AERO) aero_drag<NU>(fb, c, n1, A, uf, acc);
+                        else face_drag<NU>(fb, c, n1, A, uf, acc);
+                    } else if (PART == 2) {
+                        f3 fbi = n1 * (-A * b.w);
+                        add3(acc.Fb, fbi);
+                        add3(acc.Mb, cross(c, fbi));
+                    } else {
+                        acc.Swet += A;
+                    }
+                }
+            }
+            a = an; b = bn; v6 = v6n; f = fn;
+        }
+        for (uint32_t qb = 0; !AERO && crossing && qb < ncut; qb += 64) {
+            if (qb + lane < ncut) {
+                const StepFace q = sf.crossing(sh.cutq[qb + lane], wq);
+                const Wet wt = face_clip<float, CBON>(fb, q.p1, q.p2, q.p3, q.d0, q.d1, q.d2, acc);
+                if (wt.ok) {
+                    const f3 cpt = step_centroid<NL <= 0 && !NU>(wt.base, wt.cs, wt.ck);
+                    if (PART < 2) {
+                        if (NU)
+                            face_drag<true>(fb, cpt, wt.n1, wt.A,
+                                            flow((double)wt.base.x + (double)wt.off.x,
+                                                 (double)wt.base.y + (double)wt.off.y,
+                                                 (double)wt.base.z + (double)wt.off.z),
+                                            acc);
+                        else
+                            face_drag(fb, cpt, wt.n1, wt.A, acc);
+                    } else if (PART == 2) {
+                        const float dc = (float)wq.depth(wt.base, wt.off);
+                        f3 fbi = wt.n1 * (-wt.A * dc);
+                        add3(acc.Fb, fbi);
+                        add3(acc.Mb, cross(cpt, fbi));
+                    } else {
+                        acc.Swet += wt.A;
+                    }
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        v[k] = PART == 0 ? acc.Fdq[k] : PART == 1 ? acc.Fdf[k] : PART == 2 ? acc.Fb[k] : acc.CB[k];
+        v[3 + k] = PART == 0 ? acc.Mdq[k] : PART == 1 ? acc.Mdf[k] : PART == 2 ? acc.Mb[k]
+                   : k == 0 ? acc.V6 : k == 1 ? acc.Swet : 0.f;
+    }
+    xreduce6(v, lane);
+}
+
+// epilogue_finish on one wavefront for a hydrodynamic body: lanes 0-3 take a
+// drag vector each with its correction (a square root and two divisions in
+// FP64, one after the other on one lane), lane 4 the buoyancy; the row is put
+// together in LDS (24 doubles) and stored by 22 lanes at once.  The same
+// operations as epilogue_finish, so the same bits.
+__device__ __forceinline__ void finish_lanes(const BodyStatic& S, const BodyDyn& D, const OceanK& oc, const double* P,
+                                             double* row, double* __restrict__ o, double* __restrict__ applied, int lane)
+{
+    const uint32_t flags = D.flags;
+    const bool body_level = !(flags & (BF_MODE_SURF | BF_MODE_SUBM | BF_MODE_AERO));
+    uint32_t written = 0;
+    if (lane < 4) {
+        double x[3];
+        finish_drag(D, P, lane, x);
+        if (body_level && (flags & BF_DAMPING)) {
+            double BO[9], M[9];
+            finish_basis(S, D, BO);
+            correct_inverse(BO, M);
+            correct_vector(oc.rho, M, lane < 2 ? S.Cd : S.Cf, lane < 2, x);
+        }
+        for (int k = 0; k < 3; ++k) row[6 + 3 * lane + k] = x[k];
+    } else if (lane == 4) {
+        double Fb[3], Tb[3], Swet, Vsub;
+        written = finish_buoyancy(S, D, oc, P, Fb, Tb, Swet, Vsub);
+        for (int k = 0; k < 3; ++k) { row[k] = Fb[k]; row[3 + k] = Tb[k]; }
+        row[18] = Swet;
+        row[19] = Vsub;
+        row[20] = (double)written;
+        row[21] = (double)D.pos;
+    }
+    written = (uint32_t)__shfl((int)written, 4, 64);
+    wave_lds_sync();
+    // slot k's bit of the write mask: 3 slots per bit up to 18, then one each
+    if (lane < 22 && (lane >= 20 || (written >> (lane < 18 ? lane / 3 : lane - 12)) & 1u)) o[lane] = row[lane];
+    if (applied && lane < 6) {
+        double x[3];
+        for (int q = 0; q < 3; ++q) {   // a slot the row leaves untouched holds what it held
+            const int k = 6 * q + lane;
+            x[q] = (written >> (k / 3)) & 1u ? row[k] : o[k];
+        }
+        applied[lane] = (x[0] + x[1]) + x[2];
+    }
+}
+
+// What ApplyHydrodynamicForces / ApplyAerodynamicForces hand to Bullet from a
+// row (SolidEntity.cpp:1958-1968).
+__device__ __forceinline__ void tick_applied(const double* o, bool aero, double* a)
+{
+    for (int k = 0; k < 3; ++k) {
+        a[k] = aero ? o[6 + k] : (o[k] + o[6 + k]) + o[12 + k];
+        a[3 + k] = aero ? o[9 + k] : (o[3 + k] + o[9 + k]) + o[15 + k];
+    }
+}
+
+template <int K, bool NU, int NL, bool AERO>
+__device__ __forceinline__ void step_chunk(StepShared<K, NU, AERO>& sh, const Chunk& ch, const StepArgs& a,
+                                           const OceanK& oc)
+{
+    const int t = threadIdx.x, lane = t & 63, wl = t >> 6;
+    const BodyStatic& S = sh.S;
+    const bool first = ch.first == 0;     // this workgroup also answers for the body's row when it has no face work
+    double* o = a.out + (size_t)ch.body * SFH_OUT_DOUBLES;
+    double* ap = a.applied ? a.applied + (size_t)ch.body * 6 : nullptr;
+    const uint32_t nfc = ch.count, vlo = ch.vlo, vn = ch.vn;
+    const bool win = vn > 0 && vn <= win_cap(K);
+    const StepFaces<K, NU, NL, AERO> sf{sh, gptr(S.verts), gptr(S.faces) + 3 * (size_t)ch.first, win};
+    if (wl == 0) {
+        if (lane < kPrologueLanes) {
+            const int pos = prologue_body(S, sh.state, a.kind, oc, &sh.D, first, o, lane);
+            if (lane == 0) { sh.pos = pos; sh.wet = 0; }
+        }
+    } else {
+        if (!AERO && win)
+            for (uint32_t k = t - 64; k < vn; k += 192) {
+                const f3 p = vert(sf.verts, vlo + k);
+                sh.sv[k] = make_float4(p.x, p.y, p.z, 0.f);
+            }
+        // the geometry of face_submerged, face_aero and face_allwet
+#pragma unroll 2
+        for (uint32_t f = t - 64; f < nfc; f += 192) {
+            const SFH_GLOBAL uint32_t* i = sf.faces + 3 * (size_t)f;
+            const uint32_t i0 = i[0], i1 = i[1], i2 = i[2];
+            const f3 p1 = vert(sf.verts, i0), p2 = vert(sf.verts, i1), p3 = vert(sf.verts, i2);
+            if (!AERO && win)
+                sh.sf[f] = make_ushort4((uint16_t)(i0 - vlo), (uint16_t)(i1 - vlo), (uint16_t)(i2 - vlo), 0);
+            const f3 e1 = p2 - p1, e2 = p3 - p1;
+            const f3 n = cross(e1, e2);
+            const float n2 = dot(n, n);
+            const float inv = frsq(n2);
+            const f3 n1 = n * inv, c = step_centroid<true>(p1, e1 + e2, 1.0f / 3.0f);
+            sh.r0[f] = make_float4(n1.x, n1.y, n1.z, n2 < SFH_DEGENERATE_N2 ? -1.f : 0.5f * (n2 * inv));
+            sh.r1[f] = make_float4(c.x, c.y, c.z, 0.f);
+        }
+    }
+    __syncthreads();
+    const int pos = uni(sh.pos);
+    if (pos <= 0 || S.nchunks == 0) {
+        if (ap && first && t == 0) {
+            if (pos == 0)
+                for (int k = 0; k < 6; ++k) ap[k] = 0.0;
+            else
+                tick_applied(o, AERO, ap);
+        }
+        return;
+    }
+    const BodyDyn& D = sh.D;
+    FaceBody fb;
+    fb.vb = uni(D.fb.vb);
+    fb.w = uni(D.fb.w);
+    fb.o = uni(D.fb.o);
+    const CurFlow flow{&D.cur};
+    const bool crossing = !AERO && pos != 1;
+    const uint32_t flags = (uint32_t)uni((int)D.flags);
+    const bool damping = AERO || !crossing || (flags & BF_DAMPING);
+    const bool wave_buoy = crossing && (flags & BF_BUOYANT) && oc.nlayers > 0;
+    uint32_t ncut = 0;
+    WaveQ<NL> wq;
+    if (crossing) {
+        wq.load(D, oc);
+        if (NL >= 0) {
+            wq.tz = uni(wq.tz);
+            for (int k = 0; k < 3; ++k) wq.rz[k] = uni(wq.rz[k]);
+#pragma unroll
+            for (int l = 0; l < (NL > 0 ? NL : 0); ++l) {
+                wq.fu[l] = uni(wq.fu[l]);
+                wq.fv[l] = uni(wq.fv[l]);
+                for (int k = 0; k < 3; ++k) { wq.ru[l][k] = uni(wq.ru[l][k]); wq.rv[l][k] = uni(wq.rv[l][k]); }
+                wq.ku[l] = uni(wq.ku[l]);
+                wq.kv[l] = uni(wq.kv[l]);
+            }
+        }
+        if (win) {
+            bool wet = false;
+            const f3 zero = mk3(0.f, 0.f, 0.f);
+            for (uint32_t k = t; k < vn; k += 256) {
+                const float4 x = sh.sv[k];
+                const float d = (float)wq.depth(mk3(x.x, x.y, x.z), zero);
+                sh.sv[k].w = d;
+                wet |= !(d < 0.f);
+            }
+            if (__ballot(wet) != 0ull && lane == 0) sh.wet = 1;
+            __syncthreads();
+        }
+        if (!win || uni(sh.wet) != 0) {   // else every vertex is dry: the chunk adds nothing (SolidEntity.cpp:1353)
+            // wavefront w takes the rows w, w + 4, ... of 64 faces, all of its
+            // faces' texels requested before the first is used (a dry or cut
+            // face's are not used at all)
+            constexpr int R = (K + 3) / 4;
+            StepFace q[R];
+            typename WaveQ<NL>::Pending pd[R];
+#pragma unroll
+            for (int i = 0; i < R; ++i) {
+                q[i] = sf.crossing(min(64u * (wl + 4 * i) + lane, nfc - 1), wq);
+                if (NL > 0 && wave_buoy)
+                    pd[i] = wq.issue(q[i].p1, ((q[i].p2 - q[i].p1) + (q[i].p3 - q[i].p1)) * (1.0f / 3.0f));
+            }
+#pragma unroll
+            for (int i = 0; i < R; ++i) {
+                const uint32_t j = wl + 4 * i, f = 64u * j + lane;
+                bool cut = false;
+                if (f < nfc) {
+                    const f3 p1 = q[i].p1, e1 = q[i].p2 - p1, e2 = q[i].p3 - p1;
+                    const bool allwet = !(q[i].d0 < 0.f) && !(q[i].d1 < 0.f) && !(q[i].d2 < 0.f);
+                    cut = !allwet && !(q[i].d0 < 0.f && q[i].d1 < 0.f && q[i].d2 < 0.f);
+                    float v6 = 0.f;
+                    if (allwet) {
+                        float dc = 0.f;
+                        if (NL > 0) {
+                            Acc<float> one;
+                            acc_zero(one);
+                            tetra_term0<float, false>(p1 - fb.o, cross(e1, e2), e1 + e2, one);
+                            v6 = one.V6;
+                            if (wave_buoy) dc = (float)wq.finish(pd[i]);
+                        } else {
+                            v6 = 1.f;   // marks the face: its volume terms are formed with the centroid's
+                            const f3 off = (e1 + e2) * (1.0f / 3.0f);
+                            if (NL < 0 && wave_buoy) dc = (float)wq.depth(p1, off);
+                            if (NU) {
+                                const f3 u = flow((double)p1.x + (double)off.x, (double)p1.y + (double)off.y,
+                                                  (double)p1.z + (double)off.z);
+                                sh.uf[0][f] = u.x; sh.uf[NU ? 1 : 0][f] = u.y; sh.uf[NU ? 2 : 0][f] = u.z;
+                            }
+                        }
+                        const f3 c = step_centroid<NL <= 0 && !NU>(p1, e1 + e2, 1.0f / 3.0f);
+                        sh.r1[f] = make_float4(c.x, c.y, c.z, dc);
+                    } else {
+                        sh.r0[f].w = -1.f;
+                    }
+                    sh.v6[f] = v6;
+                }
+                const uint64_t m = __ballot(cut);
+                if (lane == 0 && j < (uint32_t)K) sh.cut[j] = m;
+            }
+            __syncthreads();
+            // the cut faces in the order of the rows
+            for (uint32_t j = 0; j < (uint32_t)K; ++j) {
+                const uint64_t m = sh.cut[j];
+                if ((j & 3u) == (uint32_t)wl && ((m >> lane) & 1ull))
+                    sh.cutq[ncut + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = (uint16_t)(64u * j + lane);
+                ncut += (uint32_t)__popcll(m);
+            }
+            ncut = (uint32_t)uni((int)ncut);
+            __syncthreads();
+        }
+    } else if (NU) {
+        for (uint32_t f = t; f < nfc; f += 256) {
+            const StepFace q = sf.points(f);
+            const f3 u = flow(((double)q.p1.x + (double)q.p2.x + (double)q.p3.x) / 3.0,
+                              ((double)q.p1.y + (double)q.p2.y + (double)q.p3.y) / 3.0,
+                              ((double)q.p1.z + (double)q.p2.z + (double)q.p3.z) / 3.0);
+            sh.uf[0][f] = u.x; sh.uf[NU ? 1 : 0][f] = u.y; sh.uf[NU ? 2 : 0][f] = u.z;
+        }
+        __syncthreads();
+    }
+    double v[6] = {};
+    if (!crossing || !win || uni(sh.wet) != 0) {
+        if (wl == 0)
+            step_sums<K, NU, NL, AERO, 0>(sh, sf, nfc, fb, wq, crossing, wave_buoy, damping, ncut, lane, v);
+        else if (AERO || (!crossing && wl > 1))
+            v[0] = 0.0;
+        else if (wl == 1)
+            step_sums<K, NU, NL, AERO, 1>(sh, sf, nfc, fb, wq, crossing, wave_buoy, damping, ncut, lane, v);
+        else if (wl == 2)
+            step_sums<K, NU, NL, AERO, 2>(sh, sf, nfc, fb, wq, crossing, wave_buoy, damping, ncut, lane, v);
+        else
+            step_sums<K, NU, NL, AERO, 3>(sh, sf, nfc, fb, wq, crossing, wave_buoy, damping, ncut, lane, v);
+    }
+    {
+        const int q = xreduce6_slot(lane);
+        if (q >= 0) sh.P[6 * wl + q] = v[0];
+    }
+    __syncthreads();
+    if (wl != 0) return;
+    if (S.nchunks > 1) {
+        // Partials and counter are agent-scope accesses (they bypass the
+        // non-coherent caches); the wait orders the partial before the count,
+        // and the count's result orders the other workgroups' partials before
+        // their loads.  An agent-scope release fence in its place writes the
+        // whole L2 back, some 46 ns per chunk serialised over the chip.
+        double* mine = a.partials + (size_t)(S.chunk0 + ch.first / (64u * K)) * kChunkDoubles;
+        if (lane < kChunkDoubles)
+            __hip_atomic_store(mine + lane, sh.P[lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        uint32_t n = 0;
+        if (lane == 0) n = __hip_atomic_fetch_add(a.done + ch.body, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if ((uint32_t)uni((int)n) + 1u != S.nchunks) return;
+        asm volatile("" ::: "memory");
+        if (lane == 0) __hip_atomic_store(a.done + ch.body, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        epilogue_sums<true>(S, a.partials, sh.P, lane);
+        wave_lds_sync();
+    }
+    if (!AERO) {
+        finish_lanes(S, D, oc, sh.P, sh.state, o, ap, lane);   // the state is not read any more
+    } else if (lane == 0) {
+        epilogue_finish(S, D, oc, sh.P, o);
+        if (ap) tick_applied(o, AERO, ap);
+    }
+}
+
+// One workgroup per chunk of a batch.
+template <int K, bool NU, int NL, bool AERO>
+__global__ __launch_bounds__(256) void k_step(StepArgs a, OceanK oc)
+{
+    __shared__ StepShared<K, NU, AERO> sh;
+    const int t = threadIdx.x;
+    const Chunk ch = a.chunks[blockIdx.x];
+    if (a.active && !a.active[ch.sidx]) {
+        if (a.applied && ch.first == 0 && t < 6) a.applied[(size_t)ch.body * 6 + t] = 0.0;
+        return;
+    }
+    const int ns = a.kind ? 38 : 22;
+    const uint32_t* src = (const uint32_t*)(a.st + ch.body);
+    for (int i = t; i < (int)(sizeof(BodyStatic) / 4); i += 256) ((uint32_t*)&sh.S)[i] = src[i];
+    if (t >= 192 && t < 192 + ns) sh.state[t - 192] = a.states[(size_t)ch.sidx * ns + (t - 192)];
+    __syncthreads();
+    step_chunk<K, NU, NL, AERO>(sh, ch, a, oc);
 }
 
 // Per row of the state array (a body, or a compound): what the surrogate's
@@ -1629,6 +2188,8 @@ struct sfh_batch_t {
     uint32_t* d_lists = nullptr;    // the step's work list [nchunks], then its two counts
     BodyDyn* d_dyn = nullptr;
     double* d_partials = nullptr;
+    uint32_t* d_done = nullptr;     // per body: chunks k_step finished in this step (zero between steps)
+    bool all_faces = false;         // every body has at least one chunk
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
     bool timing = false;
@@ -1892,6 +2453,7 @@ static void batch_free(sfh_batch_t* b)
     hipFree(b->d_lists);
     hipFree(b->d_dyn);
     hipFree(b->d_partials);
+    hipFree(b->d_done);
     hipFree(b->d_comp);
     hipFree(b->d_part_out);
     hipFree(b->d_units);
@@ -1936,8 +2498,10 @@ static int batch_build_chunks(sfh_batch_t* b)
 {
     std::vector<Chunk> chunks;
     const uint32_t csize = 64u * b->K;
+    b->all_faces = true;
     for (uint32_t i = 0; i < b->n; ++i) {
         BodyStatic& s = b->h_static[i];
+        b->all_faces = b->all_faces && s.nf > 0;
         const sfh_mesh_t* m = i < b->meshes_by_body.size() ? b->meshes_by_body[i] : nullptr;
         s.chunk0 = (uint32_t)chunks.size();
         s.nchunks = (s.nf + csize - 1) / csize;
@@ -1945,6 +2509,7 @@ static int batch_build_chunks(sfh_batch_t* b)
             Chunk ch;
             memset(&ch, 0, sizeof(ch));
             ch.body = i;
+            ch.sidx = s.sidx;
             ch.first = c * csize;
             ch.count = std::min(csize, s.nf - c * csize);
             if (m) chunk_window(m->blkwin, ch.first, ch.count, win_cap(b->K), ch.vlo, ch.vn);
@@ -1957,8 +2522,9 @@ static int batch_build_chunks(sfh_batch_t* b)
     hipFree(b->d_partials);
     hipFree(b->d_bpos);
     hipFree(b->d_lists);
+    hipFree(b->d_done);
     b->d_static = nullptr; b->d_sidx = nullptr; b->d_chunks = nullptr;
-    b->d_partials = nullptr; b->d_bpos = nullptr; b->d_lists = nullptr;
+    b->d_partials = nullptr; b->d_bpos = nullptr; b->d_lists = nullptr; b->d_done = nullptr;
     b->nchunks = (uint32_t)chunks.size();
     HIPCHK(hipMalloc(&b->d_static, sizeof(BodyStatic) * std::max<size_t>(1, b->n)));
     HIPCHK(hipMemcpy(b->d_static, b->h_static.data(), sizeof(BodyStatic) * b->n, hipMemcpyHostToDevice));
@@ -1975,6 +2541,8 @@ static int batch_build_chunks(sfh_batch_t* b)
     HIPCHK(hipMalloc(&b->d_bpos, std::max<size_t>(1, b->n)));
     HIPCHK(hipMalloc(&b->d_lists, sizeof(uint32_t) * ((size_t)b->nchunks + 2)));
     HIPCHK(hipMemset(b->d_lists + b->nchunks, 0, 2 * sizeof(uint32_t)));
+    HIPCHK(hipMalloc(&b->d_done, sizeof(uint32_t) * std::max<size_t>(1, b->n)));
+    HIPCHK(hipMemset(b->d_done, 0, sizeof(uint32_t) * std::max<size_t>(1, b->n)));
     if (b->graph_exec) { hipGraphExecDestroy(b->graph_exec); b->graph_exec = nullptr; }
     if (b->graph) { hipGraphDestroy(b->graph); b->graph = nullptr; }
     return SFH_OK;
@@ -2359,12 +2927,54 @@ static int launch_faces(sfh_batch_t* b, const OceanK& oc, hipStream_t s)
     return SFH_OK;
 }
 
-// One evaluation: the prologue, the face pass, the epilogue and, for a
-// compound batch, the composition of the parts' rows.  timed: events before
-// the prologue (ev[0]), around the face launches (ev[1], ev[2]) and after the
-// last launch (ev[3]).
-static int batch_launch(sfh_batch_t* b, const sfh_ocean_t* o, const double* d_states, int kind, double* d_out,
-                        hipStream_t s, bool timed, const uint8_t* active = nullptr, bool skip_prologue = false)
+// Whether a step runs as one launch of k_step (a workgroup per chunk): up to
+// 1,024 chunks of a batch that asks for one face launch (split_passes 0) and
+// whose bodies all have faces (k_step's workgroups are chunks), with the faces
+// per lane it is built for.  Two of its workgroups fit a CU beside each other
+// (65 KB of LDS at 16 faces per lane), so past 512 working chunks they come in
+// rounds of about 11 us, where the general path's face launch still has every
+// chunk in flight; the two cross between 850 and 1,130 chunks.  Measured, a
+// tick of bodies of 2.8 chunks on average, 16 faces per lane, general path
+// against one launch:
+//     chunks         flat sea        one wave layer   two layers
+//       279        29.7 / 17.4 us    33.9 / 17.2 us   39.2 / 18.9 us
+//       850        30.4 / 29.0       35.1 / 29.0      40.4 / 31.6
+//     1,129        30.4 / 35.8       34.4 / 35.5      40.4 / 39.1
+//     1,700        31.0 / 51.0       36.7 / 50.5      45.1 / 54.4
+// and with a mask leaving 30 % of the bodies, 28-39 / 17-20 us up to 1,129
+// chunks.  Aerodynamic batches: 850 chunks 16.8 / 11.8 us, 1,413 17.6 / 18.2.
+static constexpr uint32_t kStepChunks = 1024;
+
+static bool step_fused(const sfh_batch_t* b)
+{
+    return !b->compound && !b->split && b->all_faces && (b->K == 8 || b->K == 16) && b->nchunks <= kStepChunks;
+}
+
+static void launch_step(sfh_batch_t* b, const OceanK& oc, const StepArgs& a, hipStream_t s)
+{
+#define LAUNCH_S(KK, NU, NL, AERO) \
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_step<KK, NU, NL, AERO>), dim3(b->nchunks), dim3(256), 0, s, a, oc)
+#define LAUNCH_SK(KK)                                                                             \
+    if (b->aero) {                                                                                \
+        if (oc.ncur) LAUNCH_S(KK, true, 0, true); else LAUNCH_S(KK, false, 0, true);              \
+    } else if (oc.ncur) LAUNCH_S(KK, true, -1, false);                                            \
+    else if (oc.nlayers > 2 || (oc.nlayers > 0 && oc.nmask < 0)) LAUNCH_S(KK, false, -1, false);  \
+    else if (oc.nlayers == 0) LAUNCH_S(KK, false, 0, false);                                      \
+    else if (oc.nlayers == 1) LAUNCH_S(KK, false, 1, false);                                      \
+    else LAUNCH_S(KK, false, 2, false);
+    if (b->K == 8) { LAUNCH_SK(8) } else { LAUNCH_SK(16) }
+#undef LAUNCH_SK
+#undef LAUNCH_S
+}
+
+// One evaluation: one launch (step_fused), or the prologue, the face pass, the
+// epilogue and, for a compound batch, the composition of the parts' rows.
+// timed: events before the first launch (ev[0]), around the face launches
+// (ev[1], ev[2]; around the one launch) and after the last launch (ev[3]).
+// applied (optional): the tick driver's force and torque per row, which only
+// the one-launch step writes (step_fused says whether it does).
+static int batch_launch(sfh_batch_t* b, const sfh_ocean_t* o, const double* d_states, double* d_out, hipStream_t s,
+                        bool timed, const uint8_t* active = nullptr, double* applied = nullptr)
 {
     if (b->n == 0) return SFH_OK;
     // every launch of the step runs or none does: the epilogue zeroes the
@@ -2372,21 +2982,38 @@ static int batch_launch(sfh_batch_t* b, const sfh_ocean_t* o, const double* d_st
     if (b->K != 1 && b->K != 2 && b->K != 4 && b->K != 8 && b->K != 16 && b->K != 32)
         return fail(SFH_ERR_INVALID, "bad K");
     OceanK oc = make_oceank(o);
+    if (step_fused(b)) {
+        StepArgs a;
+        a.st = b->d_static;
+        a.chunks = b->d_chunks;
+        a.states = d_states;
+        a.active = active;
+        a.out = d_out;
+        a.applied = applied;
+        a.partials = b->d_partials;
+        a.done = b->d_done;
+        a.kind = 0;
+        if (timed) HIPCHK(hipEventRecord(b->ev[0], s));
+        if (timed) HIPCHK(hipEventRecord(b->ev[1], s));
+        launch_step(b, oc, a, s);
+        if (timed) HIPCHK(hipEventRecord(b->ev[2], s));
+        if (timed) HIPCHK(hipEventRecord(b->ev[3], s));
+        HIPCHK(hipGetLastError());
+        return SFH_OK;
+    }
     double* rows = b->compound ? b->d_part_out : d_out;
     if (timed) HIPCHK(hipEventRecord(b->ev[0], s));
-    if (!skip_prologue) {
-        const bool large = !active && b->n >= kPrologueLargeBodies;
-        const uint32_t blk = large ? kPrologueBlockLarge : kPrologueBlock;
-        const uint32_t blocks = (uint32_t)(((uint64_t)b->n * kPrologueLanes + blk - 1) / blk);
-        if (large)
-            hipLaunchKernelGGL(k_prologue<kPrologueBlockLarge>, dim3(blocks), dim3(blk), 0, s, b->d_static, d_states,
-                               kind, b->n, oc, active, b->d_sidx, b->d_dyn, b->d_bpos, rows, b->d_lists, b->nchunks,
-                               b->d_lists + b->nchunks);
-        else
-            hipLaunchKernelGGL(k_prologue<kPrologueBlock>, dim3(blocks), dim3(blk), 0, s, b->d_static, d_states, kind,
-                               b->n, oc, active, b->d_sidx, b->d_dyn, b->d_bpos, rows, b->d_lists, b->nchunks,
-                               b->d_lists + b->nchunks);
-    }
+    const bool large = !active && b->n >= kPrologueLargeBodies;
+    const uint32_t blk = large ? kPrologueBlockLarge : kPrologueBlock;
+    const uint32_t blocks = (uint32_t)(((uint64_t)b->n * kPrologueLanes + blk - 1) / blk);
+    if (large)
+        hipLaunchKernelGGL(k_prologue<kPrologueBlockLarge>, dim3(blocks), dim3(blk), 0, s, b->d_static, d_states,
+                           b->n, oc, active, b->d_sidx, b->d_dyn, b->d_bpos, rows, b->d_lists, b->nchunks,
+                           b->d_lists + b->nchunks);
+    else
+        hipLaunchKernelGGL(k_prologue<kPrologueBlock>, dim3(blocks), dim3(blk), 0, s, b->d_static, d_states,
+                           b->n, oc, active, b->d_sidx, b->d_dyn, b->d_bpos, rows, b->d_lists, b->nchunks,
+                           b->d_lists + b->nchunks);
     if (timed) HIPCHK(hipEventRecord(b->ev[1], s));
     int rc = launch_faces(b, oc, s);
     if (rc != SFH_OK) return rc;
@@ -2433,7 +3060,7 @@ extern "C" int sfh_batch_compute(sfh_batch b, sfh_ocean o, const double* d_state
     hipStream_t s = (hipStream_t)stream;
     bool timed = b->timing;
     if (timed) harvest_timing(b);
-    rc = batch_launch(b, o, d_states, 0, d_out, s, timed);
+    rc = batch_launch(b, o, d_states, d_out, s, timed);
     if (rc == SFH_OK && timed) b->ev_pending = true;
     return rc;
 }
@@ -2447,7 +3074,7 @@ extern "C" int sfh_batch_compute_masked(sfh_batch b, sfh_ocean o, const double* 
     hipStream_t s = (hipStream_t)stream;
     bool timed = b->timing;
     if (timed) harvest_timing(b);
-    rc = batch_launch(b, o, d_states, 0, d_out, s, timed, d_active);
+    rc = batch_launch(b, o, d_states, d_out, s, timed, d_active);
     if (rc == SFH_OK && timed) b->ev_pending = true;
     return rc;
 }
@@ -2494,11 +3121,11 @@ extern "C" int sfh_batch_autotune(sfh_batch b, sfh_ocean o, const double* d_stat
             sfh_batch_opts opts = {K, wpc * (uint32_t)cus, split};
             rc = apply_opts(b, &opts);
             if (rc != SFH_OK) break;
-            rc = batch_launch(b, o, d_states, 0, d_out, s, false, d_active);   // warm-up
+            rc = batch_launch(b, o, d_states, d_out, s, false, d_active);   // warm-up
             if (rc != SFH_OK) break;
             hipEventRecord(e0, s);
             for (uint32_t r = 0; r < reps && rc == SFH_OK; ++r)
-                rc = batch_launch(b, o, d_states, 0, d_out, s, r + 1 == reps, d_active);
+                rc = batch_launch(b, o, d_states, d_out, s, r + 1 == reps, d_active);
             hipEventRecord(e1, s);
             if (rc != SFH_OK) break;
             hipError_t e = hipEventSynchronize(e1);
@@ -2559,10 +3186,7 @@ __global__ __launch_bounds__(128) void k_tick_apply(const double* __restrict__ o
         for (int k = 0; k < 6; ++k) a[k] = 0.0;
         return;
     }
-    for (int k = 0; k < 3; ++k) {
-        a[k] = aero ? o[6 + k] : (o[k] + o[6 + k]) + o[12 + k];
-        a[3 + k] = aero ? o[9 + k] : (o[3 + k] + o[9 + k]) + o[15 + k];
-    }
+    tick_applied(o, aero != 0, a);
 }
 
 struct sfh_tick_t {
@@ -2592,12 +3216,17 @@ extern "C" int sfh_tick_step(sfh_tick t, sfh_ocean fluid, const double* d_states
     const bool recompute = t->counter % t->prescaler == 0;
     ++t->counter;
     hipStream_t s = (hipStream_t)stream;
-    if (recompute) {
-        rc = sfh_batch_compute_masked(t->batch, fluid, d_states, d_overlap, d_out, stream);
-        if (rc != SFH_OK) return rc;
-    }
     const uint32_t n = t->batch->nunits;
-    if (n) hipLaunchKernelGGL(k_tick_apply, dim3((n + 127) / 128), dim3(128), 0, s, d_out, d_overlap, n,
+    bool applied = false;
+    if (recompute) {
+        sfh_batch_t* b = t->batch;
+        if (b->timing) harvest_timing(b);
+        rc = batch_launch(b, fluid, d_states, d_out, s, b->timing, d_overlap, d_applied);
+        if (rc != SFH_OK) return rc;
+        if (b->timing) b->ev_pending = true;
+        applied = b->n > 0 && step_fused(b);
+    }
+    if (n && !applied) hipLaunchKernelGGL(k_tick_apply, dim3((n + 127) / 128), dim3(128), 0, s, d_out, d_overlap, n,
                               t->batch->aero ? 1 : 0, d_applied);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(SFH_ERR_HIP, "tick apply: %s", hipGetErrorString(e));
@@ -2646,7 +3275,7 @@ extern "C" int sfh_batch_capture(sfh_batch b, sfh_ocean o, const double* d_state
     if (b->graph_exec) { hipGraphExecDestroy(b->graph_exec); b->graph_exec = nullptr; }
     if (b->graph) { hipGraphDestroy(b->graph); b->graph = nullptr; }
     HIPCHK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-    rc = batch_launch(b, o, d_states, 0, d_out, s, false);
+    rc = batch_launch(b, o, d_states, d_out, s, false);
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamEndCapture(s, &g);
     if (rc != SFH_OK) { if (g) hipGraphDestroy(g); return rc; }
@@ -2688,29 +3317,16 @@ extern "C" int sfh_batch_kernel_ms(sfh_batch b, double* face_ms, double* total_m
 
 // ---- per-body evaluations ------------------------------------------------------
 
-// One per-body evaluation (a single-body batch) needs, beyond the mesh: the
-// body's static record and per-step constants, its chunks with their vertex
-// windows, the work list and the chunk partials.  They are
-// carved out of one device buffer sized for meshes of up to F faces: a
-// workspace of the per-body statics (device memory from hipMalloc, grown on
-// demand) or the no-alloc entry point's file-scope array.  One kernel writes
-// the static record and the chunks from its arguments and the mesh's block
-// windows and, in its first workgroup, runs the body's prologue (which gives
-// the body the position its call names: the Surface call the crossing loop,
-// the Submerged and aerodynamic calls the submerged one); the step is that
-// kernel, the face pass and the epilogue.
+// One per-body evaluation is one launch of k_step_one, a workgroup per 64 *
+// kSingleK faces.  Beyond the mesh it needs the chunk counter and the chunk
+// partials of a mesh of more than one chunk, in one device buffer sized for
+// meshes of up to F faces: a workspace of the per-body statics (device memory
+// from hipMalloc, grown on demand) or the no-alloc entry point's file-scope
+// array.  The counter is zero between calls (the workgroup that finishes the
+// row zeroes it).
 static constexpr uint32_t kSingleK = 8;   // faces per lane of per-body calls
 
-struct SingleHead {
-    BodyStatic st;
-    BodyDyn dyn;
-    uint32_t sidx;
-    int8_t bpos;
-    double state[38];   // T_CG, T_C, v, omega of a call whose state came by value
-};
-
-// A per-body call's state passed by value to the setup kernel (no copy
-// command of its own).
+// A per-body call's state passed by value (no copy command of its own).
 struct StateArg {
     double v[38];
 };
@@ -2718,115 +3334,80 @@ struct StateArg {
 __host__ __device__ constexpr size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 __host__ __device__ constexpr uint32_t single_nchunks(uint32_t F) { return (F + 64u * kSingleK - 1) / (64u * kSingleK); }
 
-// Byte offsets of the parts in a buffer for F faces: head, work list (with
-// its counts), chunks, partials, end.
-struct SingleLayout {
-    size_t lists, chunks, partials, end;
-};
+static constexpr size_t kSinglePartials = 256;   // byte offset of the partials; the counter is at 0
 
-__host__ __device__ constexpr SingleLayout single_layout(uint32_t F)
+__host__ __device__ constexpr size_t single_bytes(uint32_t F)
 {
     const size_t nc = single_nchunks(F);
-    const size_t lists = align256(sizeof(SingleHead));
-    const size_t chunks = align256(lists + sizeof(uint32_t) * (nc + 2));
-    const size_t partials = align256(chunks + sizeof(Chunk) * (nc ? nc : 1));
-    const size_t end = align256(partials + sizeof(double) * kChunkDoubles * (nc ? nc : 1));
-    return SingleLayout{lists, chunks, partials, end};
+    return align256(kSinglePartials + sizeof(double) * kChunkDoubles * (nc ? nc : 1));
 }
 
-// Writes the body's static record and its chunks with their vertex windows
-// (from the mesh's per-64-face block windows), and zeroes the work list's
-// counts (the buffer may hold another call's).
-// The setup of a per-body call and, in its first workgroup once the record,
-// the state and the counts are written, the body's prologue (one launch
-// instead of two; the batch's own prologue launch is skipped).
-__global__ __launch_bounds__(kPrologueBlock) void k_single_setup(SingleHead* __restrict__ H, Chunk* __restrict__ chunks,
-                                                      uint32_t* __restrict__ counts, const uint2* __restrict__ blkwin,
-                                                      BodyStatic st, StateArg sa, int with_state,
-                                                      const double* __restrict__ states, OceanK oc,
-                                                      double* __restrict__ out, uint32_t* __restrict__ list)
+// One body's step, a workgroup per chunk; the chunk's vertex window comes from
+// the mesh's per-64-face block windows.  states: the state in device memory,
+// or null with the state in sa.
+template <bool NU, int NL, bool AERO>
+__global__ __launch_bounds__(256) void k_step_one(StepArgs a, OceanK oc, BodyStatic st, StateArg sa,
+                                                  const uint2* __restrict__ blkwin)
 {
-    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t csize = 64u * kSingleK;
-    const uint32_t nc = st.nchunks;
-    if (with_state && t < 38) H->state[t] = sa.v[t];
-    if (t == 0) {
-        H->st = st;
-        H->sidx = 0;
-        counts[0] = 0u;
-        counts[1] = 0u;
+    constexpr int K = kSingleK;
+    __shared__ StepShared<K, NU, AERO> sh;
+    const int t = threadIdx.x;
+    Chunk ch;
+    ch.body = 0;
+    ch.sidx = 0;
+    ch.first = blockIdx.x * 64u * K;
+    ch.count = min(64u * K, st.nf - ch.first);
+    uint32_t lo = 0xffffffffu, hi = 0;
+    const uint32_t nblk = (st.nf + 63) / 64;
+    for (uint32_t k = blockIdx.x * K; k < min((blockIdx.x + 1) * K, nblk); ++k) {
+        const uint2 w = blkwin[k];
+        lo = min(lo, w.x);
+        hi = max(hi, w.y);
     }
-    if (t < nc) {
-        Chunk c;
-        c.body = 0;
-        c.first = t * csize;
-        c.count = min(csize, st.nf - t * csize);
-        uint32_t lo = 0xffffffffu, hi = 0;
-        const uint32_t nblk = (st.nf + 63) / 64;
-        for (uint32_t k = t * kSingleK; k < min((t + 1) * kSingleK, nblk); ++k) {
-            const uint2 w = blkwin[k];
-            lo = min(lo, w.x);
-            hi = max(hi, w.y);
-        }
-        const bool fits = lo <= hi && hi - lo + 1 <= win_cap(kSingleK);
-        c.vlo = fits ? lo : 0u;
-        c.vn = fits ? hi - lo + 1 : 0u;
-        c.pad[0] = c.pad[1] = c.pad[2] = 0;
-        chunks[t] = c;
-    }
-    if (blockIdx.x == 0) {
-        __syncthreads();   // the record, the state and the zeroed counts are this workgroup's writes
-        prologue_group<kPrologueBlock>(&H->st, states, 1, 1u, oc, nullptr, &H->sidx, &H->dyn, &H->bpos, out, list,
-                                       nc, counts, threadIdx.x);
-    }
+    const bool fits = lo <= hi && hi - lo + 1 <= win_cap(K);
+    ch.vlo = fits ? lo : 0u;
+    ch.vn = fits ? hi - lo + 1 : 0u;
+    if (t == 0) sh.S = st;
+    if (t >= 192 && t < 192 + 38) sh.state[t - 192] = a.states ? a.states[t - 192] : sa.v[t - 192];
+    __syncthreads();
+    step_chunk<K, NU, NL, AERO>(sh, ch, a, oc);
 }
 
-// One evaluation of `m` with `flags` from the 38-double state d_state into
-// the output row d_out, on stream s, in the buffer `buf` laid out for the
-// mesh's face count.  No allocation.
-// d_state: the state in device memory, or nullptr with h_state: the state's
-// 38 doubles on the host, passed to the setup kernel by value.
+// One evaluation of `m` with `flags` from the 38-double state d_state (or, with
+// d_state null, h_state on the host, passed by value) into the output row
+// d_out (device or pinned host memory), on stream s, in the buffer `buf` of
+// single_bytes of the mesh's face count.  No allocation.
 static int single_launch(unsigned char* buf, const sfh_mesh_t* m, uint32_t flags, const sfh_ocean_t* o,
-                         const double* d_state, double* d_out, hipStream_t s, uint32_t waves,
-                         const double* h_state = nullptr)
+                         const double* d_state, double* d_out, hipStream_t s, const double* h_state = nullptr)
 {
-    const SingleLayout L = single_layout(m->nf);
-    SingleHead* H = (SingleHead*)buf;
-    Chunk* chunks = (Chunk*)(buf + L.chunks);
-    uint32_t* lists = (uint32_t*)(buf + L.lists);
     BodyStatic st = make_static(m, flags);
     st.chunk0 = 0;
     st.nchunks = single_nchunks(m->nf);
     st.sidx = 0;
-    const uint32_t nt = std::max(st.nchunks, 38u);
+    StepArgs a;
+    memset(&a, 0, sizeof(a));
+    a.states = d_state;
+    a.out = d_out;
+    a.done = (uint32_t*)buf;
+    a.partials = (double*)(buf + kSinglePartials);
+    a.kind = 1;
     StateArg sa;
-    const int with_state = d_state == nullptr;
-    if (with_state) {
-        memcpy(sa.v, h_state, sizeof(sa.v));
-        d_state = H->state;
-    } else {
-        memset(sa.v, 0, sizeof(sa.v));
-    }
-    hipLaunchKernelGGL(k_single_setup, dim3((nt + kPrologueBlock - 1) / kPrologueBlock), dim3(kPrologueBlock), 0, s,
-                       H, chunks, lists + st.nchunks, m->d_blkwin, st, sa, with_state, d_state, make_oceank(o), d_out,
-                       lists);
-    // a batch view of the buffer: no allocation (empty vectors, borrowed pointers)
-    sfh_batch_t b;
-    b.n = 1;
-    b.nunits = 1;
-    b.aero = (flags & BF_MODE_AERO) != 0;
-    b.nchunks = st.nchunks;
-    b.nfaces = m->nf;
-    b.K = kSingleK;
-    b.waves = waves;
-    b.d_static = &H->st;
-    b.d_sidx = &H->sidx;
-    b.d_chunks = chunks;
-    b.d_bpos = &H->bpos;
-    b.d_lists = lists;
-    b.d_dyn = &H->dyn;
-    b.d_partials = (double*)(buf + L.partials);
-    return batch_launch(&b, o, d_state, 1, d_out, s, false, nullptr, true);   // the prologue ran in the setup
+    if (d_state) memset(sa.v, 0, sizeof(sa.v));
+    else memcpy(sa.v, h_state, sizeof(sa.v));
+    const OceanK oc = make_oceank(o);
+    const dim3 grid(std::max(1u, st.nchunks));
+#define LAUNCH_ONE(NU, NL, AERO)                                                                               \
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_step_one<NU, NL, AERO>), grid, dim3(256), 0, s, a, oc, st, sa, m->d_blkwin)
+    if (flags & BF_MODE_AERO) {
+        if (oc.ncur) LAUNCH_ONE(true, 0, true); else LAUNCH_ONE(false, 0, true);
+    } else if (oc.ncur) LAUNCH_ONE(true, -1, false);
+    else if (oc.nlayers > 2 || (oc.nlayers > 0 && oc.nmask < 0)) LAUNCH_ONE(false, -1, false);
+    else if (oc.nlayers == 0) LAUNCH_ONE(false, 0, false);
+    else if (oc.nlayers == 1) LAUNCH_ONE(false, 1, false);
+    else LAUNCH_ONE(false, 2, false);
+#undef LAUNCH_ONE
+    HIPCHK(hipGetLastError());
+    return SFH_OK;
 }
 
 // ---- per-body reference-shaped calls ------------------------------------------
@@ -2844,7 +3425,6 @@ struct Workspace {
     double* d_io = nullptr;       // device, same layout
     unsigned char* d_buf = nullptr;
     size_t cap = 0;               // bytes of d_buf
-    uint32_t waves = 0;
 };
 static constexpr size_t kIoDoubles = 128;
 
@@ -2876,7 +3456,6 @@ static int ws_acquire(Workspace** out)
     }
     Workspace* w = new Workspace();
     w->device = dev;
-    w->waves = default_waves();
     hipError_t e = hipStreamCreateWithFlags(&w->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipHostMalloc((void**)&w->h_io, sizeof(double) * kIoDoubles, hipHostMallocDefault);
     if (e == hipSuccess) e = hipMalloc(&w->d_io, sizeof(double) * kIoDoubles);
@@ -2897,7 +3476,7 @@ static void ws_release(Workspace* w)
 // Grows the workspace's buffer to the layout of an F-face mesh.
 static int ws_reserve(Workspace* w, uint32_t F)
 {
-    const size_t need = single_layout(F).end;
+    const size_t need = single_bytes(F);
     if (need <= w->cap) return SFH_OK;
     const size_t cap = std::max(need, 2 * w->cap);
     HIPCHK(hipStreamSynchronize(w->stream));
@@ -2905,6 +3484,12 @@ static int ws_reserve(Workspace* w, uint32_t F)
     w->d_buf = nullptr;
     w->cap = 0;
     HIPCHK(hipMalloc(&w->d_buf, cap));
+    const hipError_t e = hipMemset(w->d_buf, 0, kSinglePartials);   // the counter starts at zero
+    if (e != hipSuccess) {
+        hipFree(w->d_buf);
+        w->d_buf = nullptr;
+        return fail(SFH_ERR_HIP, "per-body workspace: %s", hipGetErrorString(e));
+    }
     w->cap = cap;
     return SFH_OK;
 }
@@ -2924,12 +3509,11 @@ static int single_call(sfh_mesh_t* m, uint32_t flags, const sfh_ocean_t* o, cons
         memcpy(h + 16, T_C, 16 * sizeof(double));
         memcpy(h + 32, v, 3 * sizeof(double));
         memcpy(h + 35, w, 3 * sizeof(double));
-        // the state goes to the device as the setup kernel's argument
-        rc = single_launch(ws->d_buf, m, flags, o, nullptr, ws->d_io + 38, ws->stream, ws->waves, h);
+        // the state goes to the device as the kernel's argument, the row comes
+        // back by the kernel's own stores to the pinned staging buffer: no copy
+        rc = single_launch(ws->d_buf, m, flags, o, nullptr, h + 38, ws->stream, h);
         if (rc == SFH_OK) {
-            hipError_t e = hipMemcpyAsync(h + 38, ws->d_io + 38, SFH_OUT_DOUBLES * sizeof(double),
-                                          hipMemcpyDeviceToHost, ws->stream);
-            if (e == hipSuccess) e = hipStreamSynchronize(ws->stream);
+            const hipError_t e = hipStreamSynchronize(ws->stream);
             if (e != hipSuccess) rc = fail(SFH_ERR_HIP, "per-body call: %s", hipGetErrorString(e));
             else memcpy(out, h + 38, SFH_OUT_DOUBLES * sizeof(double));
         }
@@ -3048,18 +3632,17 @@ extern "C" int sfh_correct(sfh_ocean ocean, double Fdq[3], double Tdq[3], double
 // ends; every call on a GPU shares it, so calls that overlap on one GPU (two
 // streams, or two host threads) race.
 static constexpr uint32_t kNaMaxFaces = 1u << 19;   // 524,288
-static constexpr size_t kNaBytes = single_layout(kNaMaxFaces).end;
+static constexpr size_t kNaBytes = single_bytes(kNaMaxFaces);
 static_assert(kNaBytes <= (256u << 10), "no-alloc scratch above 256 KiB");
 
 static __device__ __align__(256) unsigned char scratch[kNaBytes];
 
 static std::mutex g_na_mu;
 static void* g_na_ptr[64];       // per device: the address of `scratch` (hipGetSymbolAddress)
-static uint32_t g_na_waves[64];  // per device: resident wavefronts of the face pass
 
 // Looks up this device's copy of `scratch` once (with the device current):
 // from sfh_init, or from the first no-alloc call on a device sfh_init did not see.
-static int na_scratch(unsigned char** out, uint32_t* waves)
+static int na_scratch(unsigned char** out)
 {
     int dev = 0;
     HIPCHK(hipGetDevice(&dev));
@@ -3069,15 +3652,13 @@ static int na_scratch(unsigned char** out, uint32_t* waves)
         void* p = nullptr;
         const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
         if (e != hipSuccess || !p) return fail(SFH_ERR_HIP, "scratch symbol address: %s", hipGetErrorString(e));
-        g_na_waves[dev] = default_waves();
         g_na_ptr[dev] = p;
     }
     if (out) *out = (unsigned char*)g_na_ptr[dev];
-    if (waves) *waves = g_na_waves[dev];
     return SFH_OK;
 }
 
-int sfh_internal_na_init(void) { return na_scratch(nullptr, nullptr); }
+int sfh_internal_na_init(void) { return na_scratch(nullptr); }
 
 extern "C" int sfh_forces_noalloc(const sfh_settings* settings, int mode, sfh_mesh mesh, sfh_ocean ocean,
                                   const double* d_state, double* d_out, void* stream)
@@ -3089,8 +3670,7 @@ extern "C" int sfh_forces_noalloc(const sfh_settings* settings, int mode, sfh_me
     if (mesh->nf > kNaMaxFaces)
         return fail(SFH_ERR_SIZE, "mesh of %u faces exceeds the no-alloc limit of %u faces", mesh->nf, kNaMaxFaces);
     unsigned char* buf = nullptr;
-    uint32_t waves = 0;
-    rc = na_scratch(&buf, &waves);
+    rc = na_scratch(&buf);
     if (rc != SFH_OK) return rc;
     uint32_t flags = BF_HYDRO | BF_EXPLICIT_TC;
     if (mode == SFH_NOALLOC_SURFACE) {
@@ -3102,7 +3682,7 @@ extern "C" int sfh_forces_noalloc(const sfh_settings* settings, int mode, sfh_me
     }
     // the layout for this mesh fits in the array's: every part's offset and
     // size grows with F
-    return single_launch(buf, mesh, flags, ocean, d_state, d_out, (hipStream_t)stream, waves);
+    return single_launch(buf, mesh, flags, ocean, d_state, d_out, (hipStream_t)stream);
 }
 
 // ---- wave grid ----------------------------------------------------------------
