@@ -4220,14 +4220,14 @@ struct SurRowCtx {
 };
 
 // One workgroup per tile of TR units of one group (one network), tiles in
-// XCD-major order: groups of 256 / TR lanes build the features of one unit
+// XCD-major order: groups of 512 / TR lanes build the features of one unit
 // each (the FP64 context of k_sur_features, wave queries spread over the
 // group) into the network's input rows in LDS while the first layer's
-// weights are in flight, the four wavefronts run the fused network
+// weights are in flight, the eight wavefronts run the fused network
 // (sfm_device.h), and lanes 0..TR-1 decode their unit's outputs to
 // world-frame F, T.
 template <int TR>
-__global__ __launch_bounds__(256) void k_sur_step(const SurPlanDev* __restrict__ P, const SurTile* __restrict__ tiles,
+__global__ __launch_bounds__(64 * sfm::kWaves, 2) void k_sur_step(const SurPlanDev* __restrict__ P, const SurTile* __restrict__ tiles,
                                                   const UnitStatic* __restrict__ units,
                                                   const double* __restrict__ states, OceanK oc,
                                                   uint8_t* __restrict__ ood, int8_t* __restrict__ posout,
@@ -4240,12 +4240,12 @@ __global__ __launch_bounds__(256) void k_sur_step(const SurPlanDev* __restrict__
     const SurTile tl = tiles[sfm::xcd_tile(blockIdx.x, gridDim.x)];
     const int g = (int)tl.group;
     const int t = threadIdx.x;
-    sfm::LayerW<SFM_IN_PAD> w0;   // requested now, used after the features
-    sfm::load_layer<SFM_IN_PAD>(P->W[g][0], w0);
+    sfm::TileW<SFM_IN_PAD> w0;   // requested now, used after the features
+    sfm::load_tile<SFM_IN_PAD>(P->W[g][0], t >> 6, w0);
     sfm::load_bias(P->B[g], bias);
     {
         // G lanes per unit build its context together
-        constexpr int G = 256 / TR;
+        constexpr int G = 64 * sfm::kWaves / TR;
         const int r = t / G, sub = t % G;
         const bool valid = (uint32_t)r < tl.nvalid;
         const uint32_t u = tl.unit0 + (valid ? (uint32_t)r : 0u);
@@ -4273,7 +4273,7 @@ __global__ __launch_bounds__(256) void k_sur_step(const SurPlanDev* __restrict__
         }
     }
     __syncthreads();
-    sfm::OutW ow;
+    sfm::TileW<SFM_HIDDEN> ow;
     sfm::mlp_hidden<TR>(P->W[g], bias, act, nullptr, w0, ow);
     const int lane = t & 63, wave = t >> 6;
     if (wave < TR / 32) {
@@ -4354,7 +4354,11 @@ extern "C" int sfh_surrogate_plan_create(sfh_batch b, uint32_t ngroups, const ui
     hipDeviceProp_t prop;
     if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess)
         cus = prop.multiProcessorCount;
-    const int TR = (total / 64 >= 2 * (uint64_t)cus) ? 64 : 32;
+    // Tiles of 32 units while one workgroup per CU holds them all (half the work
+    // per wavefront), 64 beyond: 4,096 units 15.9 us against 20.9 in tiles of
+    // 64, 8,192 16.6 / 21.3, 12,000 23.9 / 21.9, 16,384 25.3 / 22.7 (with four
+    // wavefronts per workgroup 18.5 us for 4,096 and 26 for 16,384).
+    const int TR = total > 32 * (uint64_t)cus ? 64 : 32;
     std::vector<SurTile> tiles;
     uint64_t u0 = 0;
     for (uint32_t g = 0; g < ngroups; ++g) {
@@ -4407,10 +4411,10 @@ extern "C" int sfh_surrogate_run(sfh_sur_plan p, sfh_ocean o, const double* d_st
     hipStream_t s = (hipStream_t)stream;
     const OceanK oc = make_oceank(o);
     if (p->TR == 64)
-        hipLaunchKernelGGL(k_sur_step<64>, dim3(p->ntiles), dim3(256), 0, s, p->d_plan, p->d_tiles, p->batch->d_units,
+        hipLaunchKernelGGL(k_sur_step<64>, dim3(p->ntiles), dim3(64 * sfm::kWaves), 0, s, p->d_plan, p->d_tiles, p->batch->d_units,
                            d_states, oc, d_ood, d_pos, d_ft);
     else
-        hipLaunchKernelGGL(k_sur_step<32>, dim3(p->ntiles), dim3(256), 0, s, p->d_plan, p->d_tiles, p->batch->d_units,
+        hipLaunchKernelGGL(k_sur_step<32>, dim3(p->ntiles), dim3(64 * sfm::kWaves), 0, s, p->d_plan, p->d_tiles, p->batch->d_units,
                            d_states, oc, d_ood, d_pos, d_ft);
     HIPCHK(hipGetLastError());
     return SFH_OK;

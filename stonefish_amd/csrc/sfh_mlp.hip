@@ -38,6 +38,8 @@ using sfm::gelu;
 using sfm::gelu_grad;
 using sfm::kActStride;
 using sfm::ld8;
+using sfm::load_tile;
+using sfm::TileW;
 
 static thread_local char g_err[512] = "";
 
@@ -365,7 +367,7 @@ struct NetSet {
 // Inference of TR consecutive rows of one network per workgroup (the fused
 // network of sfm_device.h).
 template <int TR>
-__global__ __launch_bounds__(256) void k_mlp_fused(NetSet ns, const uint16_t* __restrict__ x, uint32_t rows,
+__global__ __launch_bounds__(64 * sfm::kWaves, 4) void k_mlp_fused(NetSet ns, const uint16_t* __restrict__ x, uint32_t rows,
                                                    float* __restrict__ y)
 {
     __shared__ __attribute__((aligned(16))) uint16_t act[2][TR * kActStride];
@@ -374,11 +376,11 @@ __global__ __launch_bounds__(256) void k_mlp_fused(NetSet ns, const uint16_t* __
     if (row0 >= rows) return;
     int k = 0;
     while (k + 1 < ns.nnets && row0 >= ns.row_end[k]) ++k;
-    sfm::LayerW<SFM_IN_PAD> w0;
-    sfm::load_layer<SFM_IN_PAD>(ns.W[k][0], w0);
+    TileW<SFM_IN_PAD> w0;
+    load_tile<SFM_IN_PAD>(ns.W[k][0], threadIdx.x >> 6, w0);
     sfm::load_bias(ns.b[k], bias);
     __syncthreads();
-    sfm::OutW ow;
+    TileW<SFM_HIDDEN> ow;
     sfm::mlp_hidden<TR>(ns.W[k], bias, act, x + (size_t)row0 * SFM_IN_PAD, w0, ow);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (wave < TR / 32) {
@@ -491,6 +493,7 @@ struct Layer {
 
 struct sfm_net_t {
     uint32_t maxb = 0;
+    uint32_t cus = 256;              // compute units of the device the network was created on
     Layer L[SFM_LAYERS];
     uint16_t* H[SFM_LAYERS] = {};    // H[l] = input of layer l (H[0] unused: the caller's x)
     uint16_t* Ht[SFM_LAYERS] = {};   // transposed inputs
@@ -560,6 +563,10 @@ extern "C" int sfm_create(uint32_t max_batch, uint64_t seed, sfm_net* out)
         return fail(SFM_ERR_SIZE, "max_batch must be a positive multiple of %d", kSplitK);
     sfm_net_t* n = new sfm_net_t();
     n->maxb = max_batch;
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) == hipSuccess &&
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0)
+        n->cus = (uint32_t)cus;
     auto alloc = [&](void** p, size_t bytes) -> bool {
         if (hipMalloc(p, bytes) != hipSuccess) return false;
         return hipMemset(*p, 0, bytes) == hipSuccess;
@@ -705,8 +712,15 @@ static void forward_hidden(sfm_net_t* n, const uint16_t* x, uint32_t M, bool tra
     }
 }
 
-// Inference through the fused kernel: 64-row tiles when every network's row
-// count allows it, else 32-row tiles.
+// Inference through the fused kernel, in tiles of 32 or 64 rows.  A workgroup
+// runs its tile's layers one after the other, so while every CU has at most a
+// few workgroups the shorter tile is the faster (half the MFMAs and GELUs per
+// wavefront); once the CUs are full the longer one is, which reads the weights
+// (405 KB per tile, from L2) half as often.  Measured (tiles of 64 / 32 rows):
+// 4,096 rows 15.5 / 10.4 us, 8,192 15.5 / 10.7, 16,384 15.7 / 15.7, 24,576
+// 24.8 / 22.7, 32,768 26.1 / 29.6, 65,536 47.7 / 55.3 (554 TFLOP/s; 68.4 us
+// with four wavefronts per workgroup).  64-row tiles only where every
+// network's row count allows them.
 static int forward_group(const sfm_net* nets, uint32_t nnets, const uint32_t* counts, const uint16_t* x, float* y,
                          hipStream_t s)
 {
@@ -732,11 +746,12 @@ static int forward_group(const sfm_net* nets, uint32_t nnets, const uint32_t* co
     }
     if (total == 0) return SFM_OK;
     sfm_net_t* t = nets[0];
+    const bool tiles64 = even64 && total > 3 * 32 * (uint64_t)t->cus;
     time_begin(t, s);
-    if (even64)
-        hipLaunchKernelGGL(k_mlp_fused<64>, dim3((unsigned)(total / 64)), dim3(256), 0, s, ns, x, (uint32_t)total, y);
+    if (tiles64)
+        hipLaunchKernelGGL(k_mlp_fused<64>, dim3((unsigned)(total / 64)), dim3(64 * sfm::kWaves), 0, s, ns, x, (uint32_t)total, y);
     else
-        hipLaunchKernelGGL(k_mlp_fused<32>, dim3((unsigned)(total / 32)), dim3(256), 0, s, ns, x, (uint32_t)total, y);
+        hipLaunchKernelGGL(k_mlp_fused<32>, dim3((unsigned)(total / 32)), dim3(64 * sfm::kWaves), 0, s, ns, x, (uint32_t)total, y);
     time_end(t, s, forward_flops((uint32_t)total));
     HIPCHK(hipGetLastError());
     return SFM_OK;

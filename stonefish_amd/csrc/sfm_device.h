@@ -2,7 +2,7 @@
 // network library (sfh_mlp.hip: sfm_forward) and the hydrodynamics library
 // (sfh_hydro.hip: the one-launch surrogate step).  gfx950 only.
 //
-// A workgroup of four wavefronts runs TR rows (samples) of one network
+// A workgroup of eight wavefronts runs TR rows (samples) of one network
 // through all five layers.  The hidden activations stay in LDS (two TR x 256
 // BF16 buffers, row-major [sample][feature], row stride kActStride).  Each
 // layer is computed transposed, H'^T = W H^T: the weights are the MFMA's A
@@ -10,8 +10,13 @@
 // BF16 per network, L2-resident) and the activations its B operand (16-byte
 // LDS reads of H[sample][k..k+7]), so an accumulator lane holds four
 // consecutive output features of one sample and stores them with one 8-byte
-// LDS write.  Wavefront w owns output features [64 w, 64 w + 64) of each
-// hidden layer; the output layer is one 32-feature tile per 32-sample tile.
+// LDS write.  Wavefront w owns output features [32 w, 32 w + 32) of each
+// hidden layer (one 32-row tile of W, 64 registers of weights), so two
+// wavefronts share each SIMD, and with two workgroups on a CU four: one's
+// MFMAs run while the others' GELUs keep the VALU busy.  (Four wavefronts of 64
+// features each need 280 registers: one wavefront per SIMD, whose MFMA and GELU
+// phases only follow one another.)  The output layer is one 32-feature tile per
+// 32-sample tile.
 //
 // v_mfma_f32_32x32x16_bf16 operand layout (checked on the device by
 // sfm_probe_mfma): lane l holds A[l % 32][8 (l / 32) + 0..7] and
@@ -62,9 +67,9 @@ __device__ __forceinline__ uint32_t f2bf2(float a, float b)
 __device__ __forceinline__ int acc_row(int r, int lane) { return 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3); }
 
 // Fragment order of a layer's BF16 weights W [out x K] (row-major indices r,
-// c) for the fused inference: the 8 consecutive columns 16 s + 8 h .. + 7 of
-// row r = 64 w + 32 m + i are the 16 bytes that lane i + 32 h of wavefront w
-// feeds to k-step s of its m-th 32-row tile, and each (w, m, s) owns 1 KB of
+// c) for the fused kernels: the 8 consecutive columns 16 s + 8 h .. + 7 of
+// row r = 64 w + 32 m + i are the 16 bytes that lane i + 32 h feeds to k-step s
+// of the 32-row tile 2 w + m, and each (tile, s) owns 1 KB of
 // contiguous memory, read by one fully coalesced load instruction.  (Row-major
 // rows are 512 bytes apart, so the same fragments would touch 32 cache lines
 // per instruction.)
@@ -74,92 +79,81 @@ __host__ __device__ __forceinline__ size_t frag_index(int r, int c, int K)
     return ((((size_t)(2 * w + m) * (K / 16) + s) * 64) + i + 32 * h) * 8 + e;
 }
 
-// Weight fragments of one wavefront for a hidden layer with K inputs: rows
-// 64 w + l % 32 and 64 w + 32 + l % 32 of W, columns 8 (l / 32) + 16 s.
+static constexpr int kWaves = SFM_HIDDEN / 32;   // wavefronts of a workgroup: one per 32 features
+
+// Weight fragments of one 32-row tile of W [rows x K]: rows 32 tile + l % 32,
+// columns 8 (l / 32) + 16 s.
 template <int K>
-struct LayerW {
-    bf16x8 a[2][K / 16];
+struct TileW {
+    bf16x8 a[K / 16];
 };
 
-// Requests a layer's weight fragments (fragment order, frag_index) (2 K / 16 16-byte loads per lane, all
-// issued at once: one L2 round trip per layer instead of one per k-step).
-// The weights do not depend on the activations, so a caller issues them one
-// layer ahead, before the previous layer's epilogue.
+// Requests a tile's weight fragments (fragment order, frag_index; K / 16
+// 16-byte loads per lane, all issued at once: one L2 round trip per layer
+// instead of one per k-step).  The weights do not depend on the activations,
+// so a caller issues them one layer ahead, before the previous layer's epilogue.
 template <int K>
-__device__ __forceinline__ void load_layer(const uint16_t* __restrict__ w, LayerW<K>& L)
+__device__ __forceinline__ void load_tile(const uint16_t* __restrict__ w, int tile, TileW<K>& T)
 {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const uint16_t* wp0 = w + ((size_t)(2 * wave) * (K / 16) * 64 + lane) * 8;   // fragment order
-    const uint16_t* wp1 = wp0 + (size_t)(K / 16) * 512;
+    const uint16_t* p = w + ((size_t)tile * (K / 16) * 64 + (threadIdx.x & 63)) * 8;
 #pragma unroll
-    for (int s = 0; s < K / 16; ++s) {
-        L.a[0][s] = ld8g(wp0 + 512 * s);
-        L.a[1][s] = ld8g(wp1 + 512 * s);
-    }
+    for (int s = 0; s < K / 16; ++s) T.a[s] = ld8g(p + 512 * s);
 }
 
-// acc = W^T-tile products of a TR-row tile: in rows at `in` with row stride
-// in_stride (LDS, or global memory for the network input), K inputs.
-template <int TR, int K>
-__device__ __forceinline__ void layer_mma(const LayerW<K>& L, const uint16_t* in, int in_stride,
-                                          f32x16 (&acc)[2][TR / 32])
+// acc[nt] = W-tile products of rows 32 nt .. + 31: input rows at `in` with row
+// stride `stride` (LDS, or global memory for the network input), K inputs.
+template <int RT, int K>
+__device__ __forceinline__ void tile_mma(const TileW<K>& T, const uint16_t* in, int stride, f32x16 (&acc)[RT])
 {
-    constexpr int RT = TR / 32;
     const int lane = threadIdx.x & 63;
-    const uint16_t* bp = in + (lane & 31) * in_stride + (lane >> 5) * 8;
+    const uint16_t* bp = in + (lane & 31) * stride + (lane >> 5) * 8;
+    bf16x8 b[RT], n[RT];
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-        for (int nt = 0; nt < RT; ++nt) acc[mt][nt] = f32x16{};
+    for (int nt = 0; nt < RT; ++nt) {
+        acc[nt] = f32x16{};
+        b[nt] = ld8(bp + 32 * nt * stride);
+    }
+    // the operands of the next k-step are read while the current one
+    // multiplies; scheduled as written, since reads hoisted further cost
+    // registers the occupancy needs
 #pragma unroll
     for (int s = 0; s < K / 16; ++s) {
+        if (s + 1 < K / 16) {
+#pragma unroll
+            for (int nt = 0; nt < RT; ++nt) n[nt] = ld8(bp + 32 * nt * stride + 16 * (s + 1));
+        }
 #pragma unroll
         for (int nt = 0; nt < RT; ++nt) {
-            const bf16x8 b = ld8(bp + 32 * nt * in_stride + 16 * s);
-            acc[0][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(L.a[0][s], b, acc[0][nt], 0, 0, 0);
-            acc[1][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(L.a[1][s], b, acc[1][nt], 0, 0, 0);
+            acc[nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(T.a[s], b[nt], acc[nt], 0, 0, 0);
+            b[nt] = n[nt];
         }
+        if (s & 1) __builtin_amdgcn_sched_barrier(0);
     }
 }
 
 // out = gelu(acc + b) in BF16 (LDS rows, stride kActStride), then a barrier.
 // The bias is read from LDS: a global load here would have to wait for the
 // next layer's weight loads issued before it (loads complete in order).
-template <int TR>
-__device__ __forceinline__ void layer_store(const f32x16 (&acc)[2][TR / 32], const float* bias, uint16_t* out)
+template <int RT>
+__device__ __forceinline__ void layer_store(const f32x16 (&acc)[RT], const float* bias, uint16_t* out)
 {
-    constexpr int RT = TR / 32;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int lr = lane & 31, lq = (lane >> 5) * 4;
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt) {
+    for (int q = 0; q < 4; ++q) {
+        const int f0 = 32 * wave + 8 * q + lq;   // four consecutive output features
+        const float4 bq = *reinterpret_cast<const float4*>(bias + f0);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int f0 = 64 * wave + 32 * mt + 8 * q + lq;   // four consecutive output features
-            const float4 bq = *reinterpret_cast<const float4*>(bias + f0);
-#pragma unroll
-            for (int nt = 0; nt < RT; ++nt) {
-                const f32x16& A = acc[mt][nt];
-                uint2 pk;
-                pk.x = f2bf2(gelu(A[4 * q] + bq.x), gelu(A[4 * q + 1] + bq.y));
-                pk.y = f2bf2(gelu(A[4 * q + 2] + bq.z), gelu(A[4 * q + 3] + bq.w));
-                *reinterpret_cast<uint2*>(out + (32 * nt + lr) * kActStride + f0) = pk;
-            }
+        for (int nt = 0; nt < RT; ++nt) {
+            const f32x16& A = acc[nt];
+            uint2 pk;
+            pk.x = f2bf2(gelu(A[4 * q] + bq.x), gelu(A[4 * q + 1] + bq.y));
+            pk.y = f2bf2(gelu(A[4 * q + 2] + bq.z), gelu(A[4 * q + 3] + bq.w));
+            *reinterpret_cast<uint2*>(out + (32 * nt + lr) * kActStride + f0) = pk;
         }
     }
     __syncthreads();
-}
-
-// Output-layer weight fragments of one lane: W[l % 32][8 (l / 32) + 16 s].
-struct OutW {
-    bf16x8 a[SFM_HIDDEN / 16];
-};
-
-__device__ __forceinline__ void load_output(const uint16_t* __restrict__ w, OutW& L)
-{
-    const uint16_t* wp = w + (size_t)(threadIdx.x & 63) * 8;   // fragment order
-#pragma unroll
-    for (int s = 0; s < SFM_HIDDEN / 16; ++s) L.a[s] = ld8g(wp + 512 * s);
 }
 
 // Hidden-layer biases of one network into LDS (bias[l][f], l < 4); the
@@ -181,31 +175,33 @@ __device__ __forceinline__ void load_bias(const float* const* B, float (*bias)[S
 template <int TR>
 __device__ __forceinline__ void mlp_hidden(const uint16_t* const* W, const float (*B)[SFM_HIDDEN],
                                            uint16_t (*act)[TR * kActStride], const uint16_t* __restrict__ xg,
-                                           const LayerW<SFM_IN_PAD>& w0, OutW& ow)
+                                           const TileW<SFM_IN_PAD>& w0, TileW<SFM_HIDDEN>& ow)
 {
-    f32x16 acc[2][TR / 32];
-    LayerW<SFM_HIDDEN> wn;
+    constexpr int RT = TR / 32;
+    const int wave = threadIdx.x >> 6;
+    f32x16 acc[RT];
+    TileW<SFM_HIDDEN> wn;
     if (xg)
-        layer_mma<TR, SFM_IN_PAD>(w0, xg, SFM_IN_PAD, acc);
+        tile_mma<RT, SFM_IN_PAD>(w0, xg, SFM_IN_PAD, acc);
     else
-        layer_mma<TR, SFM_IN_PAD>(w0, act[1], kActStride, acc);
-    load_layer<SFM_HIDDEN>(W[1], wn);
-    layer_store<TR>(acc, B[0], act[0]);
-    layer_mma<TR, SFM_HIDDEN>(wn, act[0], kActStride, acc);
-    load_layer<SFM_HIDDEN>(W[2], wn);
-    layer_store<TR>(acc, B[1], act[1]);
-    layer_mma<TR, SFM_HIDDEN>(wn, act[1], kActStride, acc);
-    load_layer<SFM_HIDDEN>(W[3], wn);
-    layer_store<TR>(acc, B[2], act[0]);
-    layer_mma<TR, SFM_HIDDEN>(wn, act[0], kActStride, acc);
-    if ((threadIdx.x >> 6) < TR / 32) load_output(W[SFM_LAYERS - 1], ow);
-    layer_store<TR>(acc, B[3], act[1]);
+        tile_mma<RT, SFM_IN_PAD>(w0, act[1], kActStride, acc);
+    load_tile<SFM_HIDDEN>(W[1], wave, wn);
+    layer_store<RT>(acc, B[0], act[0]);
+    tile_mma<RT, SFM_HIDDEN>(wn, act[0], kActStride, acc);
+    load_tile<SFM_HIDDEN>(W[2], wave, wn);
+    layer_store<RT>(acc, B[1], act[1]);
+    tile_mma<RT, SFM_HIDDEN>(wn, act[1], kActStride, acc);
+    load_tile<SFM_HIDDEN>(W[3], wave, wn);
+    layer_store<RT>(acc, B[2], act[0]);
+    tile_mma<RT, SFM_HIDDEN>(wn, act[0], kActStride, acc);
+    if (wave < RT) load_tile<SFM_HIDDEN>(W[SFM_LAYERS - 1], 0, ow);   // one tile of outputs
+    layer_store<RT>(acc, B[3], act[1]);
 }
 
 // Output layer of sample tile `wave` (< TR / 32) from act[1]: on return,
 // registers 0..3 of lane l hold outputs 4 (l / 32) + 0..3 (bias included) of
 // sample 32 wave + l % 32.
-__device__ __forceinline__ void mlp_output(const OutW& L, const float* __restrict__ bias,
+__device__ __forceinline__ void mlp_output(const TileW<SFM_HIDDEN>& L, const float* __restrict__ bias,
                                            const uint16_t* __restrict__ in, float o[4])
 {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
