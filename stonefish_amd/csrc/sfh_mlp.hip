@@ -1,22 +1,19 @@
 // sfmlp: hand-written gfx950 BF16 MFMA kernels of the hydrodynamics surrogate
 // (forward, backward, Adam).  No counterpart in the reference.
 //
-// Every matrix product is C = A * Bt^T with A [rows x K] and Bt [cols x K] both
-// row-major and contiguous in K, so each lane's MFMA operands are one 16-byte
-// load: the forward pass keeps transposed copies of its activations (H^T) and
-// of the weights (W^T, refreshed by Adam) for the backward products.
-//
-//   forward   Z = H W^T + b,  H' = gelu(Z)                 (A = H,    Bt = W)
-//   dH        dH = dZ W                                     (A = dZ,   Bt = W^T)
-//   dW        dW = dZ^T H, split over the batch             (A = dZ^T, Bt = H^T)
-//
-// Tiles are 32x32 v_mfma_f32_32x32x16_bf16 accumulators: the products of the
-// 256-wide layers run 64x64 per workgroup with the operands staged in LDS,
-// the 32-wide ones one tile per wavefront.  The epilogues fuse bias, GELU
-// (exact erf) and its derivative, the loss and its gradient, BF16 rounding
-// and the transposed stores; the weight-gradient products also sum dZ's
-// columns (the bias gradient).  Weight- and bias-gradient partials of the
-// batch splits are summed in a fixed order by the Adam kernel.
+// A training step is three launches:
+//   k_train   a workgroup takes 64 rows of the batch through the forward pass,
+//             the loss and the backward products: the activations stay in LDS
+//             and the pre-activations in registers, and only the transposed
+//             layer inputs H^T and output gradients dZ^T (BF16) go to memory;
+//   k_wgrad   dW = dZ^T H of all five layers, split over the batch, with the
+//             bias gradients (row sums of dZ^T);
+//   k_adam    sums the splits' partials in a fixed order and steps Adam.
+// Matrix products outside k_train are C = A * Bt^T with A [rows x K] and Bt
+// [cols x K] both row-major and contiguous in K, so each lane's MFMA operands
+// are one 16-byte load.  Tiles are 32x32 v_mfma_f32_32x32x16_bf16
+// accumulators: the products of the 256-wide layers run 64x64 per workgroup
+// with the operands staged in LDS, the 32-wide ones one tile per wavefront.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -39,6 +36,7 @@ using sfm::gelu_grad;
 using sfm::kActStride;
 using sfm::ld8;
 using sfm::load_tile;
+using sfm::tile_mma;
 using sfm::TileW;
 
 static thread_local char g_err[512] = "";
@@ -65,6 +63,7 @@ static constexpr int kDims[SFM_LAYERS + 1] = {SFM_IN_PAD, SFM_HIDDEN, SFM_HIDDEN
 static constexpr int kReal[SFM_LAYERS + 1] = {SFM_IN, SFM_HIDDEN, SFM_HIDDEN, SFM_HIDDEN, SFM_HIDDEN, SFM_OUT};
 static constexpr int kSplitK = 256;   // batch rows per weight-gradient split
 static constexpr int kMaxSplits = 64; // batch splits of a weight-gradient product
+static constexpr int kTrainRows = 64; // batch rows per workgroup of k_train
 
 // Batch splits of layer l's weight-gradient product at most: the 256 x 256
 // products run 16 workgroups per split, the 32-wide ones 2, so the latter
@@ -82,7 +81,7 @@ static constexpr int max_splits(int l) { return kDims[l] == SFM_HIDDEN && kDims[
 // GEMM tile kernel
 // ---------------------------------------------------------------------------
 
-enum { EPI_HIDDEN = 0, EPI_OUT = 1, EPI_BWD = 2, EPI_WGRAD = 3 };
+enum { EPI_HIDDEN = 0, EPI_OUT = 1, EPI_WGRAD = 2 };
 
 struct GemmArgs {
     const uint16_t* A;      // [rows x K], lda
@@ -90,15 +89,10 @@ struct GemmArgs {
     int lda, ldb;
     int rows, cols, K, ksplit;
     const float* bias;      // [cols]                      (HIDDEN, OUT)
-    float* Z;               // [rows x cols] FP32          (HIDDEN: written; BWD: read)
-    uint16_t* H;            // [rows x cols] BF16          (HIDDEN, OUT-train, BWD)
-    uint16_t* Ht;           // [cols x rows] BF16          (optional)
-    const float* target;    // [rows x SFM_OUT]            (OUT-train)
+    uint16_t* H;            // [rows x cols] BF16          (HIDDEN)
     float* y;               // [rows x SFM_OUT]            (OUT)
-    float* loss;            //                              (OUT-train)
-    float scale;            // 1 / (rows * SFM_OUT)         (OUT-train)
     float* part;            // [ksplit][rows x cols] FP32  (WGRAD)
-    float* bpart;           // [ksplit][rows] FP32 row sums of A over each split (WGRAD, optional: bias gradient)
+    float* bpart;           // [ksplit][rows] FP32 row sums of A over each split (WGRAD: bias gradient)
 };
 
 __device__ __forceinline__ float sum8(const bf16x8& v)
@@ -108,211 +102,134 @@ __device__ __forceinline__ float sum8(const bf16x8& v)
 }
 
 
-// The epilogue of a wavefront's TM x TN tiles of C: tile (ti, tj) covers rows
-// (rt0 + ti) * 32 .. + 31 and columns (ct0 + tj) * 32 .. + 31.
-template <int EPI, int TM, int TN>
-__device__ __forceinline__ void gemm_store(const GemmArgs& g, const f32x16 (&acc)[TM][TN], int rt0, int ct0, int split,
-                                           int lane)
+// The epilogue of a wavefront's 32x32 tile of C at rows 32 rt and columns 32 ct.
+template <int EPI>
+__device__ __forceinline__ void gemm_store(const GemmArgs& g, const f32x16& A, int rt, int ct, int split, int lane)
 {
-    float sq = 0.f;
+    const int n = ct * 32 + (lane & 31), mb = rt * 32;
+    if (EPI == EPI_WGRAD) {
+        float* out = g.part + (size_t)split * g.rows * g.cols;
 #pragma unroll
-    for (int ti = 0; ti < TM; ++ti) {
-#pragma unroll
-        for (int tj = 0; tj < TN; ++tj) {
-            const f32x16& A = acc[ti][tj];
-            const int n = (ct0 + tj) * 32 + (lane & 31);
-            const int mb = (rt0 + ti) * 32;
-            if (EPI == EPI_WGRAD) {
-                float* out = g.part + (size_t)split * g.rows * g.cols;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) out[(size_t)(mb + acc_row(r, lane)) * g.cols + n] = A[r];
-                continue;
-            }
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                uint16_t hv[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int r = 4 * q + i;
-                    const int m = mb + acc_row(r, lane);
-                    const size_t idx = (size_t)m * g.cols + n;
-                    float out;
-                    if (EPI == EPI_HIDDEN) {
-                        const float z = A[r] + g.bias[n];
-                        if (g.Z) g.Z[idx] = z;
-                        out = gelu(z);
-                    } else if (EPI == EPI_OUT) {
-                        const float z = A[r] + g.bias[n];
-                        out = 0.f;
-                        if (n < SFM_OUT) {
-                            if (g.y) g.y[(size_t)m * SFM_OUT + n] = z;
-                            if (g.target) {
-                                const float d = z - g.target[(size_t)m * SFM_OUT + n];
-                                sq += d * d;
-                                out = 2.0f * d * g.scale;   // dLoss/dz
-                            }
-                        }
-                    } else {   // EPI_BWD: dZ = dH * gelu'(Z)
-                        out = A[r] * gelu_grad(g.Z[idx]);
-                    }
-                    hv[i] = f2bf(out);
-                    if (g.H) g.H[idx] = hv[i];
-                }
-                if (g.Ht) {   // four consecutive rows -> one 8-byte store of the transposed tile
-                    const int m0 = mb + 8 * q + 4 * (lane >> 5);
-                    uint2 pk;
-                    pk.x = (uint32_t)hv[0] | ((uint32_t)hv[1] << 16);
-                    pk.y = (uint32_t)hv[2] | ((uint32_t)hv[3] << 16);
-                    *reinterpret_cast<uint2*>(g.Ht + (size_t)n * g.rows + m0) = pk;
-                }
-            }
-        }
+        for (int r = 0; r < 16; ++r) out[(size_t)(mb + acc_row(r, lane)) * g.cols + n] = A[r];
+        return;
     }
-    if (EPI == EPI_OUT && g.target) {
+    const float b = g.bias[n];
 #pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) sq += __shfl_xor(sq, off, 64);
-        if (lane == 0) atomicAdd(g.loss, sq * g.scale);
+    for (int r = 0; r < 16; ++r) {
+        const int m = mb + acc_row(r, lane);
+        const float z = A[r] + b;
+        if (EPI == EPI_HIDDEN) g.H[(size_t)m * g.cols + n] = f2bf(gelu(z));
+        else if (n < SFM_OUT) g.y[(size_t)m * SFM_OUT + n] = z;
     }
 }
 
-// One wavefront computes a (32 TM) x (32 TN) block of C as TM x TN MFMA
-// tiles: per k-step TM + TN 16-byte operand loads feed TM * TN MFMAs.
-template <int EPI, int TM, int TN>
-__global__ __launch_bounds__(256) void k_gemm(GemmArgs g)
+// One wavefront computes a 32 x 32 tile of C: per k-step two 16-byte operand
+// loads feed an MFMA.  wave: the tile; split: the part of K.
+template <int EPI>
+__device__ __forceinline__ void gemm_wave(const GemmArgs& g, int wave, int split)
 {
     const int lane = threadIdx.x & 63;
-    const int wave = blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int blocks_n = g.cols / (32 * TN);
+    const int blocks_n = g.cols / 32;
     const int bm = wave / blocks_n, bn = wave - bm * blocks_n;
-    if (bm * 32 * TM >= g.rows) return;
-    const int split = blockIdx.y;
+    if (bm * 32 >= g.rows) return;
     const int kper = g.K / g.ksplit;
-    const int k0 = split * kper;
-    const int kk = (lane >> 5) * 8;
-    const uint16_t* ap[TM];
-    const uint16_t* bp[TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i) ap[i] = g.A + (size_t)((bm * TM + i) * 32 + (lane & 31)) * g.lda + k0 + kk;
-#pragma unroll
-    for (int j = 0; j < TN; ++j) bp[j] = g.Bt + (size_t)((bn * TN + j) * 32 + (lane & 31)) * g.ldb + k0 + kk;
-    f32x16 acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = f32x16{};
+    const int kk = split * kper + (lane >> 5) * 8;
+    const uint16_t* ap = g.A + (size_t)(bm * 32 + (lane & 31)) * g.lda + kk;
+    const uint16_t* bp = g.Bt + (size_t)(bn * 32 + (lane & 31)) * g.ldb + kk;
+    f32x16 acc = {};
     // The operands of the next kPF k-steps are in flight while the current
     // one multiplies (a ring of kPF register stages, refilled right after use):
     // a k-step waits for a load issued kPF steps earlier, not for the last one.
     constexpr int kPF = 4;
-    bf16x8 ra[kPF][TM], rb[kPF][TN];
+    bf16x8 ra[kPF], rb[kPF];
 #pragma unroll
     for (int s = 0; s < kPF; ++s)
         if (16 * s < kper) {
-#pragma unroll
-            for (int i = 0; i < TM; ++i) ra[s][i] = ld8g(ap[i] + 16 * s);
-#pragma unroll
-            for (int j = 0; j < TN; ++j) rb[s][j] = ld8g(bp[j] + 16 * s);
+            ra[s] = ld8g(ap + 16 * s);
+            rb[s] = ld8g(bp + 16 * s);
         }
     // the bias gradient rides along the weight gradient: the wavefronts of the
     // first column of tiles also sum their rows of A (each lane 8 of the 16 k
     // of a k-step, the two half-waves combined at the end)
-    const bool rsum = EPI == EPI_WGRAD && g.bpart && bn == 0;
-    float rs[TM] = {};
+    const bool rsum = EPI == EPI_WGRAD && bn == 0;
+    float rs = 0.f;
     for (int k0 = 0; k0 < kper; k0 += 16 * kPF) {
 #pragma unroll
         for (int s = 0; s < kPF; ++s) {
             const int k = k0 + 16 * s;
             if (k < kper) {
-                if (rsum) {
-#pragma unroll
-                    for (int i = 0; i < TM; ++i) rs[i] += sum8(ra[s][i]);
-                }
-#pragma unroll
-                for (int i = 0; i < TM; ++i)
-#pragma unroll
-                    for (int j = 0; j < TN; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ra[s][i], rb[s][j], acc[i][j], 0, 0, 0);
+                if (rsum) rs += sum8(ra[s]);
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ra[s], rb[s], acc, 0, 0, 0);
                 if (k + 16 * kPF < kper) {
-#pragma unroll
-                    for (int i = 0; i < TM; ++i) ra[s][i] = ld8g(ap[i] + k + 16 * kPF);
-#pragma unroll
-                    for (int j = 0; j < TN; ++j) rb[s][j] = ld8g(bp[j] + k + 16 * kPF);
+                    ra[s] = ld8g(ap + k + 16 * kPF);
+                    rb[s] = ld8g(bp + k + 16 * kPF);
                 }
             }
         }
     }
     if (rsum) {
-#pragma unroll
-        for (int i = 0; i < TM; ++i) {
-            const float v = rs[i] + __shfl_xor(rs[i], 32, 64);
-            if (lane < 32) g.bpart[(size_t)split * g.rows + (bm * TM + i) * 32 + lane] = v;
-        }
+        const float v = rs + __shfl_xor(rs, 32, 64);
+        if (lane < 32) g.bpart[(size_t)split * g.rows + bm * 32 + lane] = v;
     }
-    gemm_store<EPI, TM, TN>(g, acc, bm * TM, bn * TN, split, lane);
+    gemm_store<EPI>(g, acc, bm, bn, split, lane);
 }
 
 // Workgroup-tiled product for the 256-wide layers: the four wavefronts of a
-// workgroup, in a 2 x 2 arrangement, cover (64 WM) x (64 WN) of C, each
-// wavefront WM x WN 32x32 tiles.  K advances in chunks of kKC: the workgroup
-// copies the chunk's rows of A and of Bt into LDS once (the next chunk's
-// global loads in flight while the current one multiplies; two LDS buffers)
-// and the wavefronts read their MFMA operands from there, so an operand row
-// comes from L2 once per workgroup instead of once per wavefront that uses it.
+// workgroup, in a 2 x 2 arrangement, cover (64 T) x (64 T) of C, each T x T
+// tiles of 32 x 32.  K advances in chunks of kKC: the workgroup copies the
+// chunk's rows of A and of Bt into LDS once (the next chunk's global loads in
+// flight while the current one multiplies; two LDS buffers) and the wavefronts
+// read their MFMA operands from there, so an operand row comes from L2 once per
+// workgroup instead of once per wavefront that uses it.
 static constexpr int kKC = 64;            // K per chunk
 static constexpr int kLdsRow = kKC + 8;   // bf16 per LDS row: 16 bytes of padding against bank conflicts
 
-template <int EPI, int WM, int WN>
-__global__ __launch_bounds__(256) void k_gemm_lds(GemmArgs g)
+template <int T>
+struct GemmLds {
+    uint16_t A[2][64 * T * kLdsRow];
+    uint16_t B[2][64 * T * kLdsRow];
+};
+
+template <int EPI, int T>
+__device__ __forceinline__ void gemm_group(const GemmArgs& g, GemmLds<T>& L, int tile, int split)
 {
-    constexpr int BM = 64 * WM, BN = 64 * WN;
+    constexpr int BT = 64 * T;
     constexpr int SEG = kKC / 8;                 // 16-byte segments per row and chunk
-    constexpr int SA = BM * SEG / 256, SB = BN * SEG / 256;
-    static_assert(SA * 256 == BM * SEG && SB * 256 == BN * SEG, "tile rows must fill the workgroup's copies");
-    __shared__ __attribute__((aligned(16))) uint16_t As[2][BM * kLdsRow];
-    __shared__ __attribute__((aligned(16))) uint16_t Bs[2][BN * kLdsRow];
+    constexpr int SA = BT * SEG / 256;
     const int t = threadIdx.x, lane = t & 63, w = t >> 6, wm = w >> 1, wn = w & 1;
-    const int blocks_n = g.cols / BN;
-    const int bm = blockIdx.x / blocks_n, bn = blockIdx.x - bm * blocks_n;
-    const int split = blockIdx.y;
+    const int blocks_n = g.cols / BT;
+    const int bm = tile / blocks_n, bn = tile - bm * blocks_n;
     const int kper = g.K / g.ksplit;
     const int kbase = split * kper;
     const int nch = kper / kKC;
-    bf16x8 ra[SA], rb[SB];
+    bf16x8 ra[SA], rb[SA];
     auto gload = [&](int c) {
         const int k0 = kbase + c * kKC;
 #pragma unroll
         for (int i = 0; i < SA; ++i) {
             const int idx = t + 256 * i, row = idx / SEG, seg = idx % SEG;
-            ra[i] = ld8g(g.A + (size_t)(bm * BM + row) * g.lda + k0 + seg * 8);
-        }
-#pragma unroll
-        for (int i = 0; i < SB; ++i) {
-            const int idx = t + 256 * i, row = idx / SEG, seg = idx % SEG;
-            rb[i] = ld8g(g.Bt + (size_t)(bn * BN + row) * g.ldb + k0 + seg * 8);
+            ra[i] = ld8g(g.A + (size_t)(bm * BT + row) * g.lda + k0 + seg * 8);
+            rb[i] = ld8g(g.Bt + (size_t)(bn * BT + row) * g.ldb + k0 + seg * 8);
         }
     };
-    // bias gradient (see k_gemm): the workgroups of the first column of
+    // bias gradient (see gemm_wave): the workgroups of the first column of
     // tiles sum the rows of A they copy, each thread its 8-value segments
-    const bool rsum = EPI == EPI_WGRAD && g.bpart && bn == 0;
+    const bool rsum = EPI == EPI_WGRAD && bn == 0;
     float rs[SA] = {};
     auto lstore = [&](int buf) {
 #pragma unroll
         for (int i = 0; i < SA; ++i) {
             const int idx = t + 256 * i, row = idx / SEG, seg = idx % SEG;
-            *reinterpret_cast<bf16x8*>(&As[buf][row * kLdsRow + seg * 8]) = ra[i];
+            *reinterpret_cast<bf16x8*>(&L.A[buf][row * kLdsRow + seg * 8]) = ra[i];
+            *reinterpret_cast<bf16x8*>(&L.B[buf][row * kLdsRow + seg * 8]) = rb[i];
             if (rsum) rs[i] += sum8(ra[i]);
         }
-#pragma unroll
-        for (int i = 0; i < SB; ++i) {
-            const int idx = t + 256 * i, row = idx / SEG, seg = idx % SEG;
-            *reinterpret_cast<bf16x8*>(&Bs[buf][row * kLdsRow + seg * 8]) = rb[i];
-        }
     };
-    f32x16 acc[WM][WN];
+    f32x16 acc[T][T];
 #pragma unroll
-    for (int i = 0; i < WM; ++i)
+    for (int i = 0; i < T; ++i)
 #pragma unroll
-        for (int j = 0; j < WN; ++j) acc[i][j] = f32x16{};
+        for (int j = 0; j < T; ++j) acc[i][j] = f32x16{};
     gload(0);
     lstore(0);
     __syncthreads();
@@ -322,17 +239,16 @@ __global__ __launch_bounds__(256) void k_gemm_lds(GemmArgs g)
 #pragma unroll
         for (int s = 0; s < kKC / 16; ++s) {
             const int kk = 16 * s + (lane >> 5) * 8;
-            bf16x8 fa[WM], fb[WN];
+            bf16x8 fa[T], fb[T];
 #pragma unroll
-            for (int i = 0; i < WM; ++i)
-                fa[i] = *reinterpret_cast<const bf16x8*>(&As[buf][((wm * WM + i) * 32 + (lane & 31)) * kLdsRow + kk]);
+            for (int i = 0; i < T; ++i) {
+                fa[i] = ld8(&L.A[buf][((wm * T + i) * 32 + (lane & 31)) * kLdsRow + kk]);
+                fb[i] = ld8(&L.B[buf][((wn * T + i) * 32 + (lane & 31)) * kLdsRow + kk]);
+            }
 #pragma unroll
-            for (int j = 0; j < WN; ++j)
-                fb[j] = *reinterpret_cast<const bf16x8*>(&Bs[buf][((wn * WN + j) * 32 + (lane & 31)) * kLdsRow + kk]);
+            for (int i = 0; i < T; ++i)
 #pragma unroll
-            for (int i = 0; i < WM; ++i)
-#pragma unroll
-                for (int j = 0; j < WN; ++j)
+                for (int j = 0; j < T; ++j)
                     acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
         }
         if (c + 1 < nch) lstore(buf ^ 1);
@@ -347,10 +263,252 @@ __global__ __launch_bounds__(256) void k_gemm_lds(GemmArgs g)
             v += __shfl_xor(v, 2, 64);
             v += __shfl_xor(v, 4, 64);
             const int idx = t + 256 * i;
-            if (idx % SEG == 0) g.bpart[(size_t)split * g.rows + bm * BM + idx / SEG] = v;
+            if (idx % SEG == 0) g.bpart[(size_t)split * g.rows + bm * BT + idx / SEG] = v;
         }
     }
-    gemm_store<EPI, WM, WN>(g, acc, (bm * 2 + wm) * WM, (bn * 2 + wn) * WN, split, lane);
+#pragma unroll
+    for (int i = 0; i < T; ++i)
+#pragma unroll
+        for (int j = 0; j < T; ++j)
+            gemm_store<EPI>(g, acc[i][j], (bm * 2 + wm) * T + i, (bn * 2 + wn) * T + j, split, lane);
+}
+
+template <int EPI>
+__global__ __launch_bounds__(256) void k_gemm(GemmArgs g)
+{
+    gemm_wave<EPI>(g, blockIdx.x * 4 + (threadIdx.x >> 6), blockIdx.y);
+}
+
+template <int EPI>
+__global__ __launch_bounds__(256) void k_gemm_lds(GemmArgs g)
+{
+    __shared__ __attribute__((aligned(16))) GemmLds<1> L;
+    gemm_group<EPI, 1>(g, L, blockIdx.x, blockIdx.y);
+}
+
+// The weight- and bias-gradient products of all layers in one launch: 22 us for
+// a batch of 16,384 (one launch per layer with 64 x 64 tiles: 43 us; 64 x 64
+// tiles in one launch: 30).  Each operand column is read by two workgroups, from
+// memory the training kernel has just written (Infinity Cache).
+// Workgroups from block0 of a layer on are its: the 256 x 256 layers' by
+// (split, 128 x 128 tile), the 32-wide ones' by (split, four 32 x 32 tiles).
+static constexpr int kWgradTile = 128;
+
+struct WgradSet {
+    GemmArgs g[SFM_LAYERS];
+    int block0[SFM_LAYERS];
+};
+
+__global__ __launch_bounds__(256) void k_wgrad(WgradSet W)
+{
+    __shared__ __attribute__((aligned(16))) GemmLds<kWgradTile / 64> L;
+    int i = 0;
+    while (i + 1 < SFM_LAYERS && (int)blockIdx.x >= W.block0[i + 1]) ++i;
+    const GemmArgs& g = W.g[i];
+    const int b = (int)blockIdx.x - W.block0[i];
+    if (g.rows % kWgradTile == 0 && g.cols % kWgradTile == 0) {
+        const int tiles = (g.rows / kWgradTile) * (g.cols / kWgradTile);
+        gemm_group<EPI_WGRAD, kWgradTile / 64>(g, L, b % tiles, b / tiles);
+    } else {
+        const int groups = g.rows * g.cols / (4 * 32 * 32);
+        gemm_wave<EPI_WGRAD>(g, (b % groups) * 4 + (threadIdx.x >> 6), b / groups);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// forward, loss and backward of a training step
+// ---------------------------------------------------------------------------
+
+struct TrainArgs {
+    const uint16_t* x;              // [M x 32] BF16
+    const float* target;            // [M x SFM_OUT]
+    const uint16_t* W[SFM_LAYERS];  // weights in fragment order
+    const uint16_t* Wt[SFM_LAYERS]; // transposed weights [in x out] in fragment order (layers 1..4)
+    const float* b[SFM_LAYERS];
+    uint16_t* Ht[SFM_LAYERS];       // layer inputs, transposed [in x ldt]
+    uint16_t* dZt[SFM_LAYERS];      // layer output gradients, transposed [out x ldt]
+    float* loss_part;               // per workgroup
+    float scale;                    // 1 / (M * SFM_OUT)
+    int ldt;
+};
+
+// Transposes 4 x 4 BF16 values over each four lanes: lane i brings four
+// features of row i and takes four rows of feature quad_feature(i), so the
+// transposed tile goes to memory in 8-byte stores (in 2-byte ones k_train took
+// 46 us instead of 40 on 16,384 rows).
+__device__ __forceinline__ uint32_t quad_feature(int lane) { return ((lane & 1) << 1) | ((lane >> 1) & 1); }
+
+__device__ __forceinline__ uint2 quad_transpose(uint2 v, int lane)
+{
+    const bool odd = lane & 1, up = lane & 2;
+    const uint32_t r1 = (uint32_t)__builtin_amdgcn_mov_dpp((int)(odd ? v.x : v.y), 0xB1, 0xf, 0xf, true);   // lane ^ 1
+    const uint32_t a = odd ? r1 : v.x, b = odd ? v.y : r1;   // rows i & ~1 and i | 1, two features
+    const uint32_t lo = __builtin_amdgcn_perm(b, a, 0x05040100u), hi = __builtin_amdgcn_perm(b, a, 0x07060302u);
+    const uint32_t r2 = (uint32_t)__builtin_amdgcn_mov_dpp((int)(up ? lo : hi), 0x4E, 0xf, 0xf, true);      // lane ^ 2
+    return up ? make_uint2(r2, hi) : make_uint2(lo, r2);
+}
+
+// A wavefront's tile of BF16 values to the LDS activations ([row][feature])
+// and, transposed, to memory: f(acc value, index) gives the value.
+template <typename F>
+__device__ __forceinline__ void tile_store(uint16_t* act, uint16_t* __restrict__ outt, uint32_t ldt, int f0, F f)
+{
+    const int lane = threadIdx.x & 63, lr = lane & 31, lq = (lane >> 5) * 4;
+    const uint32_t fi = quad_feature(lane);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int fq = f0 + 8 * q + lq;   // four consecutive features
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt) {
+            uint2 pk;
+            pk.x = f2bf2(f(nt, 4 * q), f(nt, 4 * q + 1));
+            pk.y = f2bf2(f(nt, 4 * q + 2), f(nt, 4 * q + 3));
+            *reinterpret_cast<uint2*>(act + (32 * nt + lr) * kActStride + fq) = pk;
+            const uint2 tr = quad_transpose(pk, lane);
+            const uint32_t o = ((uint32_t)fq + fi) * ldt + 32u * nt + (uint32_t)(lr & ~3);   // below 2^31: ldt <= 2^22
+            *reinterpret_cast<uint2*>(outt + o) = tr;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// One workgroup of eight wavefronts: 64 rows of the batch forward and back.
+// Wavefront w owns features 32 w .. + 31 of every hidden layer in both
+// directions, so the pre-activations Z that gelu' needs on the way back stay
+// where the forward pass left them: 32 registers a layer (layer 0's in LDS)
+// beside 64 for the weights requested one layer ahead, which leaves two
+// wavefronts per SIMD.  Products are W H^T and W^T dZ^T (the weights the MFMA's
+// A operand, in fragment order); the sums over K run in the order of the
+// per-layer kernels, so the gradients are theirs bit for bit.  16,384 rows
+// (one workgroup per CU): 40 us, where the launches it replaces (a transpose,
+// five forward and four backward products through Z, H, H^T, dZ and dZ^T in
+// memory) took 155.  About 6 us of it wait on the 70 MB of transposed stores,
+// 13 are the GELUs and their derivatives (VALU and transcendentals), the rest
+// the products at one workgroup's latency per layer.
+__global__ __launch_bounds__(512, 2) void k_train(TrainArgs P)
+{
+    __shared__ __attribute__((aligned(16))) uint16_t act[2][kTrainRows * kActStride];
+    __shared__ __attribute__((aligned(16))) float bias[SFM_LAYERS - 1][SFM_HIDDEN];
+    __shared__ float4 z0[8][512];   // layer 0's Z, each thread its own
+    __shared__ float lsum[2];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, lq = (lane >> 5) * 4, f0 = 32 * wave;
+    const size_t row0 = (size_t)blockIdx.x * kTrainRows;
+    const uint16_t* xg = P.x + row0 * SFM_IN_PAD;
+    TileW<SFM_IN_PAD> w0;
+    load_tile<SFM_IN_PAD>(P.W[0], wave, w0);
+    sfm::load_bias(P.b, bias);
+    {   // x^T: thread t takes row t % 64, inputs 4 (t / 64) .. + 3
+        const int r = t & 63, c = 4 * (t >> 6);
+        const uint2 v = *reinterpret_cast<const uint2*>(xg + (size_t)r * SFM_IN_PAD + c);
+        uint16_t* o = P.Ht[0] + (size_t)c * P.ldt + row0 + r;
+        o[0] = (uint16_t)v.x;
+        o[P.ldt] = (uint16_t)(v.x >> 16);
+        o[2 * (size_t)P.ldt] = (uint16_t)v.y;
+        o[3 * (size_t)P.ldt] = (uint16_t)(v.y >> 16);
+    }
+    __syncthreads();
+    f32x16 Z[SFM_LAYERS - 1][2];
+    TileW<SFM_HIDDEN> wn;
+    tile_mma<2, SFM_IN_PAD>(w0, xg, SFM_IN_PAD, Z[0]);
+#pragma unroll
+    for (int l = 0; l < SFM_LAYERS - 1; ++l) {
+        if (l > 0) tile_mma<2, SFM_HIDDEN>(wn, act[(l - 1) & 1], kActStride, Z[l]);
+        if (l < SFM_LAYERS - 2) load_tile<SFM_HIDDEN>(P.W[l + 1], wave, wn);
+        else if (wave < 2) load_tile<SFM_HIDDEN>(P.W[l + 1], 0, wn);   // the output layer: one tile of features
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const float4 b = *reinterpret_cast<const float4*>(&bias[l][f0 + 8 * q + lq]);
+#pragma unroll
+            for (int nt = 0; nt < 2; ++nt) {
+                Z[l][nt][4 * q] += b.x;
+                Z[l][nt][4 * q + 1] += b.y;
+                Z[l][nt][4 * q + 2] += b.z;
+                Z[l][nt][4 * q + 3] += b.w;
+            }
+        }
+        if (l == 0) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const f32x16& z = Z[0][i >> 2];
+                const int r = 4 * (i & 3);
+                z0[i][t] = make_float4(z[r], z[r + 1], z[r + 2], z[r + 3]);
+            }
+        }
+        tile_store(act[l & 1], P.Ht[l + 1] + row0, P.ldt, f0, [&](int nt, int r) { return gelu(Z[l][nt][r]); });
+        __syncthreads();
+    }
+    // output layer, loss and its gradient: wavefronts 0 and 1 a row tile each;
+    // dZ of the 32 padded outputs goes to act[0] (columns 0..31), whose last
+    // reader is behind the barrier above
+    TileW<SFM_OUT_PAD> wo;
+    load_tile<SFM_OUT_PAD>(P.Wt[SFM_LAYERS - 1], wave, wo);
+    if (wave < 2) {
+        const int lr = lane & 31, row = 32 * wave + lr;
+        const uint16_t* bp = act[1] + row * kActStride + (lane >> 5) * 8;
+        f32x16 acc = {};
+#pragma unroll
+        for (int s = 0; s < SFM_HIDDEN / 16; ++s)
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wn.a[s], ld8(bp + 16 * s), acc, 0, 0, 0);
+        const float* tg = P.target + (row0 + row) * SFM_OUT;
+        float sq = 0.f, dz[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {   // registers 0..3 of lane l: outputs 4 (l / 32) + 0..3
+            dz[i] = 0.f;
+            if (lq + i < SFM_OUT) {
+                const float z = acc[i] + P.b[SFM_LAYERS - 1][lq + i];
+                const float d = z - tg[lq + i];
+                sq += d * d;
+                dz[i] = 2.0f * d * P.scale;   // dLoss/dz
+            }
+        }
+        uint2 pk;
+        pk.x = f2bf2(dz[0], dz[1]);
+        pk.y = f2bf2(dz[2], dz[3]);
+        uint16_t* a = act[0] + row * kActStride;
+        *reinterpret_cast<uint2*>(a + lq) = pk;
+#pragma unroll
+        for (int c = 8; c < SFM_OUT_PAD; c += 8) *reinterpret_cast<uint2*>(a + c + lq) = make_uint2(0u, 0u);
+        uint16_t* o = P.dZt[SFM_LAYERS - 1] + row0 + row;
+        const uint32_t pw[2] = {pk.x, pk.y};
+#pragma unroll
+        for (int c = 0; c < SFM_OUT_PAD; c += 8)   // the padded outputs' rows are zero
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                o[(size_t)(c + lq + i) * P.ldt] = c == 0 ? (uint16_t)(pw[i >> 1] >> (16 * (i & 1))) : (uint16_t)0;
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) sq += __shfl_xor(sq, off, 64);
+        if (lane == 0) lsum[wave] = sq * P.scale;
+    }
+    __syncthreads();
+    if (t == 0) P.loss_part[blockIdx.x] = lsum[0] + lsum[1];
+    // back: dZ of hidden layer l = (W^T of the layer above dZ) * gelu'(Z)
+    f32x16 acc[2];
+    tile_mma<2, SFM_OUT_PAD>(wo, act[0], kActStride, acc);
+#pragma unroll
+    for (int l = SFM_LAYERS - 2; l >= 0; --l) {
+        // the gradients alternate between the LDS buffers from act[1] on
+        const int buf = (SFM_LAYERS - 1 - l) & 1;
+        if (l < SFM_LAYERS - 2) tile_mma<2, SFM_HIDDEN>(wn, act[buf ^ 1], kActStride, acc);
+        if (l > 0) load_tile<SFM_HIDDEN>(P.Wt[l], wave, wn);
+        __builtin_amdgcn_sched_barrier(0);
+        // gelu' shares its erf and exponential with the forward pass's gelu:
+        // hidden from the compiler, which would keep two more values per
+        // activation alive across the whole kernel
+        if (l == 0) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float4 z = z0[i][t];
+                const int r = 4 * (i & 3);
+                Z[0][i >> 2][r] = z.x; Z[0][i >> 2][r + 1] = z.y; Z[0][i >> 2][r + 2] = z.z; Z[0][i >> 2][r + 3] = z.w;
+            }
+        }
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt) asm volatile("" : "+v"(Z[l][nt]));
+        tile_store(act[buf], P.dZt[l] + row0, P.ldt, f0,
+                   [&](int nt, int r) { return acc[nt][r] * gelu_grad(Z[l][nt][r]); });
+        if (l > 0) __syncthreads();
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -398,15 +556,6 @@ __global__ __launch_bounds__(64 * sfm::kWaves, 4) void k_mlp_fused(NetSet ns, co
 // small kernels
 // ---------------------------------------------------------------------------
 
-// Transposes x [rows x cols] (BF16) into xt [cols x rows].
-__global__ void k_transpose(const uint16_t* __restrict__ x, int rows, int cols, uint16_t* __restrict__ xt)
-{
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (size_t)rows * cols) return;
-    int r = (int)(i / cols), c = (int)(i - (size_t)r * cols);
-    xt[(size_t)c * rows + r] = x[i];
-}
-
 // Adam on n parameters of a [rows x cols] matrix (cols = 1 for biases): the
 // gradient is the sum of nsplit partials (fixed order); keeps the FP32 master
 // copy and refreshes the BF16 copy and its transpose.
@@ -417,13 +566,17 @@ struct AdamSeg {
     float *w, *mo, *ve;
     const float* part;
     float* gsave;
-    uint16_t *wb, *wbt, *wp;
+    uint16_t *wb, *wtp, *wp;          // row-major; transposed and plain in fragment order
     int nsplit, rows, cols, block0;   // block0: first workgroup of this tensor in the launch
 };
 
 struct AdamSet {
     AdamSeg seg[2 * SFM_LAYERS];
     int nseg;
+    int nblk;                 // workgroups of the tensors; one more sums the loss
+    const float* loss_part;   // k_train's, one per workgroup
+    int nloss;
+    float* loss;
 };
 
 // Adam with bias correction for every weight and bias tensor of the network
@@ -431,6 +584,17 @@ struct AdamSet {
 __global__ __launch_bounds__(256) void k_adam(AdamSet S, float lr, float b1, float b2, float eps, float bc1,
                                               float bc2)
 {
+    if ((int)blockIdx.x >= S.nblk) {   // the loss: fixed order
+        __shared__ float red[4];
+        float v = 0.f;
+        for (int i = threadIdx.x; i < S.nloss; i += 256) v += S.loss_part[i];
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+        __syncthreads();
+        if (threadIdx.x == 0) *S.loss = (red[0] + red[1]) + (red[2] + red[3]);
+        return;
+    }
     int si = 0;
     while (si + 1 < S.nseg && (int)blockIdx.x >= S.seg[si + 1].block0) ++si;
     const AdamSeg& g = S.seg[si];
@@ -438,8 +602,15 @@ __global__ __launch_bounds__(256) void k_adam(AdamSet S, float lr, float b1, flo
     const int i = ((int)blockIdx.x - g.block0) * (int)blockDim.x + (int)threadIdx.x;
     if (i >= n) return;
     float gr = 0.f;
-#pragma unroll 8
-    for (int s = 0; s < g.nsplit; ++s) gr += g.part[(size_t)s * n + i];   // loads in flight 8 at a time
+    int s = 0;
+    for (; s + 32 <= g.nsplit; s += 32) {   // 32 loads in flight, summed in order
+        float v[32];
+#pragma unroll
+        for (int k = 0; k < 32; ++k) v[k] = g.part[(size_t)(s + k) * n + i];
+#pragma unroll
+        for (int k = 0; k < 32; ++k) gr += v[k];
+    }
+    for (; s < g.nsplit; ++s) gr += g.part[(size_t)s * n + i];
     g.gsave[i] = gr;
     const float m = b1 * g.mo[i] + (1.f - b1) * gr;
     const float v = b2 * g.ve[i] + (1.f - b2) * gr * gr;
@@ -451,9 +622,18 @@ __global__ __launch_bounds__(256) void k_adam(AdamSet S, float lr, float b1, flo
         const uint16_t h = f2bf(wn);
         g.wb[i] = h;
         const int r = i / g.cols, c = i - r * g.cols;
-        g.wbt[(size_t)c * g.rows + r] = h;
+        g.wtp[sfm::frag_index(c, r, g.rows)] = h;
         g.wp[sfm::frag_index(r, c, g.cols)] = h;
     }
+}
+
+// The summed gradients of one layer: n weights, then nb biases.
+__global__ __launch_bounds__(256) void k_gradients(const float* __restrict__ gw, const float* __restrict__ gb, int n,
+                                                   int nb, float* __restrict__ dw, float* __restrict__ db)
+{
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) dw[i] = gw[i];
+    else if (i < n + nb) db[i - n] = gb[i - n];
 }
 
 __global__ void k_to_bf16(const float* __restrict__ x, uint16_t* __restrict__ y, uint64_t n)
@@ -487,18 +667,19 @@ __global__ void k_probe(const uint16_t* __restrict__ a, const uint16_t* __restri
 struct Layer {
     float *W = nullptr, *b = nullptr, *mW = nullptr, *vW = nullptr, *mb = nullptr, *vb = nullptr;
     float *gW = nullptr, *gb = nullptr;
-    uint16_t *Wb = nullptr, *Wbt = nullptr;
-    uint16_t* Wp = nullptr;   // BF16 in fragment order (sfm::frag_index) for the fused inference
+    uint16_t* Wb = nullptr;
+    uint16_t* Wp = nullptr;   // BF16 in fragment order (sfm::frag_index) for the fused kernels
+    uint16_t* Wtp = nullptr;  // the transpose [in x out] in fragment order, for the backward products
 };
 
 struct sfm_net_t {
     uint32_t maxb = 0;
     uint32_t cus = 256;              // compute units of the device the network was created on
     Layer L[SFM_LAYERS];
-    uint16_t* H[SFM_LAYERS] = {};    // H[l] = input of layer l (H[0] unused: the caller's x)
-    uint16_t* Ht[SFM_LAYERS] = {};   // transposed inputs
-    float* Z[SFM_LAYERS] = {};       // pre-activations of layers 0..3 outputs (Z[l] = output of layer l)
-    uint16_t *dZ[2] = {}, *dZt[2] = {};
+    uint16_t* H[SFM_LAYERS] = {};    // H[l] = input of layer l (H[0] unused: the caller's x), per-layer inference
+    uint16_t* Ht[SFM_LAYERS] = {};   // training: layer inputs, transposed
+    uint16_t* dZt[SFM_LAYERS] = {};  // training: layer output gradients, transposed
+    float* loss_part = nullptr;      // per workgroup of k_train
     float* part[SFM_LAYERS] = {};    // per layer: weight-gradient partials of the batch splits (<= max_splits)
     float* dbias[SFM_LAYERS] = {};   // per layer: bias-gradient partials of the same splits
     uint64_t step = 0;
@@ -522,11 +703,11 @@ static void net_free(sfm_net_t* n)
     for (Layer& l : n->L) {
         for (float* p : {l.W, l.b, l.mW, l.vW, l.mb, l.vb, l.gW, l.gb}) hipFree(p);
         hipFree(l.Wb);
-        hipFree(l.Wbt);
+        hipFree(l.Wtp);
         hipFree(l.Wp);
     }
-    for (int i = 0; i < SFM_LAYERS; ++i) { hipFree(n->H[i]); hipFree(n->Ht[i]); hipFree(n->Z[i]); }
-    for (int i = 0; i < 2; ++i) { hipFree(n->dZ[i]); hipFree(n->dZt[i]); }
+    for (int i = 0; i < SFM_LAYERS; ++i) { hipFree(n->H[i]); hipFree(n->Ht[i]); hipFree(n->dZt[i]); }
+    hipFree(n->loss_part);
     for (int i = 0; i < SFM_LAYERS; ++i) { hipFree(n->part[i]); hipFree(n->dbias[i]); }
     for (int i = 0; i < 2; ++i)
         if (n->ev[i]) hipEventDestroy(n->ev[i]);
@@ -535,7 +716,7 @@ static void net_free(sfm_net_t* n)
 static int upload_layer(sfm_net_t* n, int l, const float* w, const float* b)
 {
     const int rows = kDims[l + 1], cols = kDims[l];
-    std::vector<uint16_t> wb((size_t)rows * cols), wbt((size_t)rows * cols), wp((size_t)rows * cols);
+    std::vector<uint16_t> wb((size_t)rows * cols), wtp((size_t)rows * cols), wp((size_t)rows * cols);
     for (int r = 0; r < rows; ++r)
         for (int c = 0; c < cols; ++c) {
             float f = w[(size_t)r * cols + c];
@@ -544,14 +725,14 @@ static int upload_layer(sfm_net_t* n, int l, const float* w, const float* b)
             u += 0x7fffu + ((u >> 16) & 1u);
             uint16_t h = (uint16_t)(u >> 16);
             wb[(size_t)r * cols + c] = h;
-            wbt[(size_t)c * rows + r] = h;
+            wtp[sfm::frag_index(c, r, rows)] = h;
             wp[sfm::frag_index(r, c, cols)] = h;
         }
     Layer& L = n->L[l];
     HIPCHK(hipMemcpy(L.W, w, sizeof(float) * rows * cols, hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(L.b, b, sizeof(float) * rows, hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(L.Wb, wb.data(), 2 * wb.size(), hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(L.Wbt, wbt.data(), 2 * wbt.size(), hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpy(L.Wtp, wtp.data(), 2 * wtp.size(), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(L.Wp, wp.data(), 2 * wp.size(), hipMemcpyHostToDevice));
     return SFM_OK;
 }
@@ -578,14 +759,12 @@ extern "C" int sfm_create(uint32_t max_batch, uint64_t seed, sfm_net* out)
         ok = alloc((void**)&L.W, 4 * nw) && alloc((void**)&L.b, 4 * nb) && alloc((void**)&L.mW, 4 * nw) &&
              alloc((void**)&L.vW, 4 * nw) && alloc((void**)&L.mb, 4 * nb) && alloc((void**)&L.vb, 4 * nb) &&
              alloc((void**)&L.gW, 4 * nw) && alloc((void**)&L.gb, 4 * nb) && alloc((void**)&L.Wb, 2 * nw) &&
-             alloc((void**)&L.Wbt, 2 * nw) && alloc((void**)&L.Wp, 2 * nw);
-        if (ok && l > 0) ok = alloc((void**)&n->H[l], 2 * (size_t)max_batch * kDims[l]) &&
-                               alloc((void**)&n->Z[l], 4 * (size_t)max_batch * kDims[l]);
-        if (ok) ok = alloc((void**)&n->Ht[l], 2 * (size_t)max_batch * kDims[l]);
+             alloc((void**)&L.Wtp, 2 * nw) && alloc((void**)&L.Wp, 2 * nw);
+        if (ok && l > 0) ok = alloc((void**)&n->H[l], 2 * (size_t)max_batch * kDims[l]);
+        if (ok) ok = alloc((void**)&n->Ht[l], 2 * (size_t)max_batch * kDims[l]) &&
+                     alloc((void**)&n->dZt[l], 2 * (size_t)max_batch * kDims[l + 1]);
     }
-    for (int i = 0; i < 2 && ok; ++i)
-        ok = alloc((void**)&n->dZ[i], 2 * (size_t)max_batch * SFM_HIDDEN) &&
-             alloc((void**)&n->dZt[i], 2 * (size_t)max_batch * SFM_HIDDEN);
+    if (ok) ok = alloc((void**)&n->loss_part, 4 * (size_t)(max_batch / kTrainRows));
     for (int l = 0; l < SFM_LAYERS && ok; ++l)
         ok = alloc((void**)&n->part[l], 4 * (size_t)max_splits(l) * kDims[l + 1] * kDims[l]) &&
              alloc((void**)&n->dbias[l], 4 * (size_t)max_splits(l) * kDims[l + 1]);
@@ -637,27 +816,16 @@ extern "C" int sfm_layer_io(sfm_net n, int l, float* w, float* b, int set)
     return SFM_OK;
 }
 
-// The products whose rows and columns are multiples of 64 and whose K (per
-// batch split) is a multiple of kKC run workgroup-tiled through LDS, 64 x 64
-// per workgroup (the 256-wide layers' forward, backward and weight-gradient
-// products: 1,024 workgroups for 16,384 x 256, where 128 x 128 tiles leave
-// 256 and the operand latency exposed; measured 97 vs 85 TFLOP/s training);
-// the 32-wide ones (the first layer's K, the output layer) one 32 x 32 tile
-// per wavefront (k_gemm).
+// Products whose rows and columns are multiples of 64 and whose K is a multiple
+// of kKC run workgroup-tiled through LDS, 64 x 64 per workgroup, the 32-wide
+// ones (the first layer's K, the output layer) one 32 x 32 tile per wavefront.
 template <int EPI>
 static void launch_gemm(const GemmArgs& g, hipStream_t s)
 {
-    if ((g.K / g.ksplit) % kKC == 0 && g.rows % 64 == 0 && g.cols % 64 == 0) {
-        hipLaunchKernelGGL((k_gemm_lds<EPI, 1, 1>), dim3((g.rows / 64) * (g.cols / 64), g.ksplit), dim3(256), 0, s, g);
-        return;
-    }
-    const bool m2 = false, n2 = false;
-    const int blocks = (g.rows / (m2 ? 64 : 32)) * (g.cols / (n2 ? 64 : 32));
-    const dim3 grid((blocks + 3) / 4, g.ksplit);
-    if (m2 && n2) hipLaunchKernelGGL((k_gemm<EPI, 2, 2>), grid, dim3(256), 0, s, g);
-    else if (m2) hipLaunchKernelGGL((k_gemm<EPI, 2, 1>), grid, dim3(256), 0, s, g);
-    else if (n2) hipLaunchKernelGGL((k_gemm<EPI, 1, 2>), grid, dim3(256), 0, s, g);
-    else hipLaunchKernelGGL((k_gemm<EPI, 1, 1>), grid, dim3(256), 0, s, g);
+    if (g.K % kKC == 0 && g.rows % 64 == 0 && g.cols % 64 == 0)
+        hipLaunchKernelGGL(k_gemm_lds<EPI>, dim3((g.rows / 64) * (g.cols / 64)), dim3(256), 0, s, g);
+    else
+        hipLaunchKernelGGL(k_gemm<EPI>, dim3((g.rows / 32 * (g.cols / 32) + 3) / 4), dim3(256), 0, s, g);
 }
 
 static GemmArgs gemm(const uint16_t* A, int lda, const uint16_t* Bt, int ldb, int rows, int cols, int K)
@@ -699,15 +867,14 @@ static void time_end(sfm_net_t* n, hipStream_t s, double flops)
     n->pending_flops = flops;
 }
 
-// Forward through the hidden layers: x -> H[1..4] (and Z, H^T when training).
-static void forward_hidden(sfm_net_t* n, const uint16_t* x, uint32_t M, bool train, hipStream_t s)
+// Forward through the hidden layers: x -> H[1..4].
+static void forward_hidden(sfm_net_t* n, const uint16_t* x, uint32_t M, hipStream_t s)
 {
     for (int l = 0; l < SFM_LAYERS - 1; ++l) {
         const uint16_t* A = (l == 0) ? x : n->H[l];
         GemmArgs g = gemm(A, kDims[l], n->L[l].Wb, kDims[l], (int)M, kDims[l + 1], kDims[l]);
         g.bias = n->L[l].b;
         g.H = n->H[l + 1];
-        if (train) { g.Z = n->Z[l + 1]; g.Ht = n->Ht[l + 1]; }
         launch_gemm<EPI_HIDDEN>(g, s);
     }
 }
@@ -770,8 +937,8 @@ extern "C" int sfm_forward_group(const sfm_net* nets, uint32_t nnets, const uint
     return forward_group(nets, nnets, counts, x, y, (hipStream_t)stream);
 }
 
-// Inference through the per-layer kernels of the training path (kept for
-// checking the fused kernel against them).
+// Inference through per-layer kernels (kept for checking the fused kernel
+// against them).
 extern "C" int sfm_forward_layers(sfm_net n, const uint16_t* x, uint32_t batch, float* y, void* stream)
 {
     if (!n || !x || !y) return fail(SFM_ERR_INVALID, "null argument");
@@ -779,7 +946,7 @@ extern "C" int sfm_forward_layers(sfm_net n, const uint16_t* x, uint32_t batch, 
     if ((uintptr_t)x % 16) return fail(SFM_ERR_INVALID, "x must be 16-byte aligned");
     hipStream_t s = (hipStream_t)stream;
     time_begin(n, s);
-    forward_hidden(n, x, batch, false, s);
+    forward_hidden(n, x, batch, s);
     GemmArgs g = gemm(n->H[SFM_LAYERS - 1], SFM_HIDDEN, n->L[SFM_LAYERS - 1].Wb, SFM_HIDDEN, (int)batch, SFM_OUT_PAD,
                       SFM_HIDDEN);
     g.bias = n->L[SFM_LAYERS - 1].b;
@@ -800,65 +967,58 @@ extern "C" int sfm_train_step(sfm_net n, const uint16_t* x, const float* target,
     hipStream_t s = (hipStream_t)stream;
     const int M = (int)batch;
     time_begin(n, s);
-    HIPCHK(hipMemsetAsync(loss, 0, sizeof(float), s));
-    // x^T for the first layer's weight gradient
-    hipLaunchKernelGGL(k_transpose, dim3((M * SFM_IN_PAD + 255) / 256), dim3(256), 0, s, x, M, SFM_IN_PAD, n->Ht[0]);
-    forward_hidden(n, x, batch, true, s);
-    // output layer: loss and dLoss/dZ (row-major and transposed)
-    {
-        GemmArgs g = gemm(n->H[SFM_LAYERS - 1], SFM_HIDDEN, n->L[SFM_LAYERS - 1].Wb, SFM_HIDDEN, M, SFM_OUT_PAD,
-                          SFM_HIDDEN);
-        g.bias = n->L[SFM_LAYERS - 1].b;
-        g.target = target;
-        g.loss = loss;
-        g.scale = 1.0f / ((float)M * SFM_OUT);
-        g.H = n->dZ[0];
-        g.Ht = n->dZt[0];
-        launch_gemm<EPI_OUT>(g, s);
+    TrainArgs ta;
+    memset(&ta, 0, sizeof(ta));
+    ta.x = x;
+    ta.target = target;
+    ta.loss_part = n->loss_part;
+    ta.scale = 1.0f / ((float)M * SFM_OUT);
+    ta.ldt = M;
+    for (int l = 0; l < SFM_LAYERS; ++l) {
+        ta.W[l] = n->L[l].Wp;
+        ta.Wt[l] = n->L[l].Wtp;
+        ta.b[l] = n->L[l].b;
+        ta.Ht[l] = n->Ht[l];
+        ta.dZt[l] = n->dZt[l];
     }
+    hipLaunchKernelGGL(k_train, dim3(M / kTrainRows), dim3(512), 0, s, ta);
     n->step++;
     const float bc1 = 1.0f - std::pow(beta1, (float)n->step), bc2 = 1.0f - std::pow(beta2, (float)n->step);
-    int cur = 0;
+    // dW = dZ^T H, split over the batch: at most max_splits(l) splits, each a
+    // multiple of 256 rows; their partial sums (weights and biases) are summed
+    // in a fixed order by k_adam
+    WgradSet wg;
     AdamSet adam;
     adam.nseg = 0;
-    int nblk = 0;
+    int nblk = 0, wblk = 0;
     for (int l = SFM_LAYERS - 1; l >= 0; --l) {
         const int dout = kDims[l + 1], din = kDims[l];
         Layer& L = n->L[l];
-        // dW = dZ^T H, split over the batch
-        {
-            // batch splits of the weight-gradient product: at most
-            // max_splits(l), each a multiple of 256 rows; their partial sums
-            // (weights and biases) are summed in a fixed order by k_adam
-            int splits = 1;
-            for (int d = max_splits(l); d >= 1; --d)
-                if ((M / kSplitK) % d == 0) { splits = d; break; }
-            GemmArgs g = gemm(n->dZt[cur], M, n->Ht[l], M, dout, din, M);
-            g.ksplit = splits;
-            g.part = n->part[l];
-            g.bpart = n->dbias[l];
-            launch_gemm<EPI_WGRAD>(g, s);
-            // dH = dZ W  (with the pre-update weights), then dZ of the layer below
-            if (l > 0) {
-                GemmArgs h = gemm(n->dZ[cur], dout, L.Wbt, dout, M, din, dout);
-                h.Z = n->Z[l];
-                h.H = n->dZ[cur ^ 1];
-                h.Ht = n->dZt[cur ^ 1];
-                launch_gemm<EPI_BWD>(h, s);
-            }
-            // every Adam update waits for the end of the step: the products
-            // above read the pre-update weights, and each layer keeps its own
-            // gradient partials, so one launch serves all tensors
-            AdamSeg& sw = adam.seg[adam.nseg++];
-            sw = AdamSeg{L.W, L.mW, L.vW, n->part[l], L.gW, L.Wb, L.Wbt, L.Wp, splits, dout, din, nblk};
-            nblk += (dout * din + 255) / 256;
-            AdamSeg& sb = adam.seg[adam.nseg++];
-            sb = AdamSeg{L.b, L.mb, L.vb, n->dbias[l], L.gb, nullptr, nullptr, nullptr, splits, dout, 1, nblk};
-            nblk += (dout + 255) / 256;
-        }
-        cur ^= 1;
+        int splits = 1;
+        for (int d = max_splits(l); d >= 1; --d)
+            if ((M / kSplitK) % d == 0) { splits = d; break; }
+        const int i = SFM_LAYERS - 1 - l;
+        GemmArgs& g = wg.g[i];
+        g = gemm(n->dZt[l], M, n->Ht[l], M, dout, din, M);
+        g.ksplit = splits;
+        g.part = n->part[l];
+        g.bpart = n->dbias[l];
+        wg.block0[i] = wblk;
+        wblk += splits * (dout % kWgradTile == 0 && din % kWgradTile == 0 ? (dout / kWgradTile) * (din / kWgradTile)
+                                                                           : dout * din / (4 * 32 * 32));
+        AdamSeg& sw = adam.seg[adam.nseg++];
+        sw = AdamSeg{L.W, L.mW, L.vW, n->part[l], L.gW, L.Wb, L.Wtp, L.Wp, splits, dout, din, nblk};
+        nblk += (dout * din + 255) / 256;
+        AdamSeg& sb = adam.seg[adam.nseg++];
+        sb = AdamSeg{L.b, L.mb, L.vb, n->dbias[l], L.gb, nullptr, nullptr, nullptr, splits, dout, 1, nblk};
+        nblk += (dout + 255) / 256;
     }
-    hipLaunchKernelGGL(k_adam, dim3(nblk), dim3(256), 0, s, adam, lr, beta1, beta2, eps, bc1, bc2);
+    hipLaunchKernelGGL(k_wgrad, dim3(wblk), dim3(256), 0, s, wg);
+    adam.nblk = nblk;
+    adam.loss_part = n->loss_part;
+    adam.nloss = M / kTrainRows;
+    adam.loss = loss;
+    hipLaunchKernelGGL(k_adam, dim3(nblk + 1), dim3(256), 0, s, adam, lr, beta1, beta2, eps, bc1, bc2);
     time_end(n, s, 3.0 * forward_flops(batch));
     HIPCHK(hipGetLastError());
     return SFM_OK;
@@ -868,8 +1028,9 @@ extern "C" int sfm_gradients(sfm_net n, int l, float* dw, float* db, void* strea
 {
     if (!n || l < 0 || l >= SFM_LAYERS || !dw || !db) return fail(SFM_ERR_INVALID, "bad argument");
     hipStream_t s = (hipStream_t)stream;
-    HIPCHK(hipMemcpyAsync(dw, n->L[l].gW, sizeof(float) * kDims[l + 1] * kDims[l], hipMemcpyDeviceToDevice, s));
-    HIPCHK(hipMemcpyAsync(db, n->L[l].gb, sizeof(float) * kDims[l + 1], hipMemcpyDeviceToDevice, s));
+    const int nw = kDims[l + 1] * kDims[l], nb = kDims[l + 1];
+    hipLaunchKernelGGL(k_gradients, dim3((nw + nb + 255) / 256), dim3(256), 0, s, n->L[l].gW, n->L[l].gb, nw, nb, dw, db);
+    HIPCHK(hipGetLastError());
     return SFM_OK;
 }
 

@@ -106,8 +106,8 @@ class Net:
 
     def gradients(self, l: int):
         o, i = LAYER_SHAPES[l]
-        dw = torch.zeros((o, i), dtype=torch.float32, device="cuda")
-        db = torch.zeros(o, dtype=torch.float32, device="cuda")
+        dw = torch.empty((o, i), dtype=torch.float32, device="cuda")
+        db = torch.empty(o, dtype=torch.float32, device="cuda")
         N.check_mlp(N.load_mlp().sfm_gradients(self.handle, l, _p(dw), _p(db), C.c_void_p(0)))
         return dw, db
 

@@ -69,3 +69,32 @@ def test_surrogate_step_is_independent_of_the_tile(gpu):
     err = (got[0][0] - got[1][0]).abs().max() / got[0][0].abs().max()
     assert float(err) < 1e-9, float(err)
     net.close()
+
+
+@pytest.mark.parametrize("batch", [256, 768, 1280, 8192])
+def test_gradients_at_batch_edges(gpu, batch):
+    """One workgroup's rows, batches whose splits are fewer than the most, and
+    a batch smaller than the one before it on the same network (whose
+    transposed activations it must not see): the same bits as on a fresh
+    network, and within the rounding of the FP32 reference."""
+    x, t = R.random_inputs(90 + batch, batch)
+    xd, td = x.to(torch.bfloat16).cuda(), t.cuda().contiguous()
+    xl, tl = R.random_inputs(3, 9216)
+    loss = torch.zeros(1, device="cuda")
+    got = []
+    for before in (False, True):
+        net, Ws, bs = _net(9216, 21)
+        if before:
+            net.train_step(xl.to(torch.bfloat16).cuda(), tl.cuda().contiguous(), loss, lr=0.0)
+        net.train_step(xd, td, loss, lr=0.0)
+        got.append([g.cpu() for l in range(5) for g in net.gradients(l)] + [loss.cpu().clone()])
+        net.close()
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+    y, cache = R.forward(Ws, bs, x, rounded=True)
+    lref, dy = R.loss_and_grad_out(y, t)
+    dWs, dbs = R.backward(Ws, cache, dy, rounded=True)
+    assert abs(float(got[0][10]) - float(lref)) <= 1e-3 * float(lref)
+    for l in range(5):
+        assert float((got[0][2 * l] - dWs[l]).norm() / dWs[l].norm()) < 1e-2, l
+        assert float((got[0][2 * l + 1] - dbs[l]).norm() / dbs[l].norm()) < 1e-2, l
