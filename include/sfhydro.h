@@ -420,7 +420,7 @@ int sfh_wave_spectrum(float state, uint32_t passes, const float grid_sizes[4], f
  * heights at time t (seconds) into d_heights, device memory of n x n x 4
  * floats (texel (x, y) at (y n + x) 4: the heights of grids 1-4), which is
  * the reference's layer-0 layout: sfh_ocean_set_waves(ocean, d_heights, 0,
- * n, 4, 2, grid_sizes) gives Ocean::GetDepth's two-grid query.  Three
+ * n, 4, 2, grid_sizes) gives Ocean::GetDepth's two-grid query.  Two
  * launches on `stream`, no allocation. */
 typedef struct sfh_wave_fft_t* sfh_wave_fft;
 int sfh_wave_fft_create(uint32_t passes, const float grid_sizes[4], const float* spectrum12,

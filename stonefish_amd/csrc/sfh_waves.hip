@@ -108,14 +108,14 @@ struct Grids {
     double inv[4];   // 2 pi n / L_g as the float uniform of the init pass
 };
 
-// h(k, t) of the four grids at every texel, packed (h1 + i h2, h3 + i h4).
-__global__ __launch_bounds__(256) void k_wave_init(const float4* __restrict__ s12, const float4* __restrict__ s34,
-                                                   uint32_t n, uint32_t lg, Grids G, double t,
-                                                   float4* __restrict__ out)
+// Threads of a line's workgroup; each has the same n / threads outputs.
+__host__ __device__ constexpr uint32_t wave_threads(uint32_t n) { return n < 1024u ? n : 1024u; }
+
+// h(k, t) of the four grids at texel (x, y), packed (h1 + i h2, h3 + i h4).
+__device__ __forceinline__ float4 wave_init(const float4* __restrict__ s12, const float4* __restrict__ s34, uint32_t n,
+                                            uint32_t x, uint32_t y, const Grids& G, double t)
 {
-    const uint32_t idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= n * n) return;
-    const uint32_t x = idx & (n - 1), y = idx >> lg;
+    const size_t idx = (size_t)y * n + x;
     const uint32_t xc = (n - x) & (n - 1), yc = (n - y) & (n - 1);   // -k, the texture repeats
     const double fx = (double)((x >= n / 2) ? (int)x - (int)n : (int)x) / (double)n;
     const double fy = (double)((y >= n / 2) ? (int)y - (int)n : (int)y) / (double)n;
@@ -136,49 +136,68 @@ __global__ __launch_bounds__(256) void k_wave_init(const float4* __restrict__ s1
         h[2 * g] = (px + qx) * c - (py + qy) * s;
         h[2 * g + 1] = (px - qx) * s + (py - qy) * c;
     }
-    out[idx] = make_float4((float)(h[0] - h[3]), (float)(h[1] + h[2]), (float)(h[4] - h[7]), (float)(h[5] + h[6]));
+    return make_float4((float)(h[0] - h[3]), (float)(h[1] + h[2]), (float)(h[4] - h[7]), (float)(h[5] + h[6]));
 }
 
 // The butterfly passes along one direction, one workgroup per line, the line
 // held in LDS (ping-pong between two copies): out[i] = in[j1] + w * in[j2]
-// for both packed complex values, with (j1, j2, w) the table's entry for
-// output i of the pass.  dir 0: lines are rows (x varies), dir 1: columns.
-__global__ __launch_bounds__(256) void k_wave_fft(float4* __restrict__ data, const int2* __restrict__ idx,
-                                                  const float2* __restrict__ tw, uint32_t n, uint32_t passes,
-                                                  uint32_t dir)
+// for both packed complex values, with w the table's twiddle for output i of
+// the pass and (j1, j2) the table's pair: the block's halves, on pass 0 bit
+// reversed.  ROWS: lines are rows (x varies), formed here from the spectra at
+// time t; otherwise columns, in place.  A thread keeps E = n / threads outputs
+// of every pass; the twiddles of all its passes are requested at the start, one
+// memory round trip instead of one per pass (they came with the index table,
+// pass by pass, and the spectra's h(k, t) from a launch of its own: 3 launches,
+// 13.5 us on 256 x 256; now 2, 11 us).  Bound by latency at that size: the
+// spectra's and twiddles' loads, the FP64 sines of h(k, t), a barrier a pass.
+template <int LG, bool ROWS>
+__global__ __launch_bounds__(1024) void k_wave_fft(float4* __restrict__ data, const float4* __restrict__ s12,
+                                                   const float4* __restrict__ s34, const float2* __restrict__ tw,
+                                                   Grids G, double t)
 {
+    constexpr uint32_t n = 1u << LG, T = wave_threads(n);
+    constexpr int E = n / T;
     extern __shared__ float4 lds[];
     float4* src = lds;
     float4* dst = lds + n;
     const uint32_t line = blockIdx.x;
-    const size_t step = dir ? (size_t)n : 1;
-    float4* base = data + (dir ? (size_t)line : (size_t)line * n);
-    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) src[i] = base[i * step];
+    float2 w[LG][E];
+#pragma unroll
+    for (int p = 0; p < LG; ++p)
+#pragma unroll
+        for (int e = 0; e < E; ++e) w[p][e] = tw[(size_t)p * n + threadIdx.x + e * T];
+    const size_t step = ROWS ? 1 : (size_t)n;
+    float4* base = data + (ROWS ? (size_t)line * n : (size_t)line);
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const uint32_t i = threadIdx.x + e * T;
+        // stored where pass 0 reads it: bit reversed
+        src[__brev(i) >> (32 - LG)] = ROWS ? wave_init(s12, s34, n, i, line, G, t) : base[i * step];
+    }
     __syncthreads();
-    for (uint32_t p = 0; p < passes; ++p) {
-        for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) {
-            const int2 j = idx[(size_t)p * n + i];
-            const float2 w = tw[(size_t)p * n + i];
-            const float4 u = src[j.x], v = src[j.y];
+#pragma unroll
+    for (int p = 0; p < LG; ++p) {
+        const uint32_t nh = 1u << p;
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const uint32_t i = threadIdx.x + e * T, j = i & ~nh;
+            const float2 c = w[p][e];
+            const float4 u = src[j], v = src[j | nh];
             float4 r;
-            r.x = u.x + (w.x * v.x - w.y * v.y);
-            r.y = u.y + (w.y * v.x + w.x * v.y);
-            r.z = u.z + (w.x * v.z - w.y * v.w);
-            r.w = u.w + (w.y * v.z + w.x * v.w);
+            r.x = u.x + (c.x * v.x - c.y * v.y);
+            r.y = u.y + (c.y * v.x + c.x * v.y);
+            r.z = u.z + (c.x * v.z - c.y * v.w);
+            r.w = u.w + (c.y * v.z + c.x * v.w);
             dst[i] = r;
         }
         __syncthreads();
-        float4* t = src; src = dst; dst = t;
+        float4* x = src; src = dst; dst = x;
     }
-    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) base[i * step] = src[i];
-}
-
-uint32_t bit_reverse(uint32_t i, uint32_t n)
-{
-    uint32_t r = 0;
-    for (uint32_t m = n >> 1, w = 1; m; m >>= 1, w <<= 1)
-        if (i & m) r += w;
-    return r;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const uint32_t i = threadIdx.x + e * T;
+        base[i * step] = src[i];
+    }
 }
 
 }  // namespace
@@ -188,7 +207,6 @@ struct sfh_wave_fft_t {
     Grids grids;
     float4* d_s12 = nullptr;
     float4* d_s34 = nullptr;
-    int2* d_idx = nullptr;
     float2* d_tw = nullptr;
 };
 
@@ -196,7 +214,6 @@ static void wave_fft_free(sfh_wave_fft_t* w)
 {
     hipFree(w->d_s12);
     hipFree(w->d_s34);
-    hipFree(w->d_idx);
     hipFree(w->d_tw);
     delete w;
 }
@@ -251,31 +268,25 @@ extern "C" int sfh_wave_fft_create(uint32_t passes, const float grid_sizes[4], c
         h12[i] = to_half(spectrum12[i]);
         h34[i] = to_half(spectrum34[i]);
     }
-    // butterfly table (j1, j2, w) per output of each pass, twiddles as binary16
-    std::vector<int2> idx((size_t)passes * n);
+    // butterfly table: the twiddle of each output of each pass, as binary16
+    // (its index pair is formed in the kernel)
     std::vector<float2> tw((size_t)passes * n);
     for (uint32_t p = 0; p < passes; ++p) {
         const uint32_t nblocks = 1u << (passes - 1 - p), nh = 1u << p;
         for (uint32_t j = 0; j < nblocks; ++j)
             for (uint32_t k = 0; k < nh; ++k) {
                 const uint32_t i1 = j * nh * 2 + k, i2 = i1 + nh;
-                const uint32_t j1 = p == 0 ? bit_reverse(i1, n) : i1;
-                const uint32_t j2 = p == 0 ? bit_reverse(i2, n) : i2;
                 const double arg = 2.0 * M_PI * (double)(k * nblocks) / (double)(float)n;
                 const float wr = to_half((float)std::cos(arg)), wi = to_half((float)std::sin(arg));
-                idx[(size_t)p * n + i1] = make_int2((int)j1, (int)j2);
-                idx[(size_t)p * n + i2] = make_int2((int)j1, (int)j2);
                 tw[(size_t)p * n + i1] = make_float2(wr, wi);
                 tw[(size_t)p * n + i2] = make_float2(-wr, -wi);
             }
     }
     hipError_t e = hipMalloc(&w->d_s12, sizeof(float4) * texels);
     if (e == hipSuccess) e = hipMalloc(&w->d_s34, sizeof(float4) * texels);
-    if (e == hipSuccess) e = hipMalloc(&w->d_idx, sizeof(int2) * idx.size());
     if (e == hipSuccess) e = hipMalloc(&w->d_tw, sizeof(float2) * tw.size());
     if (e == hipSuccess) e = hipMemcpy(w->d_s12, h12.data(), sizeof(float) * h12.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(w->d_s34, h34.data(), sizeof(float) * h34.size(), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(w->d_idx, idx.data(), sizeof(int2) * idx.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(w->d_tw, tw.data(), sizeof(float2) * tw.size(), hipMemcpyHostToDevice);
     if (e != hipSuccess) {
         wave_fft_free(w);
@@ -291,11 +302,21 @@ extern "C" int sfh_wave_fft_step(sfh_wave_fft w, float t, float* d_heights, void
     hipStream_t s = (hipStream_t)stream;
     const uint32_t n = w->n;
     float4* out = reinterpret_cast<float4*>(d_heights);
-    hipLaunchKernelGGL(k_wave_init, dim3((n * n + 255) / 256), dim3(256), 0, s, w->d_s12, w->d_s34, n, w->passes,
-                       w->grids, (double)t, out);
     const size_t lds = 2 * sizeof(float4) * n;
-    hipLaunchKernelGGL(k_wave_fft, dim3(n), dim3(256), lds, s, out, w->d_idx, w->d_tw, n, w->passes, 0u);
-    hipLaunchKernelGGL(k_wave_fft, dim3(n), dim3(256), lds, s, out, w->d_idx, w->d_tw, n, w->passes, 1u);
+#define LAUNCH_W(LG, ROWS)                                                                                         \
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_wave_fft<LG, ROWS>), dim3(n), dim3(wave_threads(n)), lds, s, out, w->d_s12, \
+                       w->d_s34, w->d_tw, w->grids, (double)t)
+#define CASE_W(LG)             \
+    case LG:                   \
+        LAUNCH_W(LG, true);    \
+        LAUNCH_W(LG, false);   \
+        break;
+    switch (w->passes) {
+        CASE_W(1) CASE_W(2) CASE_W(3) CASE_W(4) CASE_W(5) CASE_W(6) CASE_W(7) CASE_W(8) CASE_W(9) CASE_W(10) CASE_W(11)
+        default: return sfh_internal_fail(SFH_ERR_INVALID, "bad pass count");
+    }
+#undef CASE_W
+#undef LAUNCH_W
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return sfh_internal_fail(SFH_ERR_HIP, hipGetErrorString(e));
     return SFH_OK;
