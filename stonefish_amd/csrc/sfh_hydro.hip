@@ -2188,8 +2188,8 @@ struct sfh_batch_t {
     std::vector<BodyStatic> h_static;
     BodyStatic* d_static = nullptr;
     uint32_t* d_sidx = nullptr;     // per body: BodyStatic::sidx, compact (the masked prologue's first read)
-    double* d_hstates = nullptr;    // device copies of sfh_batch_compute_host's host buffers (first call)
-    double* d_hout = nullptr;
+    double* h_io = nullptr;         // sfh_batch_compute_host: pinned staging of the states, then the rows (first call)
+    double* d_io = nullptr;         // the same in device memory, for steps of several launches
     Chunk* d_chunks = nullptr;
     int8_t* d_bpos = nullptr;       // per body: this step's position (-2 inactive, -1 not hydrodynamic, 0, 1, 2)
     uint32_t* d_lists = nullptr;    // the step's work list [nchunks], then its two counts
@@ -2474,9 +2474,9 @@ static void batch_free(sfh_batch_t* b)
         if (b->ev[i]) hipEventDestroy(b->ev[i]);
     hipFree(b->d_static);
     hipFree(b->d_sidx);
-    hipFree(b->d_hstates);
-    hipFree(b->d_hout);
-    b->d_hstates = b->d_hout = nullptr;
+    hipHostFree(b->h_io);
+    hipFree(b->d_io);
+    b->h_io = b->d_io = nullptr;
     hipFree(b->d_chunks);
     hipFree(b->d_bpos);
     hipFree(b->d_lists);
@@ -3270,28 +3270,53 @@ extern "C" int sfh_tick_destroy(sfh_tick t)
     return SFH_OK;
 }
 
+// Host buffers go through pinned staging that lives with the batch.  A step of
+// one launch reads the states and writes the rows there itself: no copy
+// commands (24 bodies: 59 -> 29.5 us, where two copies in, one out and their
+// waits were half of the call; 200 bodies 79 -> 46).  Larger steps copy it to
+// device memory and back on the launch stream with one wait at the end (1,280
+// bodies 117 -> 100 us, 16,384 525 -> 518); past kHostStaged the second pass over
+// host memory costs more than the waits (100,000 bodies 2.59 -> 2.82 ms), and
+// the buffers are copied as they are.
+static constexpr size_t kHostStaged = 16u << 20;   // bytes of states and rows
+
 extern "C" int sfh_batch_compute_host(sfh_batch b, sfh_ocean o, const double* states, double* out)
 {
     if (!b || !states || !out) return fail(SFH_ERR_INVALID, "null argument");
-    size_t ns = (size_t)b->nunits * SFH_STATE_DOUBLES, no = (size_t)b->nunits * SFH_OUT_DOUBLES;
-    if (!b->d_hstates) {   // the device copies live with the batch (sizes fixed per batch)
-        HIPCHK(hipMalloc(&b->d_hstates, sizeof(double) * std::max<size_t>(1, ns)));
-        hipError_t ea = hipMalloc(&b->d_hout, sizeof(double) * std::max<size_t>(1, no));
-        if (ea != hipSuccess) {
-            hipFree(b->d_hstates);
-            b->d_hstates = nullptr;
-            return fail(SFH_ERR_HIP, "alloc: %s", hipGetErrorString(ea));
-        }
+    const size_t ns = (size_t)b->nunits * SFH_STATE_DOUBLES, no = (size_t)b->nunits * SFH_OUT_DOUBLES;
+    const size_t bytes = sizeof(double) * std::max<size_t>(1, ns + no);
+    const bool direct = step_fused(b), staged = direct || bytes <= kHostStaged;
+    if (staged && !b->h_io && hipHostMalloc((void**)&b->h_io, bytes, hipHostMallocDefault) != hipSuccess) {
+        b->h_io = nullptr;
+        return fail(SFH_ERR_HIP, "pinned staging of %zu bytes failed", bytes);
     }
-    int rc = SFH_OK;
-    hipError_t e = hipMemcpy(b->d_hstates, states, sizeof(double) * ns, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(b->d_hout, out, sizeof(double) * no, hipMemcpyHostToDevice);
+    if (!direct && !b->d_io && hipMalloc(&b->d_io, bytes) != hipSuccess) {
+        b->d_io = nullptr;
+        return fail(SFH_ERR_HIP, "device buffers of %zu bytes failed", bytes);
+    }
+    double* io = direct ? b->h_io : b->d_io;
+    hipError_t e = hipSuccess;
+    if (staged) {
+        memcpy(b->h_io, states, sizeof(double) * ns);
+        memcpy(b->h_io + ns, out, sizeof(double) * no);
+        if (!direct) e = hipMemcpyAsync(io, b->h_io, sizeof(double) * (ns + no), hipMemcpyHostToDevice, nullptr);
+    } else {
+        e = hipMemcpy(io, states, sizeof(double) * ns, hipMemcpyHostToDevice);
+        if (e == hipSuccess) e = hipMemcpy(io + ns, out, sizeof(double) * no, hipMemcpyHostToDevice);
+    }
     if (e == hipSuccess) {
-        rc = sfh_batch_compute(b, o, b->d_hstates, b->d_hout, nullptr);
-        if (rc == SFH_OK) e = hipMemcpy(out, b->d_hout, sizeof(double) * no, hipMemcpyDeviceToHost);
+        const int rc = sfh_batch_compute(b, o, io, io + ns, nullptr);
+        if (rc != SFH_OK) {
+            hipStreamSynchronize(nullptr);   // the staging is free again
+            return rc;
+        }
+        if (!staged) e = hipMemcpy(out, io + ns, sizeof(double) * no, hipMemcpyDeviceToHost);
+        else if (!direct) e = hipMemcpyAsync(b->h_io + ns, io + ns, sizeof(double) * no, hipMemcpyDeviceToHost, nullptr);
     }
+    if (e == hipSuccess && staged) e = hipStreamSynchronize(nullptr);
     if (e != hipSuccess) return fail(SFH_ERR_HIP, "batch host compute: %s", hipGetErrorString(e));
-    return rc;
+    if (staged) memcpy(out, b->h_io + ns, sizeof(double) * no);
+    return SFH_OK;
 }
 
 extern "C" int sfh_batch_capture(sfh_batch b, sfh_ocean o, const double* d_states, double* d_out, void* stream)

@@ -25,11 +25,21 @@ from .meshes import TriMesh
 
 
 def _dp(a: np.ndarray):
+    """A float64 array as a `double*` argument.  A writable array passes through
+    the buffer protocol (a tenth of the time of ndarray.ctypes.data_as, which a
+    per-body call's dozen arguments took half of)."""
     assert a.dtype == np.float64 and a.flags.c_contiguous
+    if a.size and a.flags.writeable:
+        return C.c_double.from_buffer(a)   # by reference for a POINTER(c_double) parameter
     return a.ctypes.data_as(N.c_double_p)
 
 
+_F64 = np.dtype(np.float64)
+
+
 def _vec(x, n=3) -> np.ndarray:
+    if type(x) is np.ndarray and x.dtype is _F64 and x.shape == (n,) and x.flags.c_contiguous:
+        return x
     a = np.ascontiguousarray(np.asarray(x, dtype=np.float64).reshape(-1))
     if a.size != n:
         raise ValueError(f"expected {n} values, got {a.size}")
