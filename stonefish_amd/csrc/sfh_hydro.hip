@@ -24,6 +24,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cfloat>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -85,6 +86,7 @@ enum : uint32_t {
 };
 
 static constexpr int kMaxLayers = 4;
+static constexpr uint32_t kMaskedGrid = 16384;   // its 16-byte texels are within a 32-bit offset
 static constexpr int kChunkDoubles = 24;
 static constexpr int kMaxCur = 4;   // jets and pipes evaluated per face
 
@@ -101,6 +103,10 @@ struct CurBody {
 struct BodyStatic {
     const float* verts;
     const uint32_t* faces;
+    const float4* recs;     // the mesh's face records (FaceRec)
+    const uint32_t* pidx;   // its packed vertex numbers (PackedFaces)
+    const uint2* blkwin;    // per block of 64 faces: lowest and highest vertex id
+    double lo_unit;         // unit of the records' centroid remainders
     uint32_t nf;
     uint32_t flags;
     uint32_t chunk0;
@@ -151,7 +157,7 @@ struct OceanK {
     const float4* quad[kMaxLayers];   // per layer: (h00, h10, h01, h11) per texel
     int32_t nlayers;                  // 0 = flat surface
     int32_t n;
-    int32_t nmask;                    // n - 1 when n is a power of two, else -1
+    int32_t nmask;                    // n - 1 when n is a power of two up to kMaskedGrid, else -1
     int32_t ncur;                     // enabled jets and pipes
     int32_t cur_type[kMaxCur];
     double cur_c[kMaxCur][3], cur_a[kMaxCur][3];   // world anchor and unit axis
@@ -181,6 +187,27 @@ __device__ __forceinline__ SFH_GLOBAL T* gptr_w(T* p)
     return (SFH_GLOBAL T*)p;
 }
 
+// Loads at a 32-bit byte offset from a wavefront-uniform base: the base stays
+// in scalar registers and no 64-bit address is formed per lane.
+template <typename T>
+__device__ __forceinline__ T load_at(const SFH_GLOBAL T* base, uint32_t i)
+{
+    return *(const SFH_GLOBAL T*)((const SFH_GLOBAL char*)base + i * (uint32_t)sizeof(T));
+}
+
+__device__ __forceinline__ f3 vert_at(const SFH_GLOBAL float* base, uint32_t i)
+{
+    const SFH_GLOBAL float* v = (const SFH_GLOBAL float*)((const SFH_GLOBAL char*)base + i * 12u);
+    return mk3(v[0], v[1], v[2]);
+}
+
+__device__ __forceinline__ void wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 __device__ __forceinline__ int wrap_n(int i, int n)
 {
     // i = k + floor(u) with k in [0, n) and |floor(u)| below n for any body
@@ -191,10 +218,13 @@ __device__ __forceinline__ int wrap_n(int i, int n)
     return min(max(i, 0), n - 1);
 }
 
-// Bilinear mix of a texel's four corner heights at fractions (a, b).
+// Bilinear mix of a texel's four corner heights at fractions (a, b): three
+// linear steps.
 __device__ __forceinline__ double texel_mix(double a, double b, float4 t)
 {
-    return (1.0 - a) * (1.0 - b) * t.x + a * (1.0 - b) * t.y + (1.0 - a) * b * t.z + a * b * t.w;
+    const double x0 = t.x, x1 = t.z;
+    const double y0 = __builtin_fma(a, (double)t.y - x0, x0), y1 = __builtin_fma(a, (double)t.w - x1, x1);
+    return __builtin_fma(b, y1 - y0, y0);
 }
 
 // Depth of the mesh-frame point (x, y, z), FP64: z - H(x, y) with
@@ -220,7 +250,7 @@ __device__ __forceinline__ double depth64(const BodyDyn& D, const OceanK& oc, do
             j = wrap_n(L.kv + (int)fj, oc.n);
         }
         float4 t = oc.quad[l][(size_t)j * oc.n + i];
-        d += (1.0 - a) * (1.0 - b) * t.x + a * (1.0 - b) * t.y + (1.0 - a) * b * t.z + a * b * t.w;
+        d += texel_mix(a, b, t);
     }
     return d;
 }
@@ -246,7 +276,6 @@ struct WaveQ {
     static constexpr int M = NL > 0 ? NL : 1;
     double tz, rz[3];
     double fu[M], fv[M], ru[M][3], rv[M][3];
-    int ku[M], kv[M];
     const SFH_GLOBAL f32x4* quad[M];
     int n, nmask;
     const BodyDyn* D;
@@ -264,11 +293,9 @@ struct WaveQ {
 #pragma unroll
         for (int l = 0; l < (NL > 0 ? NL : 0); ++l) {
             const LayerK& L = Dy.layer[l];
-            fu[l] = L.fu;
-            fv[l] = L.fv;
+            fu[l] = L.fu + (double)L.ku;   // below the grid size: its rounding is below 1e-12 texels
+            fv[l] = L.fv + (double)L.kv;
             for (int k = 0; k < 3; ++k) { ru[l][k] = L.ru[k]; rv[l][k] = L.rv[k]; }
-            ku[l] = L.ku;
-            kv[l] = L.kv;
             quad[l] = (const SFH_GLOBAL f32x4*)o.quad[l];
         }
     }
@@ -284,17 +311,20 @@ struct WaveQ {
 
     __device__ __forceinline__ Pending issue(f3 base, f3 off) const
     {
+        return issue((double)base.x + (double)off.x, (double)base.y + (double)off.y, (double)base.z + (double)off.z);
+    }
+
+    __device__ __forceinline__ Pending issue(double x, double y, double z) const
+    {
         Pending q;
-        const double x = (double)base.x + (double)off.x, y = (double)base.y + (double)off.y,
-                     z = (double)base.z + (double)off.z;
         q.d = tz + rz[0] * x + rz[1] * y + rz[2] * z;
 #pragma unroll
         for (int l = 0; l < (NL > 0 ? NL : 0); ++l) {
             const double u = fu[l] + ru[l][0] * x + ru[l][1] * y + ru[l][2] * z;
             const double v = fv[l] + rv[l][0] * x + rv[l][1] * y + rv[l][2] * z;
             const double fi = floor(u), fj = floor(v);
-            const int i = (ku[l] + (int)fi) & nmask, j = (kv[l] + (int)fj) & nmask;
-            q.t[l] = quad[l][(uint32_t)j * (uint32_t)n + (uint32_t)i];
+            const int i = (int)fi & nmask, j = (int)fj & nmask;
+            q.t[l] = load_at(quad[l], (uint32_t)j * (uint32_t)n + (uint32_t)i);
             q.a[l] = u - fi;
             q.b[l] = v - fj;
         }
@@ -313,20 +343,13 @@ struct WaveQ {
     // depth64 at the mesh-frame point base + off (FP32 parts, summed in FP64)
     __device__ __forceinline__ double depth(f3 base, f3 off) const
     {
-        const double x = (double)base.x + (double)off.x, y = (double)base.y + (double)off.y,
-                     z = (double)base.z + (double)off.z;
+        return depth((double)base.x + (double)off.x, (double)base.y + (double)off.y, (double)base.z + (double)off.z);
+    }
+
+    __device__ __forceinline__ double depth(double x, double y, double z) const
+    {
         if (NL < 0) return depth64(*D, *oc, x, y, z);
-        double d = tz + rz[0] * x + rz[1] * y + rz[2] * z;
-#pragma unroll
-        for (int l = 0; l < (NL > 0 ? NL : 0); ++l) {
-            const double u = fu[l] + ru[l][0] * x + ru[l][1] * y + ru[l][2] * z;
-            const double v = fv[l] + rv[l][0] * x + rv[l][1] * y + rv[l][2] * z;
-            const double fi = floor(u), fj = floor(v);
-            const int i = (ku[l] + (int)fi) & nmask, j = (kv[l] + (int)fj) & nmask;
-            const f32x4 t = quad[l][(uint32_t)j * (uint32_t)n + (uint32_t)i];
-            d += texel_mix(u - fi, v - fj, make_float4(t.x, t.y, t.z, t.w));
-        }
-        return d;
+        return finish(issue(x, y, z));
     }
 };
 
@@ -758,6 +781,43 @@ __host__ __device__ constexpr uint32_t win_cap(uint32_t K) { return K <= 16 ? 64
 // k_faces: one wavefront per chunk of up to 64*K faces of one body
 // ---------------------------------------------------------------------------
 
+// One step of a transposed reduction: lanes whose bit OFF is clear get the sum
+// of a over themselves and their partner (the lane differing in that bit),
+// the others that of b.  Bits 5 and 4 trade the halves between the two
+// registers (v_permlane32_swap, v_permlane16_swap: two and the add, where a
+// select and a shuffle through the LDS take nine), bits 3, 1 and 0 move
+// within a row of 16 lanes (DPP).
+template <int OFF>
+__device__ __forceinline__ double lane_xor(double x)
+{
+    static_assert(OFF == 8 || OFF == 4 || OFF == 2 || OFF == 1, "within a row");
+    if (OFF == 4) return __shfl_xor(x, 4, 64);
+    constexpr int dpp = OFF == 8 ? 0x128 /* row_ror:8 */ : OFF == 2 ? 0x4e /* quad_perm 2301 */ : 0xb1 /* 1032 */;
+    const int lo = __double2loint(x), hi = __double2hiint(x);
+    return __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, dpp, 0xf, 0xf, false),
+                            __builtin_amdgcn_update_dpp(lo, lo, dpp, 0xf, 0xf, false));
+}
+
+template <int OFF>
+__device__ __forceinline__ double xstep(double a, double b, int lane)
+{
+    if (OFF >= 16) {
+        const uint32_t al = (uint32_t)__double2loint(a), ah = (uint32_t)__double2hiint(a);
+        const uint32_t bl = (uint32_t)__double2loint(b), bh = (uint32_t)__double2hiint(b);
+        if (OFF == 32) {
+            const auto l = __builtin_amdgcn_permlane32_swap(al, bl, false, false);
+            const auto h = __builtin_amdgcn_permlane32_swap(ah, bh, false, false);
+            return __hiloint2double((int)h[0], (int)l[0]) + __hiloint2double((int)h[1], (int)l[1]);
+        }
+        const auto l = __builtin_amdgcn_permlane16_swap(al, bl, false, false);
+        const auto h = __builtin_amdgcn_permlane16_swap(ah, bh, false, false);
+        return __hiloint2double((int)h[0], (int)l[0]) + __hiloint2double((int)h[1], (int)l[1]);
+    }
+    const bool hi = lane & OFF;
+    const double send = hi ? a : b, keep = hi ? b : a;
+    return keep + lane_xor<(OFF < 16 ? OFF : 8)>(send);
+}
+
 // Transposed FP64 reduction of 24 per-lane values across a wavefront.  Each
 // step exchanges half of the remaining values with the partner lane, so the
 // wave moves 12+6+3+2+1+1 doubles instead of 6 per value.  On return v[0] of
@@ -765,37 +825,17 @@ __host__ __device__ constexpr uint32_t win_cap(uint32_t K) { return K <= 16 ? 64
 // (b = bits of l); q == 23 and (2 b2 + b1) == 3 are padding.
 __device__ __forceinline__ void xreduce24(double (&v)[24], int lane)
 {
-    bool hi = lane & 32;
 #pragma unroll
-    for (int i = 0; i < 12; ++i) {
-        double send = hi ? v[i] : v[i + 12], keep = hi ? v[i + 12] : v[i];
-        v[i] = keep + __shfl_xor(send, 32, 64);
-    }
-    hi = lane & 16;
+    for (int i = 0; i < 12; ++i) v[i] = xstep<32>(v[i], v[i + 12], lane);
 #pragma unroll
-    for (int i = 0; i < 6; ++i) {
-        double send = hi ? v[i] : v[i + 6], keep = hi ? v[i + 6] : v[i];
-        v[i] = keep + __shfl_xor(send, 16, 64);
-    }
-    hi = lane & 8;
+    for (int i = 0; i < 6; ++i) v[i] = xstep<16>(v[i], v[i + 6], lane);
 #pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        double send = hi ? v[i] : v[i + 3], keep = hi ? v[i + 3] : v[i];
-        v[i] = keep + __shfl_xor(send, 8, 64);
-    }
+    for (int i = 0; i < 3; ++i) v[i] = xstep<8>(v[i], v[i + 3], lane);
     v[3] = 0.0;
-    hi = lane & 4;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        double send = hi ? v[i] : v[i + 2], keep = hi ? v[i + 2] : v[i];
-        v[i] = keep + __shfl_xor(send, 4, 64);
-    }
-    hi = lane & 2;
-    {
-        double send = hi ? v[0] : v[1], keep = hi ? v[1] : v[0];
-        v[0] = keep + __shfl_xor(send, 2, 64);
-    }
-    v[0] += __shfl_xor(v[0], 1, 64);
+    for (int i = 0; i < 2; ++i) v[i] = xstep<4>(v[i], v[i + 2], lane);
+    v[0] = xstep<2>(v[0], v[1], lane);
+    v[0] += lane_xor<1>(v[0]);
 }
 
 __device__ __forceinline__ int xreduce24_slot(int lane)
@@ -812,37 +852,126 @@ __device__ __forceinline__ f3 vert(const SFH_GLOBAL float* __restrict__ verts, u
     return mk3(v[0], v[1], v[2]);
 }
 
+// A mesh's face records: what the integrand needs of a whole face and no
+// state changes, formed once per mesh (k_face_records) with the operations of
+// face_submerged and face_allwet, so the same bits: three arrays of float4
+// after one another,
+//   recs[f]          unit normal, area (negative: a degenerate face, which adds
+//                    volume only)
+//   recs[nf + f]     centroid p1 + (e1 + e2) / 3, rounded once, and the three
+//                    10-bit remainders of the exact centroid (p1 + p2 + p3) / 3
+//                    in units of lo_unit, 1e-10 of the mesh's size: the
+//                    submerged loop's
+//   recs[2 nf + f]   the same with (e1 + e2) / 3 rounded before it is added, and
+//                    the remainders of that sum: the loop's of a crossing body
+//                    on waves
+// A face so costs two coalesced 16-byte loads instead of three indices and
+// nine dependent gathers, and none of the edges, cross product and square root.
+struct FaceRec {
+    f3 n1, c;
+    float A;
+    int lo;
+};
+
+// PackedFaces: a face's three vertex numbers in one word, 10 bits each, less
+// the lowest vertex id of its block of 64 faces (blkwin): a third of the bytes
+// and loads of the three 32-bit numbers.  They stand for a face whose block
+// spans at most kPackSpan ids; a chunk with a vertex window has no other
+// blocks (chunk_window).
+static constexpr uint32_t kPackSpan = 1024;
+
+__device__ __forceinline__ uint32_t unpack_id(uint32_t w, int k) { return (w >> (10 * k)) & 1023u; }
+
+__device__ __forceinline__ FaceRec make_rec(f32x4 a, f32x4 b)
+{
+    FaceRec r;
+    r.n1 = mk3(a.x, a.y, a.z);
+    r.A = a.w;
+    r.c = mk3(b.x, b.y, b.z);
+    r.lo = __float_as_int(b.w);
+    return r;
+}
+
+__device__ __forceinline__ void rec_centroid(f3 c, int lo, double unit, double (&x)[3])
+{
+    x[0] = __builtin_fma((double)((lo << 22) >> 22), unit, (double)c.x);
+    x[1] = __builtin_fma((double)((lo << 12) >> 22), unit, (double)c.y);
+    x[2] = __builtin_fma((double)((lo << 2) >> 22), unit, (double)c.z);
+}
+
+// A wet polygon's centroid, rounded once (fused) or after the offset.
+template <bool FUSED>
+__device__ __forceinline__ f3 step_centroid(f3 base, f3 cs, float ck)
+{
+#pragma clang fp contract(off)
+    if (FUSED)
+        return mk3(__builtin_fmaf(cs.x, ck, base.x), __builtin_fmaf(cs.y, ck, base.y), __builtin_fmaf(cs.z, ck, base.z));
+    const float x = cs.x * ck, y = cs.y * ck, z = cs.z * ck;
+    return mk3(base.x + x, base.y + y, base.z + z);
+}
+
+__device__ __forceinline__ float pack_remainders(const double (&x)[3], f3 c, double unit)
+{
+    const double d[3] = {x[0] - (double)c.x, x[1] - (double)c.y, x[2] - (double)c.z};
+    uint32_t lo = 0;
+    for (int k = 0; k < 3; ++k) {
+        const double r = unit > 0.0 ? rint(d[k] / unit) : 0.0;
+        lo |= ((uint32_t)(int)fmin(fmax(r, -512.0), 511.0) & 1023u) << (10 * k);
+    }
+    return __uint_as_float(lo);
+}
+
+__global__ __launch_bounds__(256) void k_face_records(const float* __restrict__ verts,
+                                                      const uint32_t* __restrict__ faces,
+                                                      const uint2* __restrict__ blkwin, uint32_t nf, double unit,
+                                                      float4* __restrict__ recs, uint32_t* __restrict__ pidx)
+{
+    const uint32_t f = blockIdx.x * 256u + threadIdx.x;
+    if (f >= nf) return;
+    const SFH_GLOBAL float* vs = gptr(verts);
+    const uint32_t i0 = faces[3 * (size_t)f], i1 = faces[3 * (size_t)f + 1], i2 = faces[3 * (size_t)f + 2];
+    const uint32_t lowest = blkwin[f / 64].x;
+    pidx[f] = ((i0 - lowest) & 1023u) | ((i1 - lowest) & 1023u) << 10 | ((i2 - lowest) & 1023u) << 20;
+    const f3 p1 = vert(vs, i0), p2 = vert(vs, i1), p3 = vert(vs, i2);
+    const f3 e1 = p2 - p1, e2 = p3 - p1;
+    const f3 n = cross(e1, e2);
+    const float n2 = dot(n, n);
+    const float inv = frsq(n2);
+    f3 n1 = n * inv;
+    float A = 0.5f * (n2 * inv);
+    if (n2 < SFH_DEGENERATE_N2) {
+        if (!(n2 > 0.f)) {
+            n1 = mk3(0.f, 0.f, 0.f);
+            A = 0.f;
+        }
+        A = -fmaxf(A, FLT_MIN);
+    }
+    recs[f] = make_float4(n1.x, n1.y, n1.z, A);
+    const f3 s = e1 + e2, off = s * (1.0f / 3.0f);
+    const f3 c = step_centroid<true>(p1, s, 1.0f / 3.0f), d = step_centroid<false>(p1, s, 1.0f / 3.0f);
+    const double xc[3] = {((double)p1.x + (double)p2.x + (double)p3.x) / 3.0,
+                          ((double)p1.y + (double)p2.y + (double)p3.y) / 3.0,
+                          ((double)p1.z + (double)p2.z + (double)p3.z) / 3.0};
+    const double xd[3] = {(double)p1.x + (double)off.x, (double)p1.y + (double)off.y, (double)p1.z + (double)off.z};
+    recs[(size_t)nf + f] = make_float4(c.x, c.y, c.z, pack_remainders(xc, c, unit));
+    recs[2 * (size_t)nf + f] = make_float4(d.x, d.y, d.z, pack_remainders(xd, d, unit));
+}
+
 // Transposed FP64 reduction of 12 per-lane values: on return v[0] of lane l
 // holds the total of quantity q = 6 b5 + 3 b4 + 2 b3 + b2 ((2 b3 + b2) == 3 is
 // padding); lanes with b1 = b0 = 0 hold it.
 __device__ __forceinline__ void xreduce12(double (&v)[12], int lane)
 {
-    bool hi = lane & 32;
 #pragma unroll
-    for (int i = 0; i < 6; ++i) {
-        double send = hi ? v[i] : v[i + 6], keep = hi ? v[i + 6] : v[i];
-        v[i] = keep + __shfl_xor(send, 32, 64);
-    }
-    hi = lane & 16;
+    for (int i = 0; i < 6; ++i) v[i] = xstep<32>(v[i], v[i + 6], lane);
 #pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        double send = hi ? v[i] : v[i + 3], keep = hi ? v[i + 3] : v[i];
-        v[i] = keep + __shfl_xor(send, 16, 64);
-    }
+    for (int i = 0; i < 3; ++i) v[i] = xstep<16>(v[i], v[i + 3], lane);
     v[3] = 0.0;
-    hi = lane & 8;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        double send = hi ? v[i] : v[i + 2], keep = hi ? v[i + 2] : v[i];
-        v[i] = keep + __shfl_xor(send, 8, 64);
-    }
-    hi = lane & 4;
-    {
-        double send = hi ? v[0] : v[1], keep = hi ? v[1] : v[0];
-        v[0] = keep + __shfl_xor(send, 4, 64);
-    }
-    v[0] += __shfl_xor(v[0], 2, 64);
-    v[0] += __shfl_xor(v[0], 1, 64);
+    for (int i = 0; i < 2; ++i) v[i] = xstep<8>(v[i], v[i + 2], lane);
+    v[0] = xstep<4>(v[0], v[1], lane);
+    v[0] += lane_xor<2>(v[0]);
+    v[0] += lane_xor<1>(v[0]);
 }
 
 __device__ __forceinline__ int xreduce12_slot(int lane)
@@ -856,44 +985,68 @@ __device__ __forceinline__ int xreduce12_slot(int lane)
 // [f0, f0 + nfc) of body S): per-face arithmetic in FP32 with FP32 per-lane
 // partial sums over the lane's K faces, reduced across the wavefront in FP64
 // into the chunk's partial (12 doubles: Fdq Mdq Fdf Mdf).
-template <int K, bool NU, bool AERO>
+template <int K, bool NU, bool AERO, bool REC>
 __device__ __forceinline__ void sub_chunk(uint32_t c, uint32_t f0, uint32_t nfc, const BodyStatic& S,
                                           const BodyDyn& D, double* __restrict__ partials, int lane)
 {
-    const SFH_GLOBAL float* __restrict__ verts = gptr(S.verts);
-    const SFH_GLOBAL uint32_t* __restrict__ faces = gptr(S.faces) + 3 * (size_t)f0;
     const FaceBody fb = D.fb;
     const CurFlow flow{&D.cur};
     AccDrag<float> acc;
     acc_zero(acc);
-    // Two-stage software pipeline over the lane's K faces: the indices of
-    // face j+2 and the vertices of face j+1 are in flight while face j is
-    // computed.  Face numbers past the chunk are clamped to its last face
-    // so every load stays in bounds; their results are not used.
+    // Face numbers past the chunk are clamped to its last face so every load
+    // stays in bounds; their results are not used.
     const uint32_t flast = nfc - 1;
-    uint32_t fc0 = min((uint32_t)lane, flast), fc1 = min(64u + lane, flast);
-    uint32_t a0 = faces[3 * fc0], a1 = faces[3 * fc0 + 1], a2 = faces[3 * fc0 + 2];
-    uint32_t b0 = faces[3 * fc1], b1 = faces[3 * fc1 + 1], b2 = faces[3 * fc1 + 2];
-    f3 p1 = vert(verts, a0), p2 = vert(verts, a1), p3 = vert(verts, a2);
+    const int rows = (int)((nfc + 63u) / 64u);
+    if (REC) {
+        // the records of face j+1 are in flight while face j is computed
+        const SFH_GLOBAL f32x4* __restrict__ r0 = (const SFH_GLOBAL f32x4*)S.recs + f0;
+        const SFH_GLOBAL f32x4* __restrict__ r1 = r0 + S.nf;
+        const uint32_t fc = min((uint32_t)lane, flast);
+        f32x4 a = load_at(r0, fc), b = load_at(r1, fc);
 #pragma unroll 2
-    for (int j = 0; j < K; ++j) {
-        const uint32_t fn2 = min(64u * (j + 2) + lane, flast);
-        f3 q1 = vert(verts, b0), q2 = vert(verts, b1), q3 = vert(verts, b2);
-        uint32_t c0 = faces[3 * fn2], c1 = faces[3 * fn2 + 1], c2 = faces[3 * fn2 + 2];
-        if (64u * j + lane < nfc) {
-            if (AERO) {
-                if (NU)
-                    face_aero(fb, p1, p2, p3, flow, acc);
-                else
-                    face_aero(fb, p1, p2, p3, NoFlow(), acc);
-            } else if (NU) {
-                face_submerged(fb, p1, p2, p3, flow, acc);
-            } else {
-                face_submerged(fb, p1, p2, p3, acc);
+        for (int j = 0; j < rows; ++j) {
+            const uint32_t fn = min(64u * (j + 1) + lane, flast);
+            const f32x4 an = load_at(r0, fn), bn = load_at(r1, fn);
+            const FaceRec r = make_rec(a, b);
+            if (64u * j + lane < nfc && r.A >= 0.f) {
+                f3 uf = mk3(0.f, 0.f, 0.f);
+                if (NU) {
+                    double x[3];
+                    rec_centroid(r.c, r.lo, S.lo_unit, x);
+                    uf = flow(x[0], x[1], x[2]);
+                }
+                if (AERO) aero_drag<NU>(fb, r.c, r.n1, r.A, uf, acc);
+                else face_drag<NU>(fb, r.c, r.n1, r.A, uf, acc);
             }
+            a = an; b = bn;
         }
-        p1 = q1; p2 = q2; p3 = q3;
-        b0 = c0; b1 = c1; b2 = c2;
+    } else {
+        // the packed numbers of face j+2 and the vertices of face j+1 are in
+        // flight while face j is computed; lane k holds block k's lowest id
+        const SFH_GLOBAL uint32_t* __restrict__ pidx = gptr(S.pidx) + f0;
+        const SFH_GLOBAL float* __restrict__ verts = gptr(S.verts);
+        const uint32_t low = gptr((const uint32_t*)S.blkwin)[2 * (f0 / 64 + min(lane, rows - 1))];
+        auto block = [&](int j) { return verts + 3 * (size_t)__builtin_amdgcn_readlane((int)low, min(j, rows - 1)); };
+        const uint32_t w0 = load_at(pidx, min((uint32_t)lane, flast));
+        uint32_t w = load_at(pidx, min(64u + lane, flast));
+        const SFH_GLOBAL float* vb = block(0);
+        f3 p1 = vert_at(vb, unpack_id(w0, 0)), p2 = vert_at(vb, unpack_id(w0, 1)), p3 = vert_at(vb, unpack_id(w0, 2));
+        for (int j = 0; j < rows; ++j) {
+            vb = block(j + 1);
+            const f3 q1 = vert_at(vb, unpack_id(w, 0)), q2 = vert_at(vb, unpack_id(w, 1)), q3 = vert_at(vb, unpack_id(w, 2));
+            w = load_at(pidx, min(64u * (j + 2) + lane, flast));
+            if (64u * j + lane < nfc) {
+                if (AERO) {
+                    if (NU) face_aero(fb, p1, p2, p3, flow, acc);
+                    else face_aero(fb, p1, p2, p3, NoFlow(), acc);
+                } else if (NU) {
+                    face_submerged(fb, p1, p2, p3, flow, acc);
+                } else {
+                    face_submerged(fb, p1, p2, p3, acc);
+                }
+            }
+            p1 = q1; p2 = q2; p3 = q3;
+        }
     }
     double vals[12];
 #pragma unroll
@@ -947,14 +1100,23 @@ __device__ __forceinline__ void wet_contrib(const Wet& wt, const FaceBody& fb, c
     acc.Swet += wt.A;
 }
 
-// Surface loop (bodies crossing the surface), one chunk: the FP64 depths of
-// the chunk's vertex window (WIN: into the wavefront's LDS slice first;
-// otherwise per face vertex as the faces come), then the faces: all-wet
-// faces inline; faces the waterline cuts (clip cases A-F) queued in LDS and
-// clipped together afterwards, 64 at a time, so the clip code runs once per
-// 64 cut faces rather than on every pass over the chunk.  Tetra volumes,
-// pressure buoyancy with waves, drag.
-template <int K, bool NU, int NL, bool WIN>
+// Surface loop (bodies crossing the surface), one chunk: the FP64 depths of the
+// chunk's vertex window into the wavefront's LDS slice (WIN; otherwise per face
+// vertex as the faces come), then the faces: the all-wet ones as the rows of 64
+// come, the ones the waterline cuts (clip cases A-F) queued in LDS and clipped
+// together afterwards, 64 at a time, so the clip code runs once per 64 of them.
+// Tetra volumes, pressure buoyancy with waves, drag.
+//
+// SPLIT (large batches on waves, kSplitChunks): the rows are taken twice, first
+// which of their faces are all wet (a mask of the row, kept in lane `row` of a
+// register pair) and which are cut, from the packed vertex numbers and the
+// depths alone; then the all-wet faces of the rows that have any, from the face
+// records (REC) or from the vertices, so that dry rows load nothing and neither
+// pass holds the other's registers.  A chunk whose window is wholly wet needs no
+// first pass.  On a flat sea, where the volume takes the vertices of every wet
+// face, one pass is the faster (4,096 states of a hull of 5,112 faces: 87 us a
+// step, 104 in two passes).
+template <int K, bool NU, int NL, bool WIN, bool REC, bool SPLIT>
 __device__ __forceinline__ void cross_chunk(uint32_t c, uint32_t f0, uint32_t nfc, uint32_t vlo, uint32_t vn,
                                             const BodyStatic& S, const BodyDyn& D, const OceanK& oc,
                                             const WaveQ<NL>& wq, float* __restrict__ ldep,
@@ -963,20 +1125,35 @@ __device__ __forceinline__ void cross_chunk(uint32_t c, uint32_t f0, uint32_t nf
     const uint64_t below = (1ull << lane) - 1ull;
     const SFH_GLOBAL float* __restrict__ verts = gptr(S.verts);
     const SFH_GLOBAL uint32_t* __restrict__ faces = gptr(S.faces) + 3 * (size_t)f0;
+    const SFH_GLOBAL uint32_t* __restrict__ pidx = gptr(S.pidx) + f0;
+    const SFH_GLOBAL f32x4* __restrict__ r0 = (const SFH_GLOBAL f32x4*)S.recs + f0;
+    const SFH_GLOBAL f32x4* __restrict__ r2 = r0 + 2 * (size_t)S.nf;
+    const double lo_unit = S.lo_unit;
     const FaceBody fb = D.fb;
     const uint32_t flags = D.flags;
     const bool damping = flags & BF_DAMPING;
     const bool wave_buoy = (flags & BF_BUOYANT) && oc.nlayers > 0;
     const f3 zero = mk3(0.f, 0.f, 0.f);
+    // face numbers past the chunk are clamped to its last face so every load
+    // stays in bounds; their results are not used
+    const uint32_t flast = nfc - 1;
+    const int rows = (int)((nfc + 63u) / 64u);
+    const uint64_t tail = ~0ull >> (64u * rows - nfc);   // the last row's faces
+    // lane k holds block k's lowest vertex id; like the first row's numbers it
+    // is requested before the window's vertices, whose work covers it
+    const uint32_t low = SPLIT ? gptr((const uint32_t*)S.blkwin)[2 * (f0 / 64 + min(lane, rows - 1))] : 0u;
+    uint32_t w = SPLIT && WIN ? load_at(pidx, min((uint32_t)lane, flast)) : 0u;
+    bool whole = false;   // every vertex of the window is wet
     if (WIN) {
         // four vertices per lane in flight: their loads, then their texel
         // gathers, issue together (indices past the window are clamped to
         // its last vertex; those results are not stored)
-        bool wet = false;
+        bool wet = false, dry = false;
+        const SFH_GLOBAL float* __restrict__ wverts = verts + 3 * (size_t)vlo;
         for (uint32_t v0 = 0; v0 < vn; v0 += 256u) {
             f3 p[4];
 #pragma unroll
-            for (int k = 0; k < 4; ++k) p[k] = vert(verts, vlo + min(v0 + 64u * k + lane, vn - 1));
+            for (int k = 0; k < 4; ++k) p[k] = vert_at(wverts, min(v0 + 64u * k + lane, vn - 1));
             float d[4];
 #pragma unroll
             for (int k = 0; k < 4; ++k) d[k] = (float)wq.depth(p[k], zero);
@@ -985,17 +1162,17 @@ __device__ __forceinline__ void cross_chunk(uint32_t c, uint32_t f0, uint32_t nf
                 if (v0 + 64u * k + lane < vn) {
                     ldep[v0 + 64u * k + lane] = d[k];
                     wet |= !(d[k] < 0.f);
+                    dry |= d[k] < 0.f;
                 }
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_lds_sync();
         if (__ballot(wet) == 0ull) {
             // every vertex of the window is dry: every face of the chunk is
             // skipped (SolidEntity.cpp:1353), the chunk contributes nothing
             if (lane < kChunkDoubles) gptr_w(partials)[(size_t)c * kChunkDoubles + lane] = 0.0;
             return;
         }
+        whole = __ballot(dry) == 0ull;
     }
     auto dep = [&](uint32_t i, f3 p) -> float {
         if (WIN) return ldep[i - vlo];
@@ -1006,35 +1183,154 @@ __device__ __forceinline__ void cross_chunk(uint32_t c, uint32_t f0, uint32_t nf
     constexpr bool CBON = NL <= 0;
     Acc<float> acc;
     acc_zero(acc);
-    const uint32_t flast = nfc - 1;
-    uint32_t fc0 = min((uint32_t)lane, flast), fc1 = min(64u + lane, flast);
-    uint32_t a0 = faces[3 * fc0], a1 = faces[3 * fc0 + 1], a2 = faces[3 * fc0 + 2];
-    uint32_t b0 = faces[3 * fc1], b1 = faces[3 * fc1 + 1], b2 = faces[3 * fc1 + 2];
-    f3 p1 = vert(verts, a0), p2 = vert(verts, a1), p3 = vert(verts, a2);
     uint32_t ncut = 0;
-    // unrolled by two: the pipeline's registers alternate instead of being
-    // copied at the end of every face
+    if (!SPLIT) {
+        uint32_t fc0 = min((uint32_t)lane, flast), fc1 = min(64u + lane, flast);
+        uint32_t a0 = faces[3 * fc0], a1 = faces[3 * fc0 + 1], a2 = faces[3 * fc0 + 2];
+        uint32_t b0 = faces[3 * fc1], b1 = faces[3 * fc1 + 1], b2 = faces[3 * fc1 + 2];
+        f3 p1 = vert(verts, a0), p2 = vert(verts, a1), p3 = vert(verts, a2);
+        // unrolled by two: the pipeline's registers alternate instead of being
+        // copied at the end of every face
 #pragma unroll 2
-    for (int j = 0; j < K; ++j) {
-        const uint32_t fn2 = min(64u * (j + 2) + lane, flast);
-        f3 q1 = vert(verts, b0), q2 = vert(verts, b1), q3 = vert(verts, b2);
-        uint32_t c0 = faces[3 * fn2], c1 = faces[3 * fn2 + 1], c2 = faces[3 * fn2 + 2];
-        const float d0 = dep(a0, p1), d1 = dep(a1, p2), d2 = dep(a2, p3);
-        const bool valid = 64u * j + lane < nfc;
-        const bool allwet = !(d0 < 0.f) && !(d1 < 0.f) && !(d2 < 0.f);
-        const bool cut = valid && !allwet && !(d0 < 0.f && d1 < 0.f && d2 < 0.f);
-        if (valid && allwet)
-            wet_contrib<NU, NL>(face_allwet<float, CBON>(fb, p1, p2, p3, acc), fb, D, wq, wave_buoy, damping, acc);
-        const uint64_t m = __ballot(cut);
-        if (cut) cutq[ncut + (uint32_t)__popcll(m & below)] = (uint16_t)(64u * j + lane);
-        ncut += (uint32_t)__popcll(m);
-        p1 = q1; p2 = q2; p3 = q3;
-        a0 = b0; a1 = b1; a2 = b2;
-        b0 = c0; b1 = c1; b2 = c2;
+        for (int j = 0; j < K; ++j) {
+            const uint32_t fn2 = min(64u * (j + 2) + lane, flast);
+            f3 q1 = vert(verts, b0), q2 = vert(verts, b1), q3 = vert(verts, b2);
+            uint32_t c0 = faces[3 * fn2], c1 = faces[3 * fn2 + 1], c2 = faces[3 * fn2 + 2];
+            const float d0 = dep(a0, p1), d1 = dep(a1, p2), d2 = dep(a2, p3);
+            const bool valid = 64u * j + lane < nfc;
+            const bool allwet = !(d0 < 0.f) && !(d1 < 0.f) && !(d2 < 0.f);
+            const bool cut = valid && !allwet && !(d0 < 0.f && d1 < 0.f && d2 < 0.f);
+            if (valid && allwet)
+                wet_contrib<NU, NL>(face_allwet<float, CBON>(fb, p1, p2, p3, acc), fb, D, wq, wave_buoy, damping, acc);
+            const uint64_t m = __ballot(cut);
+            if (cut) cutq[ncut + (uint32_t)__popcll(m & below)] = (uint16_t)(64u * j + lane);
+            ncut += (uint32_t)__popcll(m);
+            p1 = q1; p2 = q2; p3 = q3;
+            a0 = b0; a1 = b1; a2 = b2;
+            b0 = c0; b1 = c1; b2 = c2;
+        }
+        wave_lds_sync();
+    } else {
+        uint32_t wet_rows = rows >= 32 ? 0xffffffffu : (1u << rows) - 1u;   // rows with an all-wet face
+        uint32_t mask_lo = 0xffffffffu, mask_hi = 0xffffffffu;             // row `lane`'s all-wet faces
+        if (!whole) {
+            wet_rows = 0;
+            auto classify = [&](int j, float d0, float d1, float d2) {
+                const uint64_t w0 = __ballot(!(d0 < 0.f)), w1 = __ballot(!(d1 < 0.f)), w2 = __ballot(!(d2 < 0.f));
+                const uint64_t in = j == rows - 1 ? tail : ~0ull, all = w0 & w1 & w2 & in;
+                const uint64_t cut = (w0 | w1 | w2) & in & ~all;
+                if (lane == j) { mask_lo = (uint32_t)all; mask_hi = (uint32_t)(all >> 32); }
+                if (all) wet_rows |= 1u << j;
+                if (cut) {
+                    if (__builtin_amdgcn_inverse_ballot_w64(cut))
+                        cutq[ncut + (uint32_t)__popcll(cut & below)] = (uint16_t)(64u * j + lane);
+                    ncut += (uint32_t)__popcll(cut);
+                }
+            };
+            if (WIN) {
+                for (int j = 0; j < rows; ++j) {
+                    const float* at = ldep + ((uint32_t)__builtin_amdgcn_readlane((int)low, j) - vlo);
+                    const float d0 = at[unpack_id(w, 0)], d1 = at[unpack_id(w, 1)], d2 = at[unpack_id(w, 2)];
+                    w = load_at(pidx, min(64u * (j + 1) + lane, flast));
+                    classify(j, d0, d1, d2);
+                }
+            } else {
+                for (int j = 0; j < rows; ++j) {
+                    const uint32_t f = min(64u * j + lane, flast);
+                    const uint32_t a0 = faces[3 * f], a1 = faces[3 * f + 1], a2 = faces[3 * f + 2];
+                    classify(j, dep(a0, vert(verts, a0)), dep(a1, vert(verts, a1)), dep(a2, vert(verts, a2)));
+                }
+            }
+            wave_lds_sync();
+        } else if (lane == rows - 1) {
+            mask_lo = (uint32_t)tail;
+            mask_hi = (uint32_t)(tail >> 32);
+        }
+        auto row_mask = [&](int j) {
+            return (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)mask_lo, j) |
+                   (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)mask_hi, j) << 32;
+        };
+        if (wet_rows) {
+            // the wet rows in turn; past the last one it stays
+            auto next = [&](int j) {
+                if (!wet_rows) return j;
+                const int k = __builtin_ctz(wet_rows);
+                wet_rows &= wet_rows - 1u;
+                return k;
+            };
+            int left = __builtin_popcount(wet_rows), j = next(0), jn = next(j);
+            if (REC) {
+                const uint32_t fc = min(64u * j + lane, flast);
+                f32x4 a = load_at(r0, fc), b = load_at(r2, fc);
+                for (;;) {
+                    const uint32_t fn = min(64u * jn + lane, flast);
+                    const f32x4 an = load_at(r0, fn), bn = load_at(r2, fn);   // in flight while row j is computed
+                    const FaceRec r = make_rec(a, b);
+                    if (__builtin_amdgcn_inverse_ballot_w64(row_mask(j))) {
+                        acc.V6 += record_volume(fb, r.c, r.n1, r.A);
+                        if (r.A >= 0.f) {
+                            typename WaveQ<NL>::Pending q;
+                            double x[3];
+                            rec_centroid(r.c, r.lo, lo_unit, x);
+                            if (wave_buoy) q = wq.issue(x[0], x[1], x[2]);
+                            if (damping) face_drag(fb, r.c, r.n1, r.A, acc);
+                            if (wave_buoy) {
+                                const float dc = (float)wq.finish(q);
+                                f3 fbi = r.n1 * (-r.A * dc);
+                                add3(acc.Fb, fbi);
+                                add3(acc.Mb, cross(r.c, fbi));
+                            }
+                            acc.Swet += r.A;
+                        }
+                    }
+                    if (--left == 0) break;
+                    j = jn;
+                    jn = next(jn);
+                    a = an; b = bn;
+                }
+            } else {
+                // row j is computed, row jn's vertices and the row after's numbers
+                // are in flight
+                struct Ids { uint32_t a, b, c; };
+                auto numbers = [&](int row) {
+                    const uint32_t f = min(64u * row + lane, flast);
+                    Ids n = {0, 0, 0};
+                    if (WIN) {
+                        n.a = load_at(pidx, f);
+                    } else {
+                        n.a = faces[3 * f]; n.b = faces[3 * f + 1]; n.c = faces[3 * f + 2];
+                    }
+                    return n;
+                };
+                auto points = [&](int row, Ids n, f3& p1, f3& p2, f3& p3) {
+                    if (WIN) {
+                        const SFH_GLOBAL float* vb = verts + 3 * (size_t)__builtin_amdgcn_readlane((int)low, row);
+                        p1 = vert_at(vb, unpack_id(n.a, 0));
+                        p2 = vert_at(vb, unpack_id(n.a, 1));
+                        p3 = vert_at(vb, unpack_id(n.a, 2));
+                    } else {
+                        p1 = vert(verts, n.a); p2 = vert(verts, n.b); p3 = vert(verts, n.c);
+                    }
+                };
+                const Ids nj = numbers(j);
+                Ids nn = numbers(jn);
+                f3 p1, p2, p3;
+                points(j, nj, p1, p2, p3);
+                for (;;) {
+                    f3 q1, q2, q3;
+                    points(jn, nn, q1, q2, q3);
+                    const int jm = next(jn);
+                    nn = numbers(jm);
+                    if (__builtin_amdgcn_inverse_ballot_w64(row_mask(j)))
+                        wet_contrib<NU, NL>(face_allwet<float, CBON>(fb, p1, p2, p3, acc), fb, D, wq, wave_buoy, damping, acc);
+                    if (--left == 0) break;
+                    j = jn;
+                    jn = jm;
+                    p1 = q1; p2 = q2; p3 = q3;
+                }
+            }
+        }
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     for (uint32_t qb = 0; qb < ncut; qb += 64) {
         if (qb + lane < ncut) {
             const uint32_t fo = cutq[qb + lane];
@@ -1045,9 +1341,7 @@ __device__ __forceinline__ void cross_chunk(uint32_t c, uint32_t f0, uint32_t nf
         }
     }
     // the queue and the depth window are rewritten by the next chunk
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_lds_sync();
     // chunk partial layout: Fdq Mdq Fdf Mdf Fb Mb CB (3 each), V6, Swet
     double vals[24];
 #pragma unroll
@@ -1303,13 +1597,6 @@ __device__ void epilogue_sums(const BodyStatic& S, const double* partials, doubl
     if (q >= 0) ps[q] = v[0];
 }
 
-__device__ __forceinline__ void wave_lds_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // kEpilogueWaves wavefronts per workgroup; wavefront w of W takes the bodies
 // w, w + W, w + 2W, ...: lane k reads the position of the k-th of the
 // wavefront's next 64 bodies in one load.  Of those with face work (positions
@@ -1404,15 +1691,31 @@ __global__ __launch_bounds__(64 * kEpilogueWaves, 4) void k_epilogue(
 // own occupancy.
 static constexpr int kPassSub = 1, kPassCross = 2, kPassBoth = 3, kPassAero = 4;
 
-template <int K, bool NU, int NL, int PASS>
-__global__ __launch_bounds__(256, NU ? 1 : ((PASS & kPassCross) ? 5 : 8)) void k_faces(
+// A workgroup is one wavefront: a chunk's LDS is free as soon as its own
+// wavefront ends (workgroups of four: the 6,000 compounds 3 %, the 1,280-body
+// fleet 3 % and the 4,096 states 2 % slower).
+static constexpr int kFaceWaves = 1;
+
+// Wavefronts per SIMD the face kernels are built for: 8 for the submerged loop
+// alone; 5 with the crossing loop at 16 and 32 faces per lane, which large
+// batches use (4, without a spill: the 6,000 compounds 6 %, the fleet 5 %
+// slower); 3 at up to 8 faces per lane, for batches of few chunks, whose
+// wavefronts are mostly alone and wait for their own loads, which a spill's
+// wait drains (fleets of 120 and 240 bodies at 8 faces per lane 40.4 and 44.3
+// -> 35.3 and 39.3 us a step).
+constexpr int face_occupancy(int K, bool NU, int PASS)
+{
+    return NU ? 1 : (PASS & 2) ? (K <= 8 ? 3 : 5) : 8;
+}
+template <int K, bool NU, int NL, int PASS, bool REC, bool SPLIT>
+__global__ __launch_bounds__(64 * kFaceWaves, face_occupancy(K, NU, PASS)) void k_faces(
     const uint32_t* __restrict__ list, const uint32_t* __restrict__ counts, uint32_t nc,
     const Chunk* __restrict__ chunks, const BodyStatic* __restrict__ st, const BodyDyn* __restrict__ dyn, OceanK oc,
     double* __restrict__ partials)
 {
     constexpr bool CROSS = (PASS & kPassCross) != 0;
-    __shared__ uint16_t cutq[4][CROSS ? 64 * K : 1];
-    __shared__ float ldep[4][CROSS ? win_cap(K) : 1];
+    __shared__ uint16_t cutq[kFaceWaves][CROSS ? 64 * K : 1];
+    __shared__ float ldep[kFaceWaves][CROSS ? win_cap(K) : 1];
     const int lane = threadIdx.x & 63;
     const int wl = threadIdx.x >> 6;
     const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
@@ -1430,16 +1733,16 @@ __global__ __launch_bounds__(256, NU ? 1 : ((PASS & kPassCross) ? 5 : 8)) void k
         const BodyStatic& S = st[b];
         const BodyDyn& D = dyn[b];
         if (!CROSS || !is_cross) {
-            sub_chunk<K, NU, PASS == kPassAero>(c, f0, nfc, S, D, partials, lane);
+            sub_chunk<K, NU, PASS == kPassAero, REC>(c, f0, nfc, S, D, partials, lane);
         } else {
             const uint32_t vlo = __builtin_amdgcn_readfirstlane(ch.vlo);
             const uint32_t vn = __builtin_amdgcn_readfirstlane(ch.vn);
             WaveQ<NL> wq;
             wq.load(D, oc);
             if (vn > 0 && vn <= win_cap(K))
-                cross_chunk<K, NU, NL, true>(c, f0, nfc, vlo, vn, S, D, oc, wq, ldep[wl], cutq[wl], partials, lane);
+                cross_chunk<K, NU, NL, true, REC, SPLIT>(c, f0, nfc, vlo, vn, S, D, oc, wq, ldep[wl], cutq[wl], partials, lane);
             else
-                cross_chunk<K, NU, NL, false>(c, f0, nfc, vlo, vn, S, D, oc, wq, ldep[wl], cutq[wl], partials, lane);
+                cross_chunk<K, NU, NL, false, REC, SPLIT>(c, f0, nfc, vlo, vn, S, D, oc, wq, ldep[wl], cutq[wl], partials, lane);
         }
     }
 }
@@ -1562,43 +1865,20 @@ struct StepFaces {
     }
 };
 
-// A wet polygon's centroid, rounded once (fused) or after the offset.
-template <bool FUSED>
-__device__ __forceinline__ f3 step_centroid(f3 base, f3 cs, float ck)
-{
-#pragma clang fp contract(off)
-    if (FUSED)
-        return mk3(__builtin_fmaf(cs.x, ck, base.x), __builtin_fmaf(cs.y, ck, base.y), __builtin_fmaf(cs.z, ck, base.z));
-    const float x = cs.x * ck, y = cs.y * ck, z = cs.z * ck;
-    return mk3(base.x + x, base.y + y, base.z + z);
-}
-
 // Transposed FP64 reduction of 6 per-lane values over the wavefront's lanes
 // (the tree of xreduce24): lane l with (2 b4 + b3) != 3 and b2 = b1 = b0 = 0
 // holds the total of quantity 3 b5 + 2 b4 + b3 in v[0].
 __device__ __forceinline__ void xreduce6(double (&v)[6], int lane)
 {
-    bool hi = lane & 32;
 #pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        double send = hi ? v[i] : v[i + 3], keep = hi ? v[i + 3] : v[i];
-        v[i] = keep + __shfl_xor(send, 32, 64);
-    }
+    for (int i = 0; i < 3; ++i) v[i] = xstep<32>(v[i], v[i + 3], lane);
     v[3] = 0.0;
-    hi = lane & 16;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        double send = hi ? v[i] : v[i + 2], keep = hi ? v[i + 2] : v[i];
-        v[i] = keep + __shfl_xor(send, 16, 64);
-    }
-    hi = lane & 8;
-    {
-        double send = hi ? v[0] : v[1], keep = hi ? v[1] : v[0];
-        v[0] = keep + __shfl_xor(send, 8, 64);
-    }
-    v[0] += __shfl_xor(v[0], 4, 64);
-    v[0] += __shfl_xor(v[0], 2, 64);
-    v[0] += __shfl_xor(v[0], 1, 64);
+    for (int i = 0; i < 2; ++i) v[i] = xstep<16>(v[i], v[i + 2], lane);
+    v[0] = xstep<8>(v[0], v[1], lane);
+    v[0] += lane_xor<4>(v[0]);
+    v[0] += lane_xor<2>(v[0]);
+    v[0] += lane_xor<1>(v[0]);
 }
 
 __device__ __forceinline__ int xreduce6_slot(int lane)
@@ -1767,21 +2047,18 @@ __device__ __forceinline__ void step_chunk(StepShared<K, NU, AERO>& sh, const Ch
                 const f3 p = vert(sf.verts, vlo + k);
                 sh.sv[k] = make_float4(p.x, p.y, p.z, 0.f);
             }
-        // the geometry of face_submerged, face_aero and face_allwet
+        const SFH_GLOBAL f32x4* r0 = (const SFH_GLOBAL f32x4*)S.recs + ch.first;
+        const SFH_GLOBAL f32x4* r1 = r0 + S.nf;
 #pragma unroll 2
         for (uint32_t f = t - 64; f < nfc; f += 192) {
-            const SFH_GLOBAL uint32_t* i = sf.faces + 3 * (size_t)f;
-            const uint32_t i0 = i[0], i1 = i[1], i2 = i[2];
-            const f3 p1 = vert(sf.verts, i0), p2 = vert(sf.verts, i1), p3 = vert(sf.verts, i2);
-            if (!AERO && win)
-                sh.sf[f] = make_ushort4((uint16_t)(i0 - vlo), (uint16_t)(i1 - vlo), (uint16_t)(i2 - vlo), 0);
-            const f3 e1 = p2 - p1, e2 = p3 - p1;
-            const f3 n = cross(e1, e2);
-            const float n2 = dot(n, n);
-            const float inv = frsq(n2);
-            const f3 n1 = n * inv, c = step_centroid<true>(p1, e1 + e2, 1.0f / 3.0f);
-            sh.r0[f] = make_float4(n1.x, n1.y, n1.z, n2 < SFH_DEGENERATE_N2 ? -1.f : 0.5f * (n2 * inv));
-            sh.r1[f] = make_float4(c.x, c.y, c.z, 0.f);
+            const f32x4 a = r0[f], b = r1[f];
+            if (!AERO && win) {
+                const uint32_t w = gptr(S.pidx)[ch.first + f], at = S.blkwin[(ch.first + f) / 64].x - vlo;
+                sh.sf[f] = make_ushort4((uint16_t)(at + unpack_id(w, 0)), (uint16_t)(at + unpack_id(w, 1)),
+                                        (uint16_t)(at + unpack_id(w, 2)), 0);
+            }
+            sh.r0[f] = make_float4(a.x, a.y, a.z, a.w);
+            sh.r1[f] = make_float4(b.x, b.y, b.z, b.w);
         }
     }
     __syncthreads();
@@ -1817,8 +2094,6 @@ __device__ __forceinline__ void step_chunk(StepShared<K, NU, AERO>& sh, const Ch
                 wq.fu[l] = uni(wq.fu[l]);
                 wq.fv[l] = uni(wq.fv[l]);
                 for (int k = 0; k < 3; ++k) { wq.ru[l][k] = uni(wq.ru[l][k]); wq.rv[l][k] = uni(wq.rv[l][k]); }
-                wq.ku[l] = uni(wq.ku[l]);
-                wq.kv[l] = uni(wq.kv[l]);
             }
         }
         if (win) {
@@ -1896,10 +2171,10 @@ __device__ __forceinline__ void step_chunk(StepShared<K, NU, AERO>& sh, const Ch
         }
     } else if (NU) {
         for (uint32_t f = t; f < nfc; f += 256) {
-            const StepFace q = sf.points(f);
-            const f3 u = flow(((double)q.p1.x + (double)q.p2.x + (double)q.p3.x) / 3.0,
-                              ((double)q.p1.y + (double)q.p2.y + (double)q.p3.y) / 3.0,
-                              ((double)q.p1.z + (double)q.p2.z + (double)q.p3.z) / 3.0);
+            const float4 b = sh.r1[f];
+            double x[3];
+            rec_centroid(mk3(b.x, b.y, b.z), __float_as_int(b.w), S.lo_unit, x);
+            const f3 u = flow(x[0], x[1], x[2]);
             sh.uf[0][f] = u.x; sh.uf[NU ? 1 : 0][f] = u.y; sh.uf[NU ? 2 : 0][f] = u.z;
         }
         __syncthreads();
@@ -2131,9 +2406,14 @@ __global__ __launch_bounds__(256) void k_wave_quad(const float* __restrict__ dat
 // batch (and the per-body workspace) that keeps the mesh's device pointers holds
 // another, so sfh_mesh_destroy never frees memory a batch still reads.
 struct sfh_mesh_t {
+    void* d_mem = nullptr;              // one allocation: face records, packed faces, vertices, faces, block windows
+    float4* d_recs = nullptr;
     float* d_verts = nullptr;
     uint32_t* d_faces = nullptr;
     uint2* d_blkwin = nullptr;          // per block of 64 faces: lowest and highest vertex id referenced
+    uint32_t* d_pidx = nullptr;         // packed faces
+    bool packed = true;                 // every block spans at most kPackSpan ids
+    double lo_unit = 0.0;               // of the face records
     std::vector<uint2> blkwin;          // the same on the host
     uint32_t nv = 0, nf = 0;
     float aabb_min[3], aabb_max[3];
@@ -2146,9 +2426,7 @@ static std::atomic<uint64_t> g_mesh_ids{1};
 static void mesh_release(sfh_mesh_t* m)
 {
     if (m && m->refs.fetch_sub(1) == 1) {
-        hipFree(m->d_verts);
-        hipFree(m->d_faces);
-        hipFree(m->d_blkwin);
+        hipFree(m->d_mem);
         delete m;
     }
 }
@@ -2197,6 +2475,7 @@ struct sfh_batch_t {
     double* d_partials = nullptr;
     uint32_t* d_done = nullptr;     // per body: chunks k_step finished in this step (zero between steps)
     bool all_faces = false;         // every body has at least one chunk
+    bool recs = true;               // the face launch reads the meshes' face records, else their packed faces
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
     bool timing = false;
@@ -2215,7 +2494,7 @@ static OceanK make_oceank(const sfh_ocean_t* o)
     for (int i = 0; i < 3; ++i) k.g[i] = o->g[i];
     k.nlayers = o->nlayers;
     k.n = (int32_t)o->n;
-    k.nmask = (o->n && (o->n & (o->n - 1)) == 0) ? (int32_t)o->n - 1 : -1;
+    k.nmask = (o->n && o->n <= kMaskedGrid && (o->n & (o->n - 1)) == 0) ? (int32_t)o->n - 1 : -1;
     for (int l = 0; l < kMaxLayers; ++l) {
         k.len[l] = o->len[l];
         k.scale[l] = o->len[l] > 0.0 ? (double)o->n / o->len[l] : 0.0;
@@ -2265,7 +2544,13 @@ extern "C" int sfh_mesh_create(const void* vertex_pos, size_t vertex_stride, uin
     std::vector<uint32_t> remap(nv, UINT32_MAX);
     std::vector<uint32_t> order;
     order.reserve(nv);
-    std::vector<uint32_t> faces(3 * (size_t)nf);
+    // vertices, faces and block windows as they lie in device memory, each at a multiple of 16 bytes
+    auto align16 = [](size_t x) { return (x + 15) & ~(size_t)15; };
+    const size_t nblk = ((size_t)nf + 63) / 64;
+    const size_t at_faces = align16(12 * (size_t)nv), at_blk = align16(at_faces + 12 * (size_t)nf);
+    std::vector<uint64_t> image((at_blk + 8 * nblk + 7) / 8);
+    float* verts = (float*)image.data();
+    uint32_t* faces = (uint32_t*)((char*)image.data() + at_faces);
     for (size_t i = 0; i < 3 * (size_t)nf; ++i) {
         uint32_t v = face_ids[i];
         if (remap[v] == UINT32_MAX) {
@@ -2279,7 +2564,6 @@ extern "C" int sfh_mesh_create(const void* vertex_pos, size_t vertex_stride, uin
             remap[v] = (uint32_t)order.size();
             order.push_back(v);
         }
-    std::vector<float> verts(3 * (size_t)nv);
     const char* src = (const char*)vertex_pos;
     float mn[3] = {0, 0, 0}, mx[3] = {0, 0, 0};
     for (uint32_t i = 0; i < nv; ++i) {
@@ -2303,21 +2587,37 @@ extern "C" int sfh_mesh_create(const void* vertex_pos, size_t vertex_stride, uin
             hi = std::max(hi, faces[i]);
         }
         m->blkwin[k] = make_uint2(lo, hi);
+        m->packed = m->packed && hi - lo < kPackSpan;
     }
     for (int k = 0; k < 3; ++k) { m->aabb_min[k] = mn[k]; m->aabb_max[k] = mx[k]; }
+    if (nf) memcpy((char*)image.data() + at_blk, m->blkwin.data(), sizeof(uint2) * nblk);
     if (nv) {
-        hipError_t e = hipMalloc(&m->d_verts, verts.size() * sizeof(float));
-        if (e == hipSuccess) e = hipMemcpy(m->d_verts, verts.data(), verts.size() * sizeof(float), hipMemcpyHostToDevice);
-        if (e != hipSuccess) { hipFree(m->d_verts); delete m; return fail(SFH_ERR_HIP, "mesh upload: %s", hipGetErrorString(e)); }
-    }
-    if (nf) {
-        hipError_t e = hipMalloc(&m->d_faces, faces.size() * sizeof(uint32_t));
-        if (e == hipSuccess) e = hipMemcpy(m->d_faces, faces.data(), faces.size() * sizeof(uint32_t), hipMemcpyHostToDevice);
-        if (e == hipSuccess) e = hipMalloc(&m->d_blkwin, m->blkwin.size() * sizeof(uint2));
-        if (e == hipSuccess)
-            e = hipMemcpy(m->d_blkwin, m->blkwin.data(), m->blkwin.size() * sizeof(uint2), hipMemcpyHostToDevice);
+        float size = 0.f;
+        for (int k = 0; k < 3; ++k) size = fmaxf(size, fmaxf(fabsf(mn[k]), fabsf(mx[k])));
+        // centroids lie below 2^(e + 1): their rounding is at most 2^(e - 24), 512 units
+        if (size > 0.f && std::isfinite(size)) m->lo_unit = ldexp(1.0, std::max(ilogbf(size) - 33, -1000));
+        const size_t recs = align16(52 * (size_t)nf), bytes = image.size() * 8;
+        hipError_t e = hipMalloc(&m->d_mem, recs + bytes);
+        if (e == hipSuccess) {
+            char* at = (char*)m->d_mem + recs;
+            m->d_verts = (float*)at;
+            if (nf) {
+                m->d_recs = (float4*)m->d_mem;
+                m->d_pidx = (uint32_t*)(m->d_recs + 3 * (size_t)nf);
+                m->d_faces = (uint32_t*)(at + at_faces);
+                m->d_blkwin = (uint2*)(at + at_blk);
+            }
+            e = hipMemcpy(at, image.data(), bytes, hipMemcpyHostToDevice);
+        }
+        if (e == hipSuccess && nf) {
+            hipLaunchKernelGGL(k_face_records, dim3((nf + 255) / 256), dim3(256), 0, nullptr, m->d_verts, m->d_faces,
+                               m->d_blkwin, nf, m->lo_unit, m->d_recs, m->d_pidx);
+            e = hipGetLastError();
+            if (e == hipSuccess) e = hipStreamSynchronize(nullptr);   // batches read the records on other streams
+        }
         if (e != hipSuccess) {
-            hipFree(m->d_verts); hipFree(m->d_faces); hipFree(m->d_blkwin); delete m;
+            hipFree(m->d_mem);
+            delete m;
             return fail(SFH_ERR_HIP, "mesh upload: %s", hipGetErrorString(e));
         }
     }
@@ -2509,17 +2809,32 @@ static void chunk_window(const std::vector<uint2>& blk, uint32_t first, uint32_t
                          uint32_t& vn)
 {
     uint32_t lo = UINT32_MAX, hi = 0;
+    bool packed = true;
     for (uint32_t k = first / 64; k < (first + count + 63) / 64 && k < blk.size(); ++k) {
         lo = std::min(lo, blk[k].x);
         hi = std::max(hi, blk[k].y);
+        packed = packed && blk[k].y - blk[k].x < kPackSpan;
     }
     vlo = 0;
     vn = 0;
-    if (lo <= hi && hi - lo + 1 <= cap) {
+    if (packed && lo <= hi && hi - lo + 1 <= cap) {
         vlo = lo;
         vn = hi - lo + 1;
     }
 }
+
+// Up to this many faces in the distinct meshes of a batch its face launch reads
+// their records, past it their packed faces and vertices.  The records take 32
+// bytes a face and the least arithmetic; the packed faces take 10 (with their
+// share of the vertices), and the normals, areas and centroids are formed on
+// the way.  While the records stay in the caches the face launch is bound by
+// its arithmetic, then by memory.  Fleets of bodies with a mesh of their own
+// on waves, three states in turn, records / packed (a step, us):
+//     1.4 M faces   38.6 / 40.1        7.4 M   74.9 / 62.0
+//     2.5 M         46.7 / 42.8       14.2 M  119.3 / 98.9
+// and 6,000 compounds sharing two meshes (12,288 faces) 259 / 293.  A batch with
+// a mesh that cannot be packed (faces in no order) reads records.
+static constexpr uint64_t kRecordFaces = 2000000;
 
 // (Re)builds the chunks: every body's faces cut into chunks of 64*K
 // consecutive faces, each with its vertex window.
@@ -2555,6 +2870,18 @@ static int batch_build_chunks(sfh_batch_t* b)
     b->d_static = nullptr; b->d_sidx = nullptr; b->d_chunks = nullptr;
     b->d_partials = nullptr; b->d_bpos = nullptr; b->d_lists = nullptr; b->d_done = nullptr;
     b->nchunks = (uint32_t)chunks.size();
+    std::vector<const sfh_mesh_t*> used;
+    for (const sfh_mesh_t* m : b->meshes_by_body)
+        if (m) used.push_back(m);
+    std::sort(used.begin(), used.end());
+    used.erase(std::unique(used.begin(), used.end()), used.end());
+    uint64_t faces = 0;
+    bool packed = true;
+    for (const sfh_mesh_t* m : used) {
+        faces += m->nf;
+        packed = packed && m->packed;
+    }
+    b->recs = !packed || faces <= kRecordFaces;
     HIPCHK(hipMalloc(&b->d_static, sizeof(BodyStatic) * std::max<size_t>(1, b->n)));
     HIPCHK(hipMemcpy(b->d_static, b->h_static.data(), sizeof(BodyStatic) * b->n, hipMemcpyHostToDevice));
     {
@@ -2598,6 +2925,10 @@ static BodyStatic make_static(const sfh_mesh_t* m, uint32_t flags)
     memset(&s, 0, sizeof(s));
     s.verts = m ? m->d_verts : nullptr;
     s.faces = m ? m->d_faces : nullptr;
+    s.recs = m ? m->d_recs : nullptr;
+    s.pidx = m ? m->d_pidx : nullptr;
+    s.blkwin = m ? m->d_blkwin : nullptr;
+    s.lo_unit = m ? m->lo_unit : 0.0;
     s.nf = m ? m->nf : 0;
     s.nv = m ? m->nv : 0;
     s.flags = flags;
@@ -2915,17 +3246,34 @@ extern "C" int sfh_batch_info(sfh_batch b, uint32_t* nbodies, uint32_t* nchunks,
     return SFH_OK;
 }
 
+// On waves the face launch of batches of more chunks than this takes a crossing
+// chunk's rows twice (cross_chunk's SPLIT): fewer instructions, but a longer
+// chain of waits per chunk, which shows while most wavefronts are alone on
+// their SIMD.  Measured, one pass / two (a step on one wave layer, us): fleets
+// of 1,464 chunks 36.6 / 39.9, 4,381 46.6 / 47.7, 7,520 67.8 / 61.1, 14,436
+// 105.3 / 97.4; one hull, 5,000 chunks 52.5 / 50.9, 20,480 136.0 / 126.6;
+// compounds, 2,400 chunks 48.5 / 48.8, 72,000 303.7 / 269.0.  From 8 faces per
+// lane on: with fewer a chunk is its fixed work more than its rows.
+static constexpr uint32_t kSplitChunks = 4608;
+
 // Launches the face pass over every chunk of the batch.
 static int launch_faces(sfh_batch_t* b, const OceanK& oc, hipStream_t s)
 {
     if (b->nchunks == 0) return SFH_OK;
     const uint32_t waves = std::min<uint32_t>(std::max<uint32_t>(b->waves, 1u), b->nchunks);   // grid-strided
-    const uint32_t blocks = (waves + 3) / 4;
+    const uint32_t blocks = (waves + kFaceWaves - 1) / kFaceWaves;
+#define LAUNCH_R(KK, NU, NL, PASS, REC, SP)                                                                     \
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_faces<KK, NU, NL, PASS, REC, SP>), dim3(blocks), dim3(64 * kFaceWaves), \
+                       0, s, b->d_lists, b->d_lists + b->nchunks, b->nchunks, b->d_chunks, b->d_static,         \
+                       b->d_dyn, oc, b->d_partials)
 #define LAUNCH_F(KK, NU, NL, PASS)                                                                              \
     {                                                                                                           \
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_faces<KK, NU, NL, PASS>), dim3(blocks), dim3(256), 0, s,          \
-                           b->d_lists, b->d_lists + b->nchunks, b->nchunks, b->d_chunks, b->d_static, b->d_dyn, \
-                           oc, b->d_partials);                                                                  \
+        constexpr bool sp = NL > 0 && !NU && (PASS & kPassCross) && KK >= 8;                                    \
+        if (sp && b->nchunks > kSplitChunks) {                                                                  \
+            if (b->recs) LAUNCH_R(KK, NU, NL, PASS, true, sp); else LAUNCH_R(KK, NU, NL, PASS, false, sp);      \
+        } else {                                                                                                \
+            if (b->recs) LAUNCH_R(KK, NU, NL, PASS, true, false); else LAUNCH_R(KK, NU, NL, PASS, false, false); \
+        }                                                                                                       \
     }
 #define LAUNCH_X(KK, NU, NL)                                                                                    \
     {                                                                                                           \
@@ -2953,6 +3301,7 @@ static int launch_faces(sfh_batch_t* b, const OceanK& oc, hipStream_t s)
 #undef LAUNCH_K
 #undef LAUNCH_X
 #undef LAUNCH_F
+#undef LAUNCH_R
     return SFH_OK;
 }
 
