@@ -19,7 +19,7 @@
 //   k_epilogue  one wavefront per body with face work, FP64: sums the body's
 //               chunk partials (fixed order), rotates to world, moment about
 //               the CoG, buoyancy, CorrectHydrodynamicForces, output write mask;
-//   k_compound  compound batches: one lane per compound composes its parts.
+//   k_compound  compound batches: a lane per slot composes the parts' rows.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -1597,6 +1597,50 @@ __device__ void epilogue_sums(const BodyStatic& S, const double* partials, doubl
     if (q >= 0) ps[q] = v[0];
 }
 
+// epilogue_finish on one wavefront for a hydrodynamic body: lanes 0-3 take a
+// drag vector each with its correction (a square root and two divisions in
+// FP64, one after the other on one lane), lane 4 the buoyancy; the row is put
+// together in LDS (24 doubles) and stored by 22 lanes at once.  The same
+// operations as epilogue_finish, so the same bits.
+__device__ __forceinline__ void finish_lanes(const BodyStatic& S, const BodyDyn& D, const OceanK& oc, const double* P,
+                                             double* row, double* __restrict__ o, double* __restrict__ applied, int lane)
+{
+    const uint32_t flags = D.flags;
+    const bool body_level = !(flags & (BF_MODE_SURF | BF_MODE_SUBM | BF_MODE_AERO));
+    uint32_t written = 0;
+    if (lane < 4) {
+        double x[3];
+        finish_drag(D, P, lane, x);
+        if (body_level && (flags & BF_DAMPING)) {
+            double BO[9], M[9];
+            finish_basis(S, D, BO);
+            correct_inverse(BO, M);
+            correct_vector(oc.rho, M, lane < 2 ? S.Cd : S.Cf, lane < 2, x);
+        }
+        for (int k = 0; k < 3; ++k) row[6 + 3 * lane + k] = x[k];
+    } else if (lane == 4) {
+        double Fb[3], Tb[3], Swet, Vsub;
+        written = finish_buoyancy(S, D, oc, P, Fb, Tb, Swet, Vsub);
+        for (int k = 0; k < 3; ++k) { row[k] = Fb[k]; row[3 + k] = Tb[k]; }
+        row[18] = Swet;
+        row[19] = Vsub;
+        row[20] = (double)written;
+        row[21] = (double)D.pos;
+    }
+    written = (uint32_t)__shfl((int)written, 4, 64);
+    wave_lds_sync();
+    // slot k's bit of the write mask: 3 slots per bit up to 18, then one each
+    if (lane < 22 && (lane >= 20 || (written >> (lane < 18 ? lane / 3 : lane - 12)) & 1u)) o[lane] = row[lane];
+    if (applied && lane < 6) {
+        double x[3];
+        for (int q = 0; q < 3; ++q) {   // a slot the row leaves untouched holds what it held
+            const int k = 6 * q + lane;
+            x[q] = (written >> (k / 3)) & 1u ? row[k] : o[k];
+        }
+        applied[lane] = (x[0] + x[1]) + x[2];
+    }
+}
+
 // kEpilogueWaves wavefronts per workgroup; wavefront w of W takes the bodies
 // w, w + W, w + 2W, ...: lane k reads the position of the k-th of the
 // wavefront's next 64 bodies in one load.  Of those with face work (positions
@@ -1611,12 +1655,17 @@ __device__ void epilogue_sums(const BodyStatic& S, const double* partials, doubl
 // It also zeroes the work list's counts for the next step's prologue.
 static constexpr int kEpilogueWaves = 4;
 static constexpr int kEpilogueBatch = 16;
+// Up to this many bodies of several chunks in a wavefront's 64 are finished one
+// after the other over lanes (finish_lanes), more at once with a lane each:
+// one lane's finish is a chain of some 450 FP64 operations.
+static constexpr int kEpilogueFew = 4;
 
 __global__ __launch_bounds__(64 * kEpilogueWaves, 4) void k_epilogue(
     const BodyStatic* __restrict__ st, const BodyDyn* __restrict__ dyn, const int8_t* __restrict__ bpos, uint32_t n,
-    OceanK oc, const double* __restrict__ partials, double* __restrict__ out, uint32_t* __restrict__ counts)
+    OceanK oc, const double* __restrict__ partials, double* __restrict__ out, uint32_t* __restrict__ counts, bool aero)
 {
     __shared__ double ps[kEpilogueWaves][kEpilogueBatch][24];
+    __shared__ double rows[kEpilogueWaves][24];
     const int lane = threadIdx.x & 63;
     const int wl = threadIdx.x >> 6;
     const uint32_t W = gridDim.x * kEpilogueWaves;
@@ -1644,26 +1693,24 @@ __global__ __launch_bounds__(64 * kEpilogueWaves, 4) void k_epilogue(
         }
         uint64_t m = __ballot(nck > 1);
         uint32_t mine = 0;    // lane j < nb: the body in slot j
-        uint32_t first = 0;   // the body in slot 0 (wave-uniform)
         int nb = 0;
         while (m) {
             const uint32_t k = (uint32_t)__builtin_ctzll(m);
             m &= m - 1ull;
             const uint32_t b = base + k * W;
             epilogue_sums<false>(st[b], partials, ps[wl][nb], lane);
-            if (nb == 0) first = b;
             if (lane == nb) mine = b;
             if (++nb == kEpilogueBatch || !m) {
                 wave_lds_sync();
-                // a batch of one keeps the body's index wave-uniform (its
-                // constants come in through scalar loads); the finishing
-                // arithmetic rounds the same either way
-                if (nb == 1) {
-                    if (lane == 0) {
-                        double P[23];
-#pragma unroll
-                        for (int q = 0; q < 23; ++q) P[q] = ps[wl][0][q];
-                        epilogue_finish(st[first], dyn[first], oc, P, out + (size_t)first * SFH_OUT_DOUBLES);
+                // a batch of few keeps the body's index wave-uniform (its
+                // constants come in through scalar loads) and spreads the
+                // finish over lanes; the arithmetic rounds the same either way
+                if (!aero && nb <= kEpilogueFew) {
+                    for (int i = 0; i < nb; ++i) {
+                        const uint32_t b1 = (uint32_t)__builtin_amdgcn_readlane((int)mine, i);
+                        finish_lanes(st[b1], dyn[b1], oc, ps[wl][i], rows[wl],
+                                     out + (size_t)b1 * SFH_OUT_DOUBLES, nullptr, lane);
+                        wave_lds_sync();
                     }
                 } else if (lane < nb) {
                     double P[23];
@@ -1970,50 +2017,6 @@ __device__ __forceinline__ void step_sums(const StepShared<K, NU, AERO>& sh, con
     xreduce6(v, lane);
 }
 
-// epilogue_finish on one wavefront for a hydrodynamic body: lanes 0-3 take a
-// drag vector each with its correction (a square root and two divisions in
-// FP64, one after the other on one lane), lane 4 the buoyancy; the row is put
-// together in LDS (24 doubles) and stored by 22 lanes at once.  The same
-// operations as epilogue_finish, so the same bits.
-__device__ __forceinline__ void finish_lanes(const BodyStatic& S, const BodyDyn& D, const OceanK& oc, const double* P,
-                                             double* row, double* __restrict__ o, double* __restrict__ applied, int lane)
-{
-    const uint32_t flags = D.flags;
-    const bool body_level = !(flags & (BF_MODE_SURF | BF_MODE_SUBM | BF_MODE_AERO));
-    uint32_t written = 0;
-    if (lane < 4) {
-        double x[3];
-        finish_drag(D, P, lane, x);
-        if (body_level && (flags & BF_DAMPING)) {
-            double BO[9], M[9];
-            finish_basis(S, D, BO);
-            correct_inverse(BO, M);
-            correct_vector(oc.rho, M, lane < 2 ? S.Cd : S.Cf, lane < 2, x);
-        }
-        for (int k = 0; k < 3; ++k) row[6 + 3 * lane + k] = x[k];
-    } else if (lane == 4) {
-        double Fb[3], Tb[3], Swet, Vsub;
-        written = finish_buoyancy(S, D, oc, P, Fb, Tb, Swet, Vsub);
-        for (int k = 0; k < 3; ++k) { row[k] = Fb[k]; row[3 + k] = Tb[k]; }
-        row[18] = Swet;
-        row[19] = Vsub;
-        row[20] = (double)written;
-        row[21] = (double)D.pos;
-    }
-    written = (uint32_t)__shfl((int)written, 4, 64);
-    wave_lds_sync();
-    // slot k's bit of the write mask: 3 slots per bit up to 18, then one each
-    if (lane < 22 && (lane >= 20 || (written >> (lane < 18 ? lane / 3 : lane - 12)) & 1u)) o[lane] = row[lane];
-    if (applied && lane < 6) {
-        double x[3];
-        for (int q = 0; q < 3; ++q) {   // a slot the row leaves untouched holds what it held
-            const int k = 6 * q + lane;
-            x[q] = (written >> (k / 3)) & 1u ? row[k] : o[k];
-        }
-        applied[lane] = (x[0] + x[1]) + x[2];
-    }
-}
-
 // What ApplyHydrodynamicForces / ApplyAerodynamicForces hand to Bullet from a
 // row (SolidEntity.cpp:1958-1968).
 __device__ __forceinline__ void tick_applied(const double* o, bool aero, double* a)
@@ -2263,87 +2266,102 @@ struct CompStatic {
     double P_CB[3];
 };
 
-// Composes the part rows into the compound's row (Compound.cpp:291-437), one
-// lane per compound, parts in their order.  Inside: the compound's analytic
+// Composes the part rows into the compound's row (Compound.cpp:291-437), a lane
+// per slot of the row, 32 lanes per compound, parts in their order.  It is a
+// chain of dependent loads and little else: with one lane per compound the row
+// slots and parts came one after the other (200 compounds 12.2 us, 6,000
+// 13.4; now 5.2 and 7.4).  Inside: the compound's analytic
 // buoyancy and the sum of the parts' corrected drag.  Crossing: the sums of
 // the part results, where a part's output the reference leaves untouched
 // keeps the previous part's value (the per-part temporaries are declared once
 // before the loop, Compound.cpp:392-399); internal parts add buoyancy only.
-__global__ void k_compound(const CompStatic* __restrict__ cs, const BodyStatic* __restrict__ st,
-                           const BodyDyn* __restrict__ dyn, uint32_t ncomp, OceanK oc,
-                           const uint8_t* __restrict__ active, const double* __restrict__ part_out,
-                           double* __restrict__ out)
+__global__ __launch_bounds__(256) void k_compound(const CompStatic* __restrict__ cs, const BodyStatic* __restrict__ st,
+                                                  const BodyDyn* __restrict__ dyn, uint32_t ncomp, OceanK oc,
+                                                  const uint8_t* __restrict__ active,
+                                                  const double* __restrict__ part_out, double* __restrict__ out)
 {
-    const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= ncomp) return;
+    const uint32_t c = (blockIdx.x * 256u + threadIdx.x) / 32u;
+    const int k = threadIdx.x & 31;   // the row's slot
+    if (c >= ncomp || k >= 22) return;
     if (active && !active[c]) return;
     const CompStatic& C = cs[c];
     double* o = out + (size_t)c * SFH_OUT_DOUBLES;
     const BodyDyn& D0 = dyn[C.part0];
     const int cpos = D0.cpos;
-    if (cpos < 0) { o[20] = 0.0; o[21] = -1.0; return; }
+    const uint32_t p0 = C.part0, p1 = C.part0 + C.nparts;
+    // the parts' positions, masks and values, eight parts' requests at a time
+    // (a part that takes no part in the step holds any values: they are not used)
+    struct Part {
+        int pos;
+        bool ext;
+        double mask, x;
+    };
+    const int kx = k < 20 ? k : 0;
+    auto parts = [&](auto&& f) {
+        for (uint32_t p = p0; p < p1; p += 8) {
+            Part q[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const uint32_t pi = min(p + i, p1 - 1);
+                const double* row = part_out + (size_t)pi * SFH_OUT_DOUBLES;
+                q[i].pos = dyn[pi].pos;
+                q[i].ext = st[pi].flags & BF_EXTERNAL;
+                q[i].mask = row[20];
+                q[i].x = row[kx];
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                if (p + i < p1) f(q[i]);
+        }
+    };
+    if (cpos < 0) {
+        if (k == 20) o[20] = 0.0;
+        if (k == 21) o[21] = -1.0;
+        return;
+    }
     if (cpos == 0) {
-        for (int k = 0; k < 20; ++k) o[k] = 0.0;
-        o[20] = 255.0; o[21] = 0.0;
+        o[k] = k == 20 ? 255.0 : 0.0;
         return;
     }
     if (C.flags & BF_MODE_AERO) {   // Compound::ComputeAerodynamicForces (Compound.cpp:439-464)
-        double acc[6] = {0, 0, 0, 0, 0, 0};
-        for (uint32_t p = C.part0; p < C.part0 + C.nparts; ++p) {
-            if (dyn[p].pos != 1) continue;
-            const double* row = part_out + (size_t)p * SFH_OUT_DOUBLES;
-            for (int k = 0; k < 6; ++k) acc[k] += row[6 + k];
-        }
-        for (int k = 0; k < 6; ++k) o[6 + k] = acc[k];
-        o[20] = (double)(4u | 8u);
-        o[21] = 1.0;
+        double acc = 0.0;
+        parts([&](const Part& q) { if (q.pos == 1) acc += q.x; });
+        if (k >= 6 && k < 12) o[k] = acc;
+        if (k == 20) o[20] = (double)(4u | 8u);
+        if (k == 21) o[21] = 1.0;
         return;
     }
     if (cpos == 1) {
-        double acc[12];
-        for (int k = 0; k < 12; ++k) acc[k] = 0.0;
-        for (uint32_t p = C.part0; p < C.part0 + C.nparts; ++p) {
-            if (dyn[p].pos != 1) continue;
-            const double* row = part_out + (size_t)p * SFH_OUT_DOUBLES;
-            for (int k = 0; k < 12; ++k) acc[k] += row[6 + k];
+        if (k < 6) {
+            if (C.flags & BF_BUOYANT) {
+                double Fb[3], Tb[3], cb[3];
+                for (int i = 0; i < 3; ++i) Fb[i] = -C.volume * oc.rho * oc.g[i];
+                mat_vec(D0.Rcg, C.P_CB, cb);
+                cross64(cb, Fb, Tb);
+                o[k] = k == 0 ? Fb[0] : k == 1 ? Fb[1] : k == 2 ? Fb[2] : k == 3 ? Tb[0] : k == 4 ? Tb[1] : Tb[2];
+            }
+        } else if (k < 18) {
+            double acc = 0.0;
+            parts([&](const Part& q) { if (q.pos == 1) acc += q.x; });
+            o[k] = acc;
+        } else {
+            const uint32_t written = 4u | 8u | 16u | 32u | 64u | 128u | (C.flags & BF_BUOYANT ? 3u : 0u);
+            o[k] = k == 18 ? C.surface : k == 19 ? C.volume : k == 20 ? (double)written : 1.0;
         }
-        uint32_t written = 4u | 8u | 16u | 32u | 64u | 128u;
-        if (C.flags & BF_BUOYANT) {
-            double Fb[3], Tb[3], cb[3];
-            for (int k = 0; k < 3; ++k) Fb[k] = -C.volume * oc.rho * oc.g[k];
-            mat_vec(D0.Rcg, C.P_CB, cb);
-            cross64(cb, Fb, Tb);
-            for (int k = 0; k < 3; ++k) { o[k] = Fb[k]; o[3 + k] = Tb[k]; }
-            written |= 3u;
-        }
-        for (int k = 0; k < 12; ++k) o[6 + k] = acc[k];
-        o[18] = C.surface;
-        o[19] = C.volume;
-        o[20] = (double)written;
-        o[21] = 1.0;
         return;
     }
-    double carry[20], acc[20];
-    for (int k = 0; k < 20; ++k) carry[k] = acc[k] = 0.0;
-    for (uint32_t p = C.part0; p < C.part0 + C.nparts; ++p) {
-        if (dyn[p].pos != 2) continue;
-        const double* row = part_out + (size_t)p * SFH_OUT_DOUBLES;
-        const uint32_t wm = (uint32_t)row[20];
-        for (int q = 0; q < 6; ++q)
-            if (wm & (1u << q))
-                for (int k = 0; k < 3; ++k) carry[3 * q + k] = row[3 * q + k];
-        if (wm & 64u) carry[18] = row[18];
-        if (wm & 128u) carry[19] = row[19];
-        if (st[p].flags & BF_EXTERNAL) {
-            for (int k = 0; k < 20; ++k) acc[k] += carry[k];
-        } else {
-            for (int k = 0; k < 6; ++k) acc[k] += carry[k];
-            acc[19] += carry[19];
-        }
+    if (k >= 20) {
+        o[k] = k == 20 ? 255.0 : 2.0;
+        return;
     }
-    for (int k = 0; k < 20; ++k) o[k] = acc[k];
-    o[20] = 255.0;
-    o[21] = 2.0;
+    const uint32_t bit = 1u << (k < 18 ? k / 3 : k - 12);
+    double carry = 0.0, acc = 0.0;
+    parts([&](const Part& q) {
+        if (q.pos != 2) return;
+        if ((uint32_t)q.mask & bit) carry = q.x;
+        if (k < 6 || k == 19 || q.ext) acc += carry;
+    });
+    o[k] = acc;
 }
 
 // Standalone CorrectHydrodynamicForces for the per-body entry point.
@@ -3397,13 +3415,17 @@ static int batch_launch(sfh_batch_t* b, const sfh_ocean_t* o, const double* d_st
     if (rc != SFH_OK) return rc;
     if (timed) HIPCHK(hipEventRecord(b->ev[2], s));
     if (b->nchunks) {
-        const uint32_t ewaves = std::min<uint32_t>(b->n, std::max<uint32_t>(1, b->waves / 2));
+        // a quarter of the face launch's wavefronts: the 30,000 parts of 6,000
+        // compounds, most of one chunk and finished by a lane each, leave more
+        // of a wavefront's lanes with work (28.4 -> 20.0 us with kEpilogueFew;
+        // an eighth: 20.5, and 4,096 bodies of five chunks 8.1 -> 10.5)
+        const uint32_t ewaves = std::min<uint32_t>(b->n, std::max<uint32_t>(1, b->waves / 4));
         const uint32_t eblocks = (ewaves + kEpilogueWaves - 1) / kEpilogueWaves;
         hipLaunchKernelGGL(k_epilogue, dim3(eblocks), dim3(64 * kEpilogueWaves), 0, s, b->d_static, b->d_dyn, b->d_bpos, b->n, oc,
-                           b->d_partials, rows, b->d_lists + b->nchunks);
+                           b->d_partials, rows, b->d_lists + b->nchunks, b->aero);
     }
     if (b->compound && b->nunits)
-        hipLaunchKernelGGL(k_compound, dim3((b->nunits + 127) / 128), dim3(128), 0, s, b->d_comp, b->d_static,
+        hipLaunchKernelGGL(k_compound, dim3((b->nunits + 7) / 8), dim3(256), 0, s, b->d_comp, b->d_static,
                            b->d_dyn, b->nunits, oc, active, b->d_part_out, d_out);
     if (timed) HIPCHK(hipEventRecord(b->ev[3], s));
     HIPCHK(hipGetLastError());
