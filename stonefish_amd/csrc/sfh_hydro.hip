@@ -15,7 +15,8 @@
 //               FP32 face arithmetic with FP32 per-lane partials, FP64
 //               wavefront reduction into one 24-double partial per chunk (a
 //               crossing chunk first evaluates the FP64 depths of its vertex
-//               window into LDS);
+//               window into LDS); whole faces come from the mesh's face
+//               records or packed faces (k_face_records, once per mesh);
 //   k_epilogue  one wavefront per body with face work, FP64: sums the body's
 //               chunk partials (fixed order), rotates to world, moment about
 //               the CoG, buoyancy, CorrectHydrodynamicForces, output write mask;
@@ -1806,9 +1807,9 @@ __global__ __launch_bounds__(64 * kFaceWaves, face_occupancy(K, NU, PASS)) void 
 // row:
 //   1. the body's record and state into LDS;
 //   2. wavefront 0 runs the body's prologue (every chunk's workgroup its own;
-//      the record stays in LDS) while the others stage the chunk's vertices
-//      and its faces' window-relative vertex numbers in LDS and form every
-//      face's unit normal, area and centroid, which need no state;
+//      the record stays in LDS) while the others stage the chunk's vertices,
+//      its faces' window-relative vertex numbers and their face records in
+//      LDS, which need no state;
 //   3. crossing chunks: the FP64 depths of the window, then per face whether
 //      it is wet, its tetra volume and its centroid's depth, over all four
 //      wavefronts;
@@ -1823,7 +1824,7 @@ __global__ __launch_bounds__(64 * kFaceWaves, face_occupancy(K, NU, PASS)) void 
 //      counts last sums the partials in chunk order and finishes the row.
 //      It also zeroes the counter for the next step.
 // Measured: a tick of 203 bodies (576 chunks, 60 % overlapped, two wave
-// layers) 39.4 -> 18.3 us, an aerodynamic batch of 300 bodies 16.5 -> 10.8 us,
+// layers) 39.4 -> 17.9 us, an aerodynamic batch of 300 bodies 16.5 -> 9.4 us,
 // the per-body calls 38 -> 32 us (2,070 faces, submerged) and 52 -> 43 us
 // (12,000 faces, surface), 13 us of which are the caller's Python.  Of the
 // tick's kernel 1.0 us are its loads, 2.9 the prologue, 4.3 the depths and the
