@@ -941,7 +941,9 @@ __global__ __launch_bounds__(256) void k_face_records(const float* __restrict__ 
     f3 n1 = n * inv;
     float A = 0.5f * (n2 * inv);
     if (n2 < SFH_DEGENERATE_N2) {
-        if (!(n2 > 0.f)) {
+        // v_rsq_f32 takes no subnormal number (it returns infinity); the volume
+        // of a face of |n| < 1.1e-19 is below the rounding of any body's
+        if (n2 < FLT_MIN) {
             n1 = mk3(0.f, 0.f, 0.f);
             A = 0.f;
         }
