@@ -2920,6 +2920,7 @@ static int batch_build_chunks(sfh_batch_t* b)
     HIPCHK(hipMemset(b->d_lists + b->nchunks, 0, 2 * sizeof(uint32_t)));
     HIPCHK(hipMalloc(&b->d_done, sizeof(uint32_t) * std::max<size_t>(1, b->n)));
     HIPCHK(hipMemset(b->d_done, 0, sizeof(uint32_t) * std::max<size_t>(1, b->n)));
+    HIPCHK(hipStreamSynchronize(nullptr));   // the counters are clear before a step on any stream
     if (b->graph_exec) { hipGraphExecDestroy(b->graph_exec); b->graph_exec = nullptr; }
     if (b->graph) { hipGraphDestroy(b->graph); b->graph = nullptr; }
     return SFH_OK;
@@ -3912,7 +3913,9 @@ static int ws_reserve(Workspace* w, uint32_t F)
     w->d_buf = nullptr;
     w->cap = 0;
     HIPCHK(hipMalloc(&w->d_buf, cap));
-    const hipError_t e = hipMemset(w->d_buf, 0, kSinglePartials);   // the counter starts at zero
+    // the counter starts at zero, cleared on the stream of the launches that
+    // count on it (no other stream orders a non-blocking one)
+    const hipError_t e = hipMemsetAsync(w->d_buf, 0, kSinglePartials, w->stream);
     if (e != hipSuccess) {
         hipFree(w->d_buf);
         w->d_buf = nullptr;
