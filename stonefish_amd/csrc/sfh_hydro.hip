@@ -858,7 +858,8 @@ __device__ __forceinline__ f3 vert(const SFH_GLOBAL float* __restrict__ verts, u
 // face_submerged and face_allwet, so the same bits: three arrays of float4
 // after one another,
 //   recs[f]          unit normal, area (negative: a degenerate face, which adds
-//                    volume only)
+//                    volume only; not a number where |n|^2 overflows, which the
+//                    sums then show as they would from the vertices)
 //   recs[nf + f]     centroid p1 + (e1 + e2) / 3, rounded once, and the three
 //                    10-bit remainders of the exact centroid (p1 + p2 + p3) / 3
 //                    in units of lo_unit, 1e-10 of the mesh's size: the
@@ -1011,7 +1012,7 @@ __device__ __forceinline__ void sub_chunk(uint32_t c, uint32_t f0, uint32_t nfc,
             const uint32_t fn = min(64u * (j + 1) + lane, flast);
             const f32x4 an = load_at(r0, fn), bn = load_at(r1, fn);
             const FaceRec r = make_rec(a, b);
-            if (64u * j + lane < nfc && r.A >= 0.f) {
+            if (64u * j + lane < nfc && !(r.A < 0.f)) {
                 f3 uf = mk3(0.f, 0.f, 0.f);
                 if (NU) {
                     double x[3];
@@ -1271,7 +1272,7 @@ __device__ __forceinline__ void cross_chunk(uint32_t c, uint32_t f0, uint32_t nf
                     const FaceRec r = make_rec(a, b);
                     if (__builtin_amdgcn_inverse_ballot_w64(row_mask(j))) {
                         acc.V6 += record_volume(fb, r.c, r.n1, r.A);
-                        if (r.A >= 0.f) {
+                        if (!(r.A < 0.f)) {
                             typename WaveQ<NL>::Pending q;
                             double x[3];
                             rec_centroid(r.c, r.lo, lo_unit, x);
@@ -1968,7 +1969,7 @@ __device__ __forceinline__ void step_sums(const StepShared<K, NU, AERO>& sh, con
                     const StepFace q = sf.points(f);
                     face_allwet<float, true>(fb, q.p1, q.p2, q.p3, acc);
                 }
-                if (A >= 0.f) {
+                if (!(A < 0.f)) {
                     if (PART < 2) {
                         const f3 uf = NU ? mk3(sh.uf[0][f], sh.uf[NU ? 1 : 0][f], sh.uf[NU ? 2 : 0][f]) : none;
                         if (AERO) aero_drag<NU>(fb, c, n1, A, uf, acc);

@@ -1,0 +1,47 @@
+"""A face too large for FP32 arithmetic (|n|^2 overflows) has an area that is not
+a number, and so has its body's skin friction (and, crossing, its wetted area),
+on every path to a whole face: the face is never left out of a finite row.
+Submerged and crossing bodies, the one-launch step, the face launch with records
+and, past 4,608 chunks on waves, its two passes over a crossing chunk."""
+import numpy as np
+import pytest
+
+from stonefish_amd import hydro as H
+from stonefish_amd import meshes as M
+from stonefish_amd import waves as W
+
+pytestmark = pytest.mark.gpu
+
+
+def _mesh():
+    box = M.box(0.3, 0.2, 0.1, 2)
+    far = np.array([[0, 0, 1e12], [1e12, 0, 1e12], [0, 1e12, 1e12]], np.float32)
+    n = len(box.verts)
+    return H.Mesh(M.TriMesh(np.concatenate([box.verts, far]),
+                            np.concatenate([box.faces, np.array([[n, n + 1, n + 2]], np.uint32)])))
+
+
+def _states(n, z):
+    st = np.zeros((n, 22))
+    st[:, [0, 5, 10, 15]] = 1.0
+    st[:, 12] = st[:, 13] = 10.0
+    st[:, 14] = z
+    st[:, 16:] = 0.3
+    return st
+
+
+@pytest.mark.parametrize("bodies,waves,split", [(3, False, 0), (3, False, 1), (3, True, 0), (3, True, 1), (4700, True, 0)])
+def test_overflowing_face_is_not_left_out(gpu, bodies, waves, split):
+    print(f"case: overflowing face, {bodies} bodies, waves {waves}, split_passes {split}", flush=True)
+    mesh, ocn = _mesh(), H.Ocean()
+    if waves:
+        ocn.set_waves(W.grid_reference(W.pm_components(8, 3.0, 64.0, seed=3), 64), 64, 1, [64.0])
+    ext = np.array([0.3, 0.2, 0.1])
+    desc = H.BodyDesc(mesh=mesh, aabb_min=-ext, aabb_max=ext, volume=0.05, surface=0.9)
+    batch = H.BodyBatch([desc] * bodies, faces_per_lane=16, split_passes=split)
+    for z, pos in ((4.0, 1.0), (0.0, 2.0)):
+        got = batch.compute_host(ocn, _states(bodies, z))
+        assert (got[:, 21] == pos).all()
+        assert np.isnan(got[:, 12:18]).all()
+        if pos == 2.0:
+            assert np.isnan(got[:, 18]).all()
