@@ -860,13 +860,13 @@ __device__ __forceinline__ f3 vert(const SFH_GLOBAL float* __restrict__ verts, u
 //   recs[f]          unit normal, area (negative: a degenerate face, which adds
 //                    volume only; not a number where |n|^2 overflows, which the
 //                    sums then show as they would from the vertices)
-//   recs[nf + f]     centroid p1 + (e1 + e2) / 3, rounded once, and the three
-//                    10-bit remainders of the exact centroid (p1 + p2 + p3) / 3
-//                    in units of lo_unit, 1e-10 of the mesh's size: the
-//                    submerged loop's
+//   recs[nf + f]     centroid p1 + (e1 + e2) / 3, rounded once: the submerged
+//                    loop's in a uniform flow (a varying one is sampled at the
+//                    centroid of the vertices in FP64)
 //   recs[2 nf + f]   the same with (e1 + e2) / 3 rounded before it is added, and
-//                    the remainders of that sum: the loop's of a crossing body
-//                    on waves
+//                    the three 10-bit remainders of that sum in units of
+//                    lo_unit, 1e-10 of the mesh's size: the loop's of a
+//                    crossing body on waves
 // A face so costs two coalesced 16-byte loads instead of three indices and
 // nine dependent gathers, and none of the edges, cross product and square root.
 struct FaceRec {
@@ -953,11 +953,8 @@ __global__ __launch_bounds__(256) void k_face_records(const float* __restrict__ 
     recs[f] = make_float4(n1.x, n1.y, n1.z, A);
     const f3 s = e1 + e2, off = s * (1.0f / 3.0f);
     const f3 c = step_centroid<true>(p1, s, 1.0f / 3.0f), d = step_centroid<false>(p1, s, 1.0f / 3.0f);
-    const double xc[3] = {((double)p1.x + (double)p2.x + (double)p3.x) / 3.0,
-                          ((double)p1.y + (double)p2.y + (double)p3.y) / 3.0,
-                          ((double)p1.z + (double)p2.z + (double)p3.z) / 3.0};
     const double xd[3] = {(double)p1.x + (double)off.x, (double)p1.y + (double)off.y, (double)p1.z + (double)off.z};
-    recs[(size_t)nf + f] = make_float4(c.x, c.y, c.z, pack_remainders(xc, c, unit));
+    recs[(size_t)nf + f] = make_float4(c.x, c.y, c.z, 0.f);
     recs[2 * (size_t)nf + f] = make_float4(d.x, d.y, d.z, pack_remainders(xd, d, unit));
 }
 
@@ -1001,7 +998,29 @@ __device__ __forceinline__ void sub_chunk(uint32_t c, uint32_t f0, uint32_t nfc,
     // stays in bounds; their results are not used.
     const uint32_t flast = nfc - 1;
     const int rows = (int)((nfc + 63u) / 64u);
-    if (REC) {
+    if (NU) {
+        // a varying flow is sampled at the centroid the vertices give in FP64
+        // (face_submerged); the vertices of face j+1 are in flight while face j
+        // is computed
+        const SFH_GLOBAL float* __restrict__ verts = gptr(S.verts);
+        const SFH_GLOBAL uint32_t* __restrict__ faces = gptr(S.faces) + 3 * (size_t)f0;
+        auto points = [&](uint32_t f, f3& p1, f3& p2, f3& p3) {
+            p1 = vert(verts, faces[3 * f]);
+            p2 = vert(verts, faces[3 * f + 1]);
+            p3 = vert(verts, faces[3 * f + 2]);
+        };
+        f3 p1, p2, p3;
+        points(min((uint32_t)lane, flast), p1, p2, p3);
+        for (int j = 0; j < rows; ++j) {
+            f3 q1, q2, q3;
+            points(min(64u * (j + 1) + lane, flast), q1, q2, q3);
+            if (64u * j + lane < nfc) {
+                if (AERO) face_aero(fb, p1, p2, p3, flow, acc);
+                else face_submerged(fb, p1, p2, p3, flow, acc);
+            }
+            p1 = q1; p2 = q2; p3 = q3;
+        }
+    } else if (REC) {
         // the records of face j+1 are in flight while face j is computed
         const SFH_GLOBAL f32x4* __restrict__ r0 = (const SFH_GLOBAL f32x4*)S.recs + f0;
         const SFH_GLOBAL f32x4* __restrict__ r1 = r0 + S.nf;
@@ -1013,14 +1032,8 @@ __device__ __forceinline__ void sub_chunk(uint32_t c, uint32_t f0, uint32_t nfc,
             const f32x4 an = load_at(r0, fn), bn = load_at(r1, fn);
             const FaceRec r = make_rec(a, b);
             if (64u * j + lane < nfc && !(r.A < 0.f)) {
-                f3 uf = mk3(0.f, 0.f, 0.f);
-                if (NU) {
-                    double x[3];
-                    rec_centroid(r.c, r.lo, S.lo_unit, x);
-                    uf = flow(x[0], x[1], x[2]);
-                }
-                if (AERO) aero_drag<NU>(fb, r.c, r.n1, r.A, uf, acc);
-                else face_drag<NU>(fb, r.c, r.n1, r.A, uf, acc);
+                if (AERO) aero_drag<false>(fb, r.c, r.n1, r.A, mk3(0.f, 0.f, 0.f), acc);
+                else face_drag(fb, r.c, r.n1, r.A, acc);
             }
             a = an; b = bn;
         }
@@ -1040,14 +1053,8 @@ __device__ __forceinline__ void sub_chunk(uint32_t c, uint32_t f0, uint32_t nfc,
             const f3 q1 = vert_at(vb, unpack_id(w, 0)), q2 = vert_at(vb, unpack_id(w, 1)), q3 = vert_at(vb, unpack_id(w, 2));
             w = load_at(pidx, min(64u * (j + 2) + lane, flast));
             if (64u * j + lane < nfc) {
-                if (AERO) {
-                    if (NU) face_aero(fb, p1, p2, p3, flow, acc);
-                    else face_aero(fb, p1, p2, p3, NoFlow(), acc);
-                } else if (NU) {
-                    face_submerged(fb, p1, p2, p3, flow, acc);
-                } else {
-                    face_submerged(fb, p1, p2, p3, acc);
-                }
+                if (AERO) face_aero(fb, p1, p2, p3, NoFlow(), acc);
+                else face_submerged(fb, p1, p2, p3, acc);
             }
             p1 = q1; p2 = q2; p3 = q3;
         }
@@ -2178,10 +2185,10 @@ __device__ __forceinline__ void step_chunk(StepShared<K, NU, AERO>& sh, const Ch
         }
     } else if (NU) {
         for (uint32_t f = t; f < nfc; f += 256) {
-            const float4 b = sh.r1[f];
-            double x[3];
-            rec_centroid(mk3(b.x, b.y, b.z), __float_as_int(b.w), S.lo_unit, x);
-            const f3 u = flow(x[0], x[1], x[2]);
+            const StepFace q = sf.points(f);
+            const f3 u = flow(((double)q.p1.x + (double)q.p2.x + (double)q.p3.x) / 3.0,
+                              ((double)q.p1.y + (double)q.p2.y + (double)q.p3.y) / 3.0,
+                              ((double)q.p1.z + (double)q.p2.z + (double)q.p3.z) / 3.0);
             sh.uf[0][f] = u.x; sh.uf[NU ? 1 : 0][f] = u.y; sh.uf[NU ? 2 : 0][f] = u.z;
         }
         __syncthreads();
@@ -3295,7 +3302,7 @@ static int launch_faces(sfh_batch_t* b, const OceanK& oc, hipStream_t s)
         if (sp && b->nchunks > kSplitChunks) {                                                                  \
             if (b->recs) LAUNCH_R(KK, NU, NL, PASS, true, sp); else LAUNCH_R(KK, NU, NL, PASS, false, sp);      \
         } else {                                                                                                \
-            if (b->recs) LAUNCH_R(KK, NU, NL, PASS, true, false); else LAUNCH_R(KK, NU, NL, PASS, false, false); \
+            if (b->recs) LAUNCH_R(KK, NU, NL, PASS, true, false); else LAUNCH_R(KK, NU, NL, PASS, NU, false);    \
         }                                                                                                       \
     }
 #define LAUNCH_X(KK, NU, NL)                                                                                    \
