@@ -371,15 +371,4 @@ SFH_HD Wet face_allwet(const FaceBody& B, f3 p1, f3 p2, f3 p3, Acc<T>& acc)
     return r;
 }
 
-// 6V of an all-wet face's tetra (tetra_term) from its record: the centroid lies
-// in the face's plane, so with |n| = 2 |A| it is (c - o).n1 2|A|.  Multiply-adds
-// are spelled out, so that every kernel rounds it the same way.  A is negative
-// for a degenerate face, whose volume still counts.
-SFH_HD float record_volume(const FaceBody& B, f3 c, f3 n1, float A)
-{
-    const f3 g = c - B.o;
-    const float h = __builtin_fmaf(g.z, n1.z, __builtin_fmaf(g.y, n1.y, g.x * n1.x)), a = fabsf(A);
-    return h * (a + a);
-}
-
 }  // namespace sfh

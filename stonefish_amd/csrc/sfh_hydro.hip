@@ -25,7 +25,6 @@
 
 #include <algorithm>
 #include <atomic>
-#include <cfloat>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -105,9 +104,9 @@ struct BodyStatic {
     const float* verts;
     const uint32_t* faces;
     const float4* recs;     // the mesh's face records (FaceRec)
+    const float4* xrecs;    // the batch's records of its crossing faces (k_cross_records), or null
     const uint32_t* pidx;   // its packed vertex numbers (PackedFaces)
     const uint2* blkwin;    // per block of 64 faces: lowest and highest vertex id
-    double lo_unit;         // unit of the records' centroid remainders
     uint32_t nf;
     uint32_t flags;
     uint32_t chunk0;
@@ -853,26 +852,20 @@ __device__ __forceinline__ f3 vert(const SFH_GLOBAL float* __restrict__ verts, u
     return mk3(v[0], v[1], v[2]);
 }
 
-// A mesh's face records: what the integrand needs of a whole face and no
+// A mesh's face records: what the submerged loop needs of a whole face and no
 // state changes, formed once per mesh (k_face_records) with the operations of
-// face_submerged and face_allwet, so the same bits: three arrays of float4
-// after one another,
+// face_submerged, so the same bits: two arrays of float4 after one another,
 //   recs[f]          unit normal, area (negative: a degenerate face, which adds
-//                    volume only; not a number where |n|^2 overflows, which the
+//                    nothing; not a number where |n|^2 overflows, which the
 //                    sums then show as they would from the vertices)
-//   recs[nf + f]     centroid p1 + (e1 + e2) / 3, rounded once: the submerged
-//                    loop's in a uniform flow (a varying one is sampled at the
-//                    centroid of the vertices in FP64)
-//   recs[2 nf + f]   the same with (e1 + e2) / 3 rounded before it is added, and
-//                    the three 10-bit remainders of that sum in units of
-//                    lo_unit, 1e-10 of the mesh's size: the loop's of a
-//                    crossing body on waves
+//   recs[nf + f]     centroid p1 + (e1 + e2) / 3, rounded once, for a uniform
+//                    flow (a varying one is sampled at the centroid of the
+//                    vertices in FP64)
 // A face so costs two coalesced 16-byte loads instead of three indices and
 // nine dependent gathers, and none of the edges, cross product and square root.
 struct FaceRec {
     f3 n1, c;
     float A;
-    int lo;
 };
 
 // PackedFaces: a face's three vertex numbers in one word, 10 bits each, less
@@ -890,15 +883,7 @@ __device__ __forceinline__ FaceRec make_rec(f32x4 a, f32x4 b)
     r.n1 = mk3(a.x, a.y, a.z);
     r.A = a.w;
     r.c = mk3(b.x, b.y, b.z);
-    r.lo = __float_as_int(b.w);
     return r;
-}
-
-__device__ __forceinline__ void rec_centroid(f3 c, int lo, double unit, double (&x)[3])
-{
-    x[0] = __builtin_fma((double)((lo << 22) >> 22), unit, (double)c.x);
-    x[1] = __builtin_fma((double)((lo << 12) >> 22), unit, (double)c.y);
-    x[2] = __builtin_fma((double)((lo << 2) >> 22), unit, (double)c.z);
 }
 
 // A wet polygon's centroid, rounded once (fused) or after the offset.
@@ -912,20 +897,9 @@ __device__ __forceinline__ f3 step_centroid(f3 base, f3 cs, float ck)
     return mk3(base.x + x, base.y + y, base.z + z);
 }
 
-__device__ __forceinline__ float pack_remainders(const double (&x)[3], f3 c, double unit)
-{
-    const double d[3] = {x[0] - (double)c.x, x[1] - (double)c.y, x[2] - (double)c.z};
-    uint32_t lo = 0;
-    for (int k = 0; k < 3; ++k) {
-        const double r = unit > 0.0 ? rint(d[k] / unit) : 0.0;
-        lo |= ((uint32_t)(int)fmin(fmax(r, -512.0), 511.0) & 1023u) << (10 * k);
-    }
-    return __uint_as_float(lo);
-}
-
 __global__ __launch_bounds__(256) void k_face_records(const float* __restrict__ verts,
                                                       const uint32_t* __restrict__ faces,
-                                                      const uint2* __restrict__ blkwin, uint32_t nf, double unit,
+                                                      const uint2* __restrict__ blkwin, uint32_t nf,
                                                       float4* __restrict__ recs, uint32_t* __restrict__ pidx)
 {
     const uint32_t f = blockIdx.x * 256u + threadIdx.x;
@@ -939,23 +913,42 @@ __global__ __launch_bounds__(256) void k_face_records(const float* __restrict__ 
     const f3 n = cross(e1, e2);
     const float n2 = dot(n, n);
     const float inv = frsq(n2);
-    f3 n1 = n * inv;
-    float A = 0.5f * (n2 * inv);
-    if (n2 < SFH_DEGENERATE_N2) {
-        // v_rsq_f32 takes no subnormal number (it returns infinity); the volume
-        // of a face of |n| < 1.1e-19 is below the rounding of any body's
-        if (n2 < FLT_MIN) {
-            n1 = mk3(0.f, 0.f, 0.f);
-            A = 0.f;
-        }
-        A = -fmaxf(A, FLT_MIN);
-    }
-    recs[f] = make_float4(n1.x, n1.y, n1.z, A);
-    const f3 s = e1 + e2, off = s * (1.0f / 3.0f);
-    const f3 c = step_centroid<true>(p1, s, 1.0f / 3.0f), d = step_centroid<false>(p1, s, 1.0f / 3.0f);
-    const double xd[3] = {(double)p1.x + (double)off.x, (double)p1.y + (double)off.y, (double)p1.z + (double)off.z};
+    const f3 n1 = n * inv, c = step_centroid<true>(p1, e1 + e2, 1.0f / 3.0f);
+    const bool thin = n2 < SFH_DEGENERATE_N2;
+    recs[f] = thin ? make_float4(0.f, 0.f, 0.f, -1.f) : make_float4(n1.x, n1.y, n1.z, 0.5f * (n2 * inv));
     recs[(size_t)nf + f] = make_float4(c.x, c.y, c.z, 0.f);
-    recs[2 * (size_t)nf + f] = make_float4(d.x, d.y, d.z, pack_remainders(xd, d, unit));
+}
+
+// The records of a mesh's faces for the loop of a crossing body on waves, formed
+// with the operations of face_allwet: per face
+//   x[f]             normal vector e1 x e2, one over its length
+//   x[nf + f]        first vertex, area (negative: a degenerate face, which adds
+//                    its volume only)
+//   and after those  (e1 + e2) / 3, 12 bytes
+// The parts whose sums are the volume's term and the centroid, not the results:
+// a centroid rounded to FP32 and a volume from the unit normal, 16 bytes less,
+// moved the depth's point by 2e-8 of the mesh and the volume by 7e-9.
+static constexpr size_t kCrossRecBytes = 44;
+
+__global__ __launch_bounds__(256) void k_cross_records(const float* __restrict__ verts,
+                                                       const uint32_t* __restrict__ faces, uint32_t nf,
+                                                       float4* __restrict__ x)
+{
+    const uint32_t f = blockIdx.x * 256u + threadIdx.x;
+    if (f >= nf) return;
+    const SFH_GLOBAL float* vs = gptr(verts);
+    const f3 p1 = vert(vs, faces[3 * (size_t)f]), p2 = vert(vs, faces[3 * (size_t)f + 1]),
+             p3 = vert(vs, faces[3 * (size_t)f + 2]);
+    const f3 e1 = p2 - p1, e2 = p3 - p1;
+    const f3 n = cross(e1, e2), off = (e1 + e2) * (1.0f / 3.0f);
+    const float n2 = dot(n, n);
+    const float inv = frsq(n2);
+    x[f] = make_float4(n.x, n.y, n.z, inv);
+    x[(size_t)nf + f] = make_float4(p1.x, p1.y, p1.z, n2 < SFH_DEGENERATE_N2 ? -1.f : 0.5f * (n2 * inv));
+    float* o = (float*)(x + 2 * (size_t)nf) + 3 * (size_t)f;
+    o[0] = off.x;
+    o[1] = off.y;
+    o[2] = off.z;
 }
 
 // Transposed FP64 reduction of 12 per-lane values: on return v[0] of lane l
@@ -1137,9 +1130,6 @@ __device__ __forceinline__ void cross_chunk(uint32_t c, uint32_t f0, uint32_t nf
     const SFH_GLOBAL float* __restrict__ verts = gptr(S.verts);
     const SFH_GLOBAL uint32_t* __restrict__ faces = gptr(S.faces) + 3 * (size_t)f0;
     const SFH_GLOBAL uint32_t* __restrict__ pidx = gptr(S.pidx) + f0;
-    const SFH_GLOBAL f32x4* __restrict__ r0 = (const SFH_GLOBAL f32x4*)S.recs + f0;
-    const SFH_GLOBAL f32x4* __restrict__ r2 = r0 + 2 * (size_t)S.nf;
-    const double lo_unit = S.lo_unit;
     const FaceBody fb = D.fb;
     const uint32_t flags = D.flags;
     const bool damping = flags & BF_DAMPING;
@@ -1271,33 +1261,32 @@ __device__ __forceinline__ void cross_chunk(uint32_t c, uint32_t f0, uint32_t nf
             };
             int left = __builtin_popcount(wet_rows), j = next(0), jn = next(j);
             if (REC) {
+                const SFH_GLOBAL f32x4* __restrict__ x0 = (const SFH_GLOBAL f32x4*)S.xrecs;
+                const SFH_GLOBAL float* __restrict__ x2 = (const SFH_GLOBAL float*)(x0 + 2 * (size_t)S.nf) + 3 * (size_t)f0;
+                x0 += f0;
+                const SFH_GLOBAL f32x4* __restrict__ x1 = x0 + S.nf;
                 const uint32_t fc = min(64u * j + lane, flast);
-                f32x4 a = load_at(r0, fc), b = load_at(r2, fc);
+                f32x4 a = load_at(x0, fc), b = load_at(x1, fc);
+                f3 off = vert_at(x2, fc);
                 for (;;) {
                     const uint32_t fn = min(64u * jn + lane, flast);
-                    const f32x4 an = load_at(r0, fn), bn = load_at(r2, fn);   // in flight while row j is computed
-                    const FaceRec r = make_rec(a, b);
+                    const f32x4 an = load_at(x0, fn), bn = load_at(x1, fn);   // in flight while row j is computed
+                    const f3 offn = vert_at(x2, fn);
                     if (__builtin_amdgcn_inverse_ballot_w64(row_mask(j))) {
-                        acc.V6 += record_volume(fb, r.c, r.n1, r.A);
-                        if (!(r.A < 0.f)) {
-                            typename WaveQ<NL>::Pending q;
-                            double x[3];
-                            rec_centroid(r.c, r.lo, lo_unit, x);
-                            if (wave_buoy) q = wq.issue(x[0], x[1], x[2]);
-                            if (damping) face_drag(fb, r.c, r.n1, r.A, acc);
-                            if (wave_buoy) {
-                                const float dc = (float)wq.finish(q);
-                                f3 fbi = r.n1 * (-r.A * dc);
-                                add3(acc.Fb, fbi);
-                                add3(acc.Mb, cross(r.c, fbi));
-                            }
-                            acc.Swet += r.A;
-                        }
+                        const f3 n = mk3(a.x, a.y, a.z);
+                        Wet wt;
+                        wt.base = mk3(b.x, b.y, b.z);
+                        wt.off = off;
+                        wt.n1 = n * a.w;
+                        wt.A = b.w;
+                        wt.ok = !(b.w < 0.f);
+                        tetra_term0<float, false>(wt.base - fb.o, n, off, acc);
+                        wet_contrib<NU, NL>(wt, fb, D, wq, wave_buoy, damping, acc);
                     }
                     if (--left == 0) break;
                     j = jn;
                     jn = next(jn);
-                    a = an; b = bn;
+                    a = an; b = bn; off = offn;
                 }
             } else {
                 // row j is computed, row jn's vertices and the row after's numbers
@@ -2442,7 +2431,6 @@ struct sfh_mesh_t {
     uint2* d_blkwin = nullptr;          // per block of 64 faces: lowest and highest vertex id referenced
     uint32_t* d_pidx = nullptr;         // packed faces
     bool packed = true;                 // every block spans at most kPackSpan ids
-    double lo_unit = 0.0;               // of the face records
     std::vector<uint2> blkwin;          // the same on the host
     uint32_t nv = 0, nf = 0;
     float aabb_min[3], aabb_max[3];
@@ -2502,6 +2490,7 @@ struct sfh_batch_t {
     uint32_t* d_lists = nullptr;    // the step's work list [nchunks], then its two counts
     BodyDyn* d_dyn = nullptr;
     double* d_partials = nullptr;
+    float4* d_xrecs = nullptr;      // records of the meshes' crossing faces, for steps that read them
     uint32_t* d_done = nullptr;     // per body: chunks k_step finished in this step (zero between steps)
     bool all_faces = false;         // every body has at least one chunk
     bool recs = true;               // the face launch reads the meshes' face records, else their packed faces
@@ -2621,18 +2610,14 @@ extern "C" int sfh_mesh_create(const void* vertex_pos, size_t vertex_stride, uin
     for (int k = 0; k < 3; ++k) { m->aabb_min[k] = mn[k]; m->aabb_max[k] = mx[k]; }
     if (nf) memcpy((char*)image.data() + at_blk, m->blkwin.data(), sizeof(uint2) * nblk);
     if (nv) {
-        float size = 0.f;
-        for (int k = 0; k < 3; ++k) size = fmaxf(size, fmaxf(fabsf(mn[k]), fabsf(mx[k])));
-        // centroids lie below 2^(e + 1): their rounding is at most 2^(e - 24), 512 units
-        if (size > 0.f && std::isfinite(size)) m->lo_unit = ldexp(1.0, std::max(ilogbf(size) - 33, -1000));
-        const size_t recs = align16(52 * (size_t)nf), bytes = image.size() * 8;
+        const size_t recs = align16(36 * (size_t)nf), bytes = image.size() * 8;
         hipError_t e = hipMalloc(&m->d_mem, recs + bytes);
         if (e == hipSuccess) {
             char* at = (char*)m->d_mem + recs;
             m->d_verts = (float*)at;
             if (nf) {
                 m->d_recs = (float4*)m->d_mem;
-                m->d_pidx = (uint32_t*)(m->d_recs + 3 * (size_t)nf);
+                m->d_pidx = (uint32_t*)(m->d_recs + 2 * (size_t)nf);
                 m->d_faces = (uint32_t*)(at + at_faces);
                 m->d_blkwin = (uint2*)(at + at_blk);
             }
@@ -2640,7 +2625,7 @@ extern "C" int sfh_mesh_create(const void* vertex_pos, size_t vertex_stride, uin
         }
         if (e == hipSuccess && nf) {
             hipLaunchKernelGGL(k_face_records, dim3((nf + 255) / 256), dim3(256), 0, nullptr, m->d_verts, m->d_faces,
-                               m->d_blkwin, nf, m->lo_unit, m->d_recs, m->d_pidx);
+                               m->d_blkwin, nf, m->d_recs, m->d_pidx);
             e = hipGetLastError();
             if (e == hipSuccess) e = hipStreamSynchronize(nullptr);   // batches read the records on other streams
         }
@@ -2812,6 +2797,7 @@ static void batch_free(sfh_batch_t* b)
     hipFree(b->d_dyn);
     hipFree(b->d_partials);
     hipFree(b->d_done);
+    hipFree(b->d_xrecs);
     hipFree(b->d_comp);
     hipFree(b->d_part_out);
     hipFree(b->d_units);
@@ -2854,16 +2840,29 @@ static void chunk_window(const std::vector<uint2>& blk, uint32_t first, uint32_t
 
 // Up to this many faces in the distinct meshes of a batch its face launch reads
 // their records, past it their packed faces and vertices.  The records take 32
-// bytes a face and the least arithmetic; the packed faces take 10 (with their
-// share of the vertices), and the normals, areas and centroids are formed on
-// the way.  While the records stay in the caches the face launch is bound by
-// its arithmetic, then by memory.  Fleets of bodies with a mesh of their own
-// on waves, three states in turn, records / packed (a step, us):
-//     1.4 M faces   38.6 / 40.1        7.4 M   74.9 / 62.0
-//     2.5 M         46.7 / 42.8       14.2 M  119.3 / 98.9
-// and 6,000 compounds sharing two meshes (12,288 faces) 259 / 293.  A batch with
+// bytes a face (44 in the crossing loop) and the least arithmetic; the packed
+// faces take 10 (with their share of the vertices), and the normals, areas and
+// centroids are formed on the way.  While the records stay in the caches the
+// face launch is bound by its arithmetic, then by memory.  Fleets of bodies with
+// a mesh of their own on waves, three states in turn, records / packed (a step,
+// us):
+//     1.4 M faces   34.6 / 34.6        7.6 M   86.4 / 61.4
+//     2.4 M         38.6 / 38.1       14.2 M  138.6 / 95.6
+// and 6,000 compounds sharing two meshes (12,288 faces) 256 / 292.  A batch with
 // a mesh that cannot be packed (faces in no order) reads records.
 static constexpr uint64_t kRecordFaces = 2000000;
+
+// On waves the face launch of batches of more chunks than this takes a crossing
+// chunk's rows twice (cross_chunk's SPLIT): fewer instructions, but a longer
+// chain of waits per chunk, which shows while most wavefronts are alone on
+// their SIMD.  Measured, one pass / two (a step on one wave layer, us): fleets
+// of 1,464 chunks 36.6 / 39.9, 4,381 46.6 / 47.7, 7,520 67.8 / 61.1, 14,436
+// 105.3 / 97.4; one hull, 5,000 chunks 52.5 / 50.9, 20,480 136.0 / 126.6;
+// compounds, 2,400 chunks 48.5 / 48.8, 72,000 303.7 / 269.0.  From 8 faces per
+// lane on: with fewer a chunk is its fixed work more than its rows.
+static constexpr uint32_t kSplitChunks = 4608;
+
+static bool two_pass(const sfh_batch_t* b) { return b->K >= 8 && b->nchunks > kSplitChunks; }
 
 // (Re)builds the chunks: every body's faces cut into chunks of 64*K
 // consecutive faces, each with its vertex window.
@@ -2896,6 +2895,8 @@ static int batch_build_chunks(sfh_batch_t* b)
     hipFree(b->d_bpos);
     hipFree(b->d_lists);
     hipFree(b->d_done);
+    hipFree(b->d_xrecs);
+    b->d_xrecs = nullptr;
     b->d_static = nullptr; b->d_sidx = nullptr; b->d_chunks = nullptr;
     b->d_partials = nullptr; b->d_bpos = nullptr; b->d_lists = nullptr; b->d_done = nullptr;
     b->nchunks = (uint32_t)chunks.size();
@@ -2911,6 +2912,24 @@ static int batch_build_chunks(sfh_batch_t* b)
         packed = packed && m->packed;
     }
     b->recs = !packed || faces <= kRecordFaces;
+    for (BodyStatic& s : b->h_static) s.xrecs = nullptr;
+    if (b->recs && two_pass(b)) {
+        HIPCHK(hipMalloc(&b->d_xrecs, kCrossRecBytes * (faces + 4 * used.size())));
+        std::vector<float4*> at(used.size());
+        size_t next = 0;   // in float4: each mesh's block starts at a multiple of 16 bytes
+        for (size_t i = 0; i < used.size(); ++i) {
+            const sfh_mesh_t* m = used[i];
+            at[i] = b->d_xrecs + next;
+            next += (kCrossRecBytes * m->nf + 15) / 16;
+            if (m->nf)
+                hipLaunchKernelGGL(k_cross_records, dim3((m->nf + 255) / 256), dim3(256), 0, nullptr, m->d_verts,
+                                   m->d_faces, m->nf, at[i]);
+        }
+        HIPCHK(hipGetLastError());
+        for (uint32_t i = 0; i < b->n; ++i)
+            if (const sfh_mesh_t* m = i < b->meshes_by_body.size() ? b->meshes_by_body[i] : nullptr)
+                b->h_static[i].xrecs = at[std::lower_bound(used.begin(), used.end(), m) - used.begin()];
+    }
     HIPCHK(hipMalloc(&b->d_static, sizeof(BodyStatic) * std::max<size_t>(1, b->n)));
     HIPCHK(hipMemcpy(b->d_static, b->h_static.data(), sizeof(BodyStatic) * b->n, hipMemcpyHostToDevice));
     {
@@ -2928,7 +2947,7 @@ static int batch_build_chunks(sfh_batch_t* b)
     HIPCHK(hipMemset(b->d_lists + b->nchunks, 0, 2 * sizeof(uint32_t)));
     HIPCHK(hipMalloc(&b->d_done, sizeof(uint32_t) * std::max<size_t>(1, b->n)));
     HIPCHK(hipMemset(b->d_done, 0, sizeof(uint32_t) * std::max<size_t>(1, b->n)));
-    HIPCHK(hipStreamSynchronize(nullptr));   // the counters are clear before a step on any stream
+    HIPCHK(hipStreamSynchronize(nullptr));   // the records are written and the counters clear before a step on any stream
     if (b->graph_exec) { hipGraphExecDestroy(b->graph_exec); b->graph_exec = nullptr; }
     if (b->graph) { hipGraphDestroy(b->graph); b->graph = nullptr; }
     return SFH_OK;
@@ -2958,7 +2977,6 @@ static BodyStatic make_static(const sfh_mesh_t* m, uint32_t flags)
     s.recs = m ? m->d_recs : nullptr;
     s.pidx = m ? m->d_pidx : nullptr;
     s.blkwin = m ? m->d_blkwin : nullptr;
-    s.lo_unit = m ? m->lo_unit : 0.0;
     s.nf = m ? m->nf : 0;
     s.nv = m ? m->nv : 0;
     s.flags = flags;
@@ -3276,16 +3294,6 @@ extern "C" int sfh_batch_info(sfh_batch b, uint32_t* nbodies, uint32_t* nchunks,
     return SFH_OK;
 }
 
-// On waves the face launch of batches of more chunks than this takes a crossing
-// chunk's rows twice (cross_chunk's SPLIT): fewer instructions, but a longer
-// chain of waits per chunk, which shows while most wavefronts are alone on
-// their SIMD.  Measured, one pass / two (a step on one wave layer, us): fleets
-// of 1,464 chunks 36.6 / 39.9, 4,381 46.6 / 47.7, 7,520 67.8 / 61.1, 14,436
-// 105.3 / 97.4; one hull, 5,000 chunks 52.5 / 50.9, 20,480 136.0 / 126.6;
-// compounds, 2,400 chunks 48.5 / 48.8, 72,000 303.7 / 269.0.  From 8 faces per
-// lane on: with fewer a chunk is its fixed work more than its rows.
-static constexpr uint32_t kSplitChunks = 4608;
-
 // Launches the face pass over every chunk of the batch.
 static int launch_faces(sfh_batch_t* b, const OceanK& oc, hipStream_t s)
 {
@@ -3299,7 +3307,7 @@ static int launch_faces(sfh_batch_t* b, const OceanK& oc, hipStream_t s)
 #define LAUNCH_F(KK, NU, NL, PASS)                                                                              \
     {                                                                                                           \
         constexpr bool sp = NL > 0 && !NU && (PASS & kPassCross) && KK >= 8;                                    \
-        if (sp && b->nchunks > kSplitChunks) {                                                                  \
+        if (sp && two_pass(b)) {                                                                                \
             if (b->recs) LAUNCH_R(KK, NU, NL, PASS, true, sp); else LAUNCH_R(KK, NU, NL, PASS, false, sp);      \
         } else {                                                                                                \
             if (b->recs) LAUNCH_R(KK, NU, NL, PASS, true, false); else LAUNCH_R(KK, NU, NL, PASS, NU, false);    \
