@@ -164,9 +164,10 @@ int sfh_correct(sfh_ocean ocean, double Fdq[3], double Tdq[3], double Fdf[3], do
  * GPU (held until the process ends), sized for meshes of at most 524,288
  * faces; a larger mesh returns SFH_ERR_SIZE.  It calls
  * no hipMalloc, hipFree or allocating routine.  Every call on one GPU shares
- * that array (a chunk counter, zero between calls, and the chunks' partial
- * sums): calls that overlap on one GPU (several streams or threads)
- * race, so the caller orders them.  mesh must not be NULL. */
+ * that array (chunk counters, zero between calls, and the chunks' partial
+ * sums): the rows of calls that overlap on one GPU (several streams or
+ * threads) are undefined, so the caller orders them; calls after those have
+ * ended are not affected.  mesh must not be NULL. */
 int sfh_forces_noalloc(const sfh_settings* settings, int mode, sfh_mesh mesh, sfh_ocean ocean,
                        const double* d_state, double* d_out, void* stream);
 

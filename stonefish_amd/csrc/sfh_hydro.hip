@@ -1821,7 +1821,7 @@ __global__ __launch_bounds__(64 * kFaceWaves, face_occupancy(K, NU, PASS)) void 
 //      goes to memory past the caches (agent-scope stores, waited for), the
 //      workgroup counts itself done on the body's counter, and the one that
 //      counts last sums the partials in chunk order and finishes the row.
-//      It also zeroes the counter for the next step.
+//      The counter has wrapped to zero for the next step.
 // Measured: a tick of 203 bodies (576 chunks, 60 % overlapped, two wave
 // layers) 39.4 -> 17.9 us, an aerodynamic batch of 300 bodies 16.5 -> 9.4 us,
 // the per-body calls 38 -> 32 us (2,070 faces, submerged) and 52 -> 43 us
@@ -1838,7 +1838,7 @@ struct StepArgs {
     double* out;
     double* applied;           // the tick driver's force and torque per row, or null
     double* partials;
-    uint32_t* done;            // per body: chunks finished in this step
+    uint32_t* done;            // per body: chunks finished in this step (modulo the body's chunks)
     int kind;
 };
 
@@ -2211,11 +2211,13 @@ __device__ __forceinline__ void step_chunk(StepShared<K, NU, AERO>& sh, const Ch
         if (lane < kChunkDoubles)
             __hip_atomic_store(mine + lane, sh.P[lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        // the count wraps at the body's chunks: zero again after the last one,
+        // whatever order launches that overlap count in, so that rows of steps
+        // that were not ordered are undefined and later ones are not
         uint32_t n = 0;
-        if (lane == 0) n = __hip_atomic_fetch_add(a.done + ch.body, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (lane == 0) n = atomicInc(a.done + ch.body, S.nchunks - 1u);
         if ((uint32_t)uni((int)n) + 1u != S.nchunks) return;
         asm volatile("" ::: "memory");
-        if (lane == 0) __hip_atomic_store(a.done + ch.body, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         epilogue_sums<true>(S, a.partials, sh.P, lane);
         wave_lds_sync();
     }
@@ -3767,8 +3769,9 @@ extern "C" int sfh_batch_kernel_ms(sfh_batch b, double* face_ms, double* total_m
 // partials of a mesh of more than one chunk, in one device buffer sized for
 // meshes of up to F faces: a workspace of the per-body statics (device memory
 // from hipMalloc, grown on demand) or the no-alloc entry point's file-scope
-// array.  The counter is zero between calls (the workgroup that finishes the
-// row zeroes it).
+// array.  The counter is zero between calls (it wraps at the mesh's chunks); a
+// mesh of each number of chunks has its own, so that it stays so when calls of
+// several meshes overlap in the no-alloc array.
 static constexpr uint32_t kSingleK = 8;   // faces per lane of per-body calls
 
 // A per-body call's state passed by value (no copy command of its own).
@@ -3779,7 +3782,9 @@ struct StateArg {
 __host__ __device__ constexpr size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 __host__ __device__ constexpr uint32_t single_nchunks(uint32_t F) { return (F + 64u * kSingleK - 1) / (64u * kSingleK); }
 
-static constexpr size_t kSinglePartials = 256;   // byte offset of the partials; the counter is at 0
+static constexpr uint32_t kNaMaxFaces = 1u << 19;   // faces of the no-alloc entry point's meshes: 524,288
+static constexpr uint32_t kSingleCounters = single_nchunks(kNaMaxFaces) + 1;   // 0: larger meshes, in a workspace
+static constexpr size_t kSinglePartials = align256(sizeof(uint32_t) * kSingleCounters);   // byte offset of the partials
 
 __host__ __device__ constexpr size_t single_bytes(uint32_t F)
 {
@@ -3833,7 +3838,7 @@ static int single_launch(unsigned char* buf, const sfh_mesh_t* m, uint32_t flags
     memset(&a, 0, sizeof(a));
     a.states = d_state;
     a.out = d_out;
-    a.done = (uint32_t*)buf;
+    a.done = (uint32_t*)buf + (st.nchunks < kSingleCounters ? st.nchunks : 0u);
     a.partials = (double*)(buf + kSinglePartials);
     a.kind = 1;
     StateArg sa;
@@ -3929,8 +3934,8 @@ static int ws_reserve(Workspace* w, uint32_t F)
     w->d_buf = nullptr;
     w->cap = 0;
     HIPCHK(hipMalloc(&w->d_buf, cap));
-    // the counter starts at zero, cleared on the stream of the launches that
-    // count on it (no other stream orders a non-blocking one)
+    // the counters start at zero, cleared on the stream of the launches that
+    // count on them (no other stream orders a non-blocking one)
     const hipError_t e = hipMemsetAsync(w->d_buf, 0, kSinglePartials, w->stream);
     if (e != hipSuccess) {
         hipFree(w->d_buf);
@@ -4078,7 +4083,6 @@ extern "C" int sfh_correct(sfh_ocean ocean, double Fdq[3], double Tdq[3], double
 // up to kNaMaxFaces faces, in one file-scope device array.  Each GPU the library runs on holds its own copy until the process
 // ends; every call on a GPU shares it, so calls that overlap on one GPU (two
 // streams, or two host threads) race.
-static constexpr uint32_t kNaMaxFaces = 1u << 19;   // 524,288
 static constexpr size_t kNaBytes = single_bytes(kNaMaxFaces);
 static_assert(kNaBytes <= (256u << 10), "no-alloc scratch above 256 KiB");
 
