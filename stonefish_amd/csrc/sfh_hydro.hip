@@ -1746,16 +1746,19 @@ static constexpr int kFaceWaves = 1;
 // Wavefronts per SIMD the face kernels are built for: 8 for the submerged loop
 // alone; 5 with the crossing loop at 16 and 32 faces per lane, which large
 // batches use (4, without a spill: the 6,000 compounds 6 %, the fleet 5 %
-// slower); 3 at up to 8 faces per lane, for batches of few chunks, whose
-// wavefronts are mostly alone and wait for their own loads, which a spill's
-// wait drains (fleets of 120 and 240 bodies at 8 faces per lane 40.4 and 44.3
-// -> 35.3 and 39.3 us a step).
-constexpr int face_occupancy(int K, bool NU, int PASS)
+// slower), but 4 on two layers, whose second texel and its fractions do not fit
+// 5 (spills of 100 bytes: fleets of 220 and 1,280 bodies 52.7 and 163.7 -> 43.4
+// and 119.8 us a step, 300 and 6,000 compounds 56.4 and 423 -> 49.8 and 324);
+// 3 at up to 8 faces per lane, for batches of few chunks, whose wavefronts are
+// mostly alone and wait for their own loads, which a spill's wait drains (fleets
+// of 120 and 240 bodies at 8 faces per lane 40.4 and 44.3 -> 35.3 and 39.3 us a
+// step).
+constexpr int face_occupancy(int K, bool NU, int NL, int PASS)
 {
-    return NU ? 1 : (PASS & 2) ? (K <= 8 ? 3 : 5) : 8;
+    return NU ? 1 : (PASS & 2) ? (K <= 8 ? 3 : NL == 2 ? 4 : 5) : 8;
 }
 template <int K, bool NU, int NL, int PASS, bool REC, bool SPLIT>
-__global__ __launch_bounds__(64 * kFaceWaves, face_occupancy(K, NU, PASS)) void k_faces(
+__global__ __launch_bounds__(64 * kFaceWaves, face_occupancy(K, NU, NL, PASS)) void k_faces(
     const uint32_t* __restrict__ list, const uint32_t* __restrict__ counts, uint32_t nc,
     const Chunk* __restrict__ chunks, const BodyStatic* __restrict__ st, const BodyDyn* __restrict__ dyn, OceanK oc,
     double* __restrict__ partials)
