@@ -993,20 +993,18 @@ __device__ __forceinline__ void sub_chunk(uint32_t c, uint32_t f0, uint32_t nfc,
     const int rows = (int)((nfc + 63u) / 64u);
     if (NU) {
         // a varying flow is sampled at the centroid the vertices give in FP64
-        // (face_submerged); the vertices of face j+1 are in flight while face j
-        // is computed
+        // (face_submerged); the numbers of face j+2 and the vertices of face j+1
+        // are in flight while face j is computed
         const SFH_GLOBAL float* __restrict__ verts = gptr(S.verts);
         const SFH_GLOBAL uint32_t* __restrict__ faces = gptr(S.faces) + 3 * (size_t)f0;
-        auto points = [&](uint32_t f, f3& p1, f3& p2, f3& p3) {
-            p1 = vert(verts, faces[3 * f]);
-            p2 = vert(verts, faces[3 * f + 1]);
-            p3 = vert(verts, faces[3 * f + 2]);
-        };
-        f3 p1, p2, p3;
-        points(min((uint32_t)lane, flast), p1, p2, p3);
+        const uint32_t fc0 = min((uint32_t)lane, flast), fc1 = min(64u + lane, flast);
+        uint32_t b0 = faces[3 * fc1], b1 = faces[3 * fc1 + 1], b2 = faces[3 * fc1 + 2];
+        f3 p1 = vert(verts, faces[3 * fc0]), p2 = vert(verts, faces[3 * fc0 + 1]), p3 = vert(verts, faces[3 * fc0 + 2]);
+#pragma unroll 2
         for (int j = 0; j < rows; ++j) {
-            f3 q1, q2, q3;
-            points(min(64u * (j + 1) + lane, flast), q1, q2, q3);
+            const uint32_t fn = min(64u * (j + 2) + lane, flast);
+            const f3 q1 = vert(verts, b0), q2 = vert(verts, b1), q3 = vert(verts, b2);
+            b0 = faces[3 * fn]; b1 = faces[3 * fn + 1]; b2 = faces[3 * fn + 2];
             if (64u * j + lane < nfc) {
                 if (AERO) face_aero(fb, p1, p2, p3, flow, acc);
                 else face_submerged(fb, p1, p2, p3, flow, acc);
