@@ -1109,7 +1109,7 @@ __device__ __forceinline__ void wet_contrib(const Wet& wt, const FaceBody& fb, c
 // together afterwards, 64 at a time, so the clip code runs once per 64 of them.
 // Tetra volumes, pressure buoyancy with waves, drag.
 //
-// SPLIT (large batches on waves, kSplitChunks): the rows are taken twice, first
+// SPLIT (large batches on one wave layer, kSplitChunks): the rows are taken twice, first
 // which of their faces are all wet (a mask of the row, kept in lane `row` of a
 // register pair) and which are cut, from the packed vertex numbers and the
 // depths alone; then the all-wet faces of the rows that have any, from the face
@@ -2861,15 +2861,20 @@ static void chunk_window(const std::vector<uint2>& blk, uint32_t first, uint32_t
 // a mesh that cannot be packed (faces in no order) reads records.
 static constexpr uint64_t kRecordFaces = 2000000;
 
-// On waves the face launch of batches of more chunks than this takes a crossing
-// chunk's rows twice (cross_chunk's SPLIT): fewer instructions, but a longer
-// chain of waits per chunk, which shows while most wavefronts are alone on
-// their SIMD.  Measured, one pass / two (a step on one wave layer, us): fleets
-// of 1,464 chunks 36.6 / 39.9, 4,381 46.6 / 47.7, 7,520 67.8 / 61.1, 14,436
-// 105.3 / 97.4; one hull, 5,000 chunks 52.5 / 50.9, 20,480 136.0 / 126.6;
-// compounds, 2,400 chunks 48.5 / 48.8, 72,000 303.7 / 269.0.  From 8 faces per
-// lane on: with fewer a chunk is its fixed work more than its rows.
-static constexpr uint32_t kSplitChunks = 4608;
+// On one wave layer the face launch of batches of more chunks than this takes a
+// crossing chunk's rows twice (cross_chunk's SPLIT): fewer instructions, but a
+// longer chain of waits per chunk, which shows while the chip is not full of
+// them.  Measured, one pass / two (a step, us), bodies with a mesh of their own:
+//     4,698 chunks  45.5 / 48.6       9,108 chunks  70.0 / 71.0
+//     6,840         55.9 / 59.3      12,599         88.4 / 88.5
+//     7,552         59.9 / 60.3      14,436         97.9 / 94.9
+// and compounds sharing two meshes: 4,800 chunks 46.9 / 48.2, 12,000 66.8 / 67.4,
+// 28,800 125.2 / 124.0, 72,000 265 / 259.  From 8 faces per lane on: with fewer
+// a chunk is its fixed work more than its rows.  On two layers, whose depths
+// outweigh the rows, one pass is never the slower by more than a run's spread
+// (4,842 chunks 55.1 / 59.0, 9,108 86.0 / 90.8, 14,436 121.1 / 120.7, 72,000
+// compounds' 324 / 326).
+static constexpr uint32_t kSplitChunks = 12288;
 
 static bool two_pass(const sfh_batch_t* b) { return b->K >= 8 && b->nchunks > kSplitChunks; }
 
@@ -3315,7 +3320,7 @@ static int launch_faces(sfh_batch_t* b, const OceanK& oc, hipStream_t s)
                        b->d_dyn, oc, b->d_partials)
 #define LAUNCH_F(KK, NU, NL, PASS)                                                                              \
     {                                                                                                           \
-        constexpr bool sp = NL > 0 && !NU && (PASS & kPassCross) && KK >= 8;                                    \
+        constexpr bool sp = NL == 1 && !NU && (PASS & kPassCross) && KK >= 8;                                   \
         if (sp && two_pass(b)) {                                                                                \
             if (b->recs) LAUNCH_R(KK, NU, NL, PASS, true, sp); else LAUNCH_R(KK, NU, NL, PASS, false, sp);      \
         } else {                                                                                                \

@@ -2,7 +2,7 @@
 a number, and so has its body's skin friction (and, crossing, its wetted area),
 on every path to a whole face: the face is never left out of a finite row.
 Submerged and crossing bodies, the one-launch step, the face launch with records
-and, past 4,608 chunks on waves, its two passes over a crossing chunk."""
+and, past 12,288 chunks on waves, its two passes over a crossing chunk."""
 import numpy as np
 import pytest
 
@@ -30,7 +30,7 @@ def _states(n, z):
     return st
 
 
-@pytest.mark.parametrize("bodies,waves,split", [(3, False, 0), (3, False, 1), (3, True, 0), (3, True, 1), (4700, True, 0)])
+@pytest.mark.parametrize("bodies,waves,split", [(3, False, 0), (3, False, 1), (3, True, 0), (3, True, 1), (12400, True, 0)])
 def test_overflowing_face_is_not_left_out(gpu, bodies, waves, split):
     print(f"case: overflowing face, {bodies} bodies, waves {waves}, split_passes {split}", flush=True)
     mesh, ocn = _mesh(), H.Ocean()

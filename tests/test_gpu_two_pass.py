@@ -1,7 +1,7 @@
 """Large batches on waves, where the face launch takes a crossing chunk's rows
-twice (more than 4,608 chunks, 8 faces per lane or more, one or two layers): from
-face records, and from packed faces and vertices where the batch's distinct
-meshes hold more than two million faces.  Meshes of one face, of a row of 64, of
+twice (more than 12,288 chunks, 8 faces per lane or more, one layer; on two layers
+once): from face records, and from packed faces and vertices where the batch's
+distinct meshes hold more than two million faces.  Meshes of one face, of a row of 64, of
 a chunk with one face more or less, and shuffled ones, whose vertex windows are
 too large to stage.  Every body's row is held to the FP64 oracle with the error
 statement of tests/util.py, and does not depend on the launch's shape."""
@@ -20,8 +20,8 @@ from util import NAMES, RTOL, STOL, bound_ratio
 pytestmark = pytest.mark.gpu
 
 SIZES = (1, 63, 64, 65, 511, 513, 1023, 1025, 2047, 2049, 4096 + 65)
-COPIES = 400   # 5,600 chunks at 32 faces per lane
-CHUNKS, RADIUS = 4608, 1.1
+COPIES = 900   # 12,600 chunks at 32 faces per lane
+CHUNKS, RADIUS = 12288, 1.1
 
 
 def _tris(shuffle):
