@@ -203,11 +203,12 @@ typedef struct {
     uint32_t split_passes;    /* 0: one face launch runs the submerged and the crossing
                                  chunks; 1: a launch for each, each at its own occupancy */
 } sfh_batch_opts;
-/* With split_passes 0 a batch of at most 1,024 chunks (of bodies that all have
- * faces, 8 or 16 faces per lane, not compounds) runs its whole step in one
- * launch, a workgroup per chunk; `waves` then has no effect, and both times of
- * sfh_batch_kernel_ms are that launch's.  The rows are the same bits either
- * way. */
+/* With split_passes 0 a step of a batch of at most 1,024 chunks (of bodies that
+ * all have faces, 8 or 16 faces per lane, not compounds) runs in one launch, a
+ * workgroup per chunk.  At 16 faces per lane it does so up to 512 chunks on a
+ * flat sea (900 with a mask, 1,024 from host buffers) and up to 2,048 in the air
+ * without a varying wind.  `waves` then has no effect, and both times of
+ * sfh_batch_kernel_ms are that launch's.  The rows are the same bits either way. */
 
 /* Replaces the per-body pool fan-out of SimulationManager::SimulationTickCallback
  * (SimulationManager.cpp:1619-1655) + Ocean::ApplyFluidForces (Ocean.cpp:219-268)

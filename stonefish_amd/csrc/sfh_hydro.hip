@@ -3357,27 +3357,41 @@ static int launch_faces(sfh_batch_t* b, const OceanK& oc, hipStream_t s)
     return SFH_OK;
 }
 
-// Whether a step runs as one launch of k_step (a workgroup per chunk): up to
-// 1,024 chunks of a batch that asks for one face launch (split_passes 0) and
-// whose bodies all have faces (k_step's workgroups are chunks), with the faces
-// per lane it is built for.  Two of its workgroups fit a CU beside each other
-// (65 KB of LDS at 16 faces per lane), so past 512 working chunks they come in
-// rounds of about 11 us, where the general path's face launch still has every
-// chunk in flight; the two cross between 850 and 1,130 chunks.  Measured, a
-// tick of bodies of 2.8 chunks on average, 16 faces per lane, general path
-// against one launch:
-//     chunks         flat sea        one wave layer   two layers
-//       279        29.7 / 17.4 us    33.9 / 17.2 us   39.2 / 18.9 us
-//       850        30.4 / 29.0       35.1 / 29.0      40.4 / 31.6
-//     1,129        30.4 / 35.8       34.4 / 35.5      40.4 / 39.1
-//     1,700        31.0 / 51.0       36.7 / 50.5      45.1 / 54.4
-// and with a mask leaving 30 % of the bodies, 28-39 / 17-20 us up to 1,129
-// chunks.  Aerodynamic batches: 850 chunks 16.8 / 11.8 us, 1,413 17.6 / 18.2.
-static constexpr uint32_t kStepChunks = 1024;
+// Whether a step runs as one launch of k_step (a workgroup per chunk): a batch
+// that asks for one face launch (split_passes 0) and whose bodies all have faces
+// (k_step's workgroups are chunks), with the faces per lane it is built for, of
+// up to 1,024 chunks.  At 16 faces per lane two of its workgroups fit a CU beside
+// each other (65 KB of LDS; in the air four), so past 512 working chunks they
+// come in rounds of about 11 us, where the general path's face launch still has
+// every chunk in flight.  What the rounds cost depends on the general path: least
+// on waves, most on a flat sea, where steps that leave no body out take the
+// general path past 512 chunks and masked ones past 900 (steps on host buffers,
+// whose general path has copies besides, 1,024: 577 chunks 56.4 / 41.4, 817 57.3 /
+// 48.1); in the air, without a varying wind, the one launch is the faster up to
+// 2,048.  Measured at 16 faces per lane, general path / one launch (us a step):
+//                          512 chunks     700       850       1,024
+//     flat, one-chunk hulls 24.6 / 14.8  24.5/25.6 24.5/26.7  24.4 / 27.2
+//     flat, three chunks    26.1 / 17.8  26.3/29.1 26.3/31.1  26.3 / 33.0
+//     flat tick, all bodies 29.4 / 23.5  29.9/27.4 30.0/28.4  30.3 / 32.6
+//     flat tick, 40 %       28.0 / 16.8  28.1/17.0 28.1/18.6  28.6 / 21.2
+//     one layer tick, all   34.3 / 23.5  34.8/26.7 35.1/28.4  35.4 / 32.1
+//     two layers tick, all  37.3 / 25.5  38.3/29.3 38.6/31.7  38.8 / 35.7
+// (the ticks at 563, 707, 850 and 1,020 chunks), and in the air 1,190 chunks 17.9 /
+// 14.3, 2,040 19.2 / 18.0, 2,263 20.0 / 20.0.  At 8 faces per lane, four to a CU,
+// one launch is the faster up to 1,024 everywhere (flat, 1,024 chunks: 20.2 / 12.8).
+static constexpr uint32_t kStepChunks = 1024, kStepChunksFlat = 512, kStepChunksFlatMasked = 900, kStepChunksAir = 2048;
 
-static bool step_fused(const sfh_batch_t* b)
+enum class Step { whole, masked, host };
+
+static bool step_fused(const sfh_batch_t* b, const OceanK& oc, Step kind)
 {
-    return !b->compound && !b->split && b->all_faces && (b->K == 8 || b->K == 16) && b->nchunks <= kStepChunks;
+    if (b->compound || b->split || !b->all_faces || (b->K != 8 && b->K != 16)) return false;
+    uint32_t most = kStepChunks;
+    if (b->K == 16 && oc.ncur == 0) {
+        if (b->aero) most = kStepChunksAir;
+        else if (oc.nlayers == 0 && kind != Step::host) most = kind == Step::masked ? kStepChunksFlatMasked : kStepChunksFlat;
+    }
+    return b->nchunks <= most;
 }
 
 static void launch_step(sfh_batch_t* b, const OceanK& oc, const StepArgs& a, hipStream_t s)
@@ -3404,7 +3418,7 @@ static void launch_step(sfh_batch_t* b, const OceanK& oc, const StepArgs& a, hip
 // applied (optional): the tick driver's force and torque per row, which only
 // the one-launch step writes (step_fused says whether it does).
 static int batch_launch(sfh_batch_t* b, const sfh_ocean_t* o, const double* d_states, double* d_out, hipStream_t s,
-                        bool timed, const uint8_t* active = nullptr, double* applied = nullptr)
+                        bool timed, const uint8_t* active = nullptr, double* applied = nullptr, Step kind = Step::whole)
 {
     if (b->n == 0) return SFH_OK;
     // every launch of the step runs or none does: the epilogue zeroes the
@@ -3412,7 +3426,7 @@ static int batch_launch(sfh_batch_t* b, const sfh_ocean_t* o, const double* d_st
     if (b->K != 1 && b->K != 2 && b->K != 4 && b->K != 8 && b->K != 16 && b->K != 32)
         return fail(SFH_ERR_INVALID, "bad K");
     OceanK oc = make_oceank(o);
-    if (step_fused(b)) {
+    if (step_fused(b, oc, active ? Step::masked : kind)) {
         StepArgs a;
         a.st = b->d_static;
         a.chunks = b->d_chunks;
@@ -3658,7 +3672,7 @@ extern "C" int sfh_tick_step(sfh_tick t, sfh_ocean fluid, const double* d_states
         rc = batch_launch(b, fluid, d_states, d_out, s, b->timing, d_overlap, d_applied);
         if (rc != SFH_OK) return rc;
         if (b->timing) b->ev_pending = true;
-        applied = b->n > 0 && step_fused(b);
+        applied = b->n > 0 && step_fused(b, make_oceank(fluid), d_overlap ? Step::masked : Step::whole);
     }
     if (n && !applied) hipLaunchKernelGGL(k_tick_apply, dim3((n + 127) / 128), dim3(128), 0, s, d_out, d_overlap, n,
                               t->batch->aero ? 1 : 0, d_applied);
@@ -3688,9 +3702,11 @@ static constexpr size_t kHostStaged = 16u << 20;   // bytes of states and rows
 extern "C" int sfh_batch_compute_host(sfh_batch b, sfh_ocean o, const double* states, double* out)
 {
     if (!b || !states || !out) return fail(SFH_ERR_INVALID, "null argument");
+    const int bad = check_ocean(o);
+    if (bad != SFH_OK) return bad;
     const size_t ns = (size_t)b->nunits * SFH_STATE_DOUBLES, no = (size_t)b->nunits * SFH_OUT_DOUBLES;
     const size_t bytes = sizeof(double) * std::max<size_t>(1, ns + no);
-    const bool direct = step_fused(b), staged = direct || bytes <= kHostStaged;
+    const bool direct = step_fused(b, make_oceank(o), Step::host), staged = direct || bytes <= kHostStaged;
     if (staged && !b->h_io && hipHostMalloc((void**)&b->h_io, bytes, hipHostMallocDefault) != hipSuccess) {
         b->h_io = nullptr;
         return fail(SFH_ERR_HIP, "pinned staging of %zu bytes failed", bytes);
@@ -3710,7 +3726,9 @@ extern "C" int sfh_batch_compute_host(sfh_batch b, sfh_ocean o, const double* st
         if (e == hipSuccess) e = hipMemcpy(io + ns, out, sizeof(double) * no, hipMemcpyHostToDevice);
     }
     if (e == hipSuccess) {
-        const int rc = sfh_batch_compute(b, o, io, io + ns, nullptr);
+        if (b->timing) harvest_timing(b);
+        const int rc = batch_launch(b, o, io, io + ns, nullptr, b->timing, nullptr, nullptr, Step::host);
+        if (rc == SFH_OK && b->timing) b->ev_pending = true;
         if (rc != SFH_OK) {
             hipStreamSynchronize(nullptr);   // the staging is free again
             return rc;
