@@ -1109,15 +1109,15 @@ __device__ __forceinline__ void wet_contrib(const Wet& wt, const FaceBody& fb, c
 // together afterwards, 64 at a time, so the clip code runs once per 64 of them.
 // Tetra volumes, pressure buoyancy with waves, drag.
 //
-// SPLIT (large batches on one wave layer, kSplitChunks): the rows are taken twice, first
-// which of their faces are all wet (a mask of the row, kept in lane `row` of a
-// register pair) and which are cut, from the packed vertex numbers and the
-// depths alone; then the all-wet faces of the rows that have any, from the face
-// records (REC) or from the vertices, so that dry rows load nothing and neither
-// pass holds the other's registers.  A chunk whose window is wholly wet needs no
-// first pass.  On a flat sea, where the volume takes the vertices of every wet
-// face, one pass is the faster (4,096 states of a hull of 5,112 faces: 87 us a
-// step, 104 in two passes).
+// SPLIT (large batches on one wave layer whose chunks all have a window,
+// two_pass): the rows are taken twice, first which of their faces are all wet (a
+// mask of the row, kept in lane `row` of a register pair) and which are cut, from
+// the packed vertex numbers and the depths alone; then the all-wet faces of the
+// rows that have any, from records of them (REC, k_cross_records) or from the
+// vertices, so that dry rows load nothing and neither pass holds the other's
+// registers.  A chunk whose window is wholly wet needs no first pass.  On a flat
+// sea, where the volume takes the vertices of every wet face, one pass is the
+// faster (4,096 states of a hull of 5,112 faces: 87 us a step, 104 in two passes).
 template <int K, bool NU, int NL, bool WIN, bool REC, bool SPLIT>
 __device__ __forceinline__ void cross_chunk(uint32_t c, uint32_t f0, uint32_t nfc, uint32_t vlo, uint32_t vn,
                                             const BodyStatic& S, const BodyDyn& D, const OceanK& oc,
@@ -1141,7 +1141,7 @@ __device__ __forceinline__ void cross_chunk(uint32_t c, uint32_t f0, uint32_t nf
     // lane k holds block k's lowest vertex id; like the first row's numbers it
     // is requested before the window's vertices, whose work covers it
     const uint32_t low = SPLIT ? gptr((const uint32_t*)S.blkwin)[2 * (f0 / 64 + min(lane, rows - 1))] : 0u;
-    uint32_t w = SPLIT && WIN ? load_at(pidx, min((uint32_t)lane, flast)) : 0u;
+    uint32_t w = SPLIT ? load_at(pidx, min((uint32_t)lane, flast)) : 0u;
     bool whole = false;   // every vertex of the window is wet
     if (WIN) {
         // four vertices per lane in flight: their loads, then their texel
@@ -1226,19 +1226,11 @@ __device__ __forceinline__ void cross_chunk(uint32_t c, uint32_t f0, uint32_t nf
                     ncut += (uint32_t)__popcll(cut);
                 }
             };
-            if (WIN) {
-                for (int j = 0; j < rows; ++j) {
-                    const float* at = ldep + ((uint32_t)__builtin_amdgcn_readlane((int)low, j) - vlo);
-                    const float d0 = at[unpack_id(w, 0)], d1 = at[unpack_id(w, 1)], d2 = at[unpack_id(w, 2)];
-                    w = load_at(pidx, min(64u * (j + 1) + lane, flast));
-                    classify(j, d0, d1, d2);
-                }
-            } else {
-                for (int j = 0; j < rows; ++j) {
-                    const uint32_t f = min(64u * j + lane, flast);
-                    const uint32_t a0 = faces[3 * f], a1 = faces[3 * f + 1], a2 = faces[3 * f + 2];
-                    classify(j, dep(a0, vert(verts, a0)), dep(a1, vert(verts, a1)), dep(a2, vert(verts, a2)));
-                }
+            for (int j = 0; j < rows; ++j) {
+                const float* at = ldep + ((uint32_t)__builtin_amdgcn_readlane((int)low, j) - vlo);
+                const float d0 = at[unpack_id(w, 0)], d1 = at[unpack_id(w, 1)], d2 = at[unpack_id(w, 2)];
+                w = load_at(pidx, min(64u * (j + 1) + lane, flast));
+                classify(j, d0, d1, d2);
             }
             wave_lds_sync();
         } else if (lane == rows - 1) {
@@ -1289,29 +1281,15 @@ __device__ __forceinline__ void cross_chunk(uint32_t c, uint32_t f0, uint32_t nf
             } else {
                 // row j is computed, row jn's vertices and the row after's numbers
                 // are in flight
-                struct Ids { uint32_t a, b, c; };
-                auto numbers = [&](int row) {
-                    const uint32_t f = min(64u * row + lane, flast);
-                    Ids n = {0, 0, 0};
-                    if (WIN) {
-                        n.a = load_at(pidx, f);
-                    } else {
-                        n.a = faces[3 * f]; n.b = faces[3 * f + 1]; n.c = faces[3 * f + 2];
-                    }
-                    return n;
+                auto numbers = [&](int row) { return load_at(pidx, min(64u * row + lane, flast)); };
+                auto points = [&](int row, uint32_t n, f3& p1, f3& p2, f3& p3) {
+                    const SFH_GLOBAL float* vb = verts + 3 * (size_t)__builtin_amdgcn_readlane((int)low, row);
+                    p1 = vert_at(vb, unpack_id(n, 0));
+                    p2 = vert_at(vb, unpack_id(n, 1));
+                    p3 = vert_at(vb, unpack_id(n, 2));
                 };
-                auto points = [&](int row, Ids n, f3& p1, f3& p2, f3& p3) {
-                    if (WIN) {
-                        const SFH_GLOBAL float* vb = verts + 3 * (size_t)__builtin_amdgcn_readlane((int)low, row);
-                        p1 = vert_at(vb, unpack_id(n.a, 0));
-                        p2 = vert_at(vb, unpack_id(n.a, 1));
-                        p3 = vert_at(vb, unpack_id(n.a, 2));
-                    } else {
-                        p1 = vert(verts, n.a); p2 = vert(verts, n.b); p3 = vert(verts, n.c);
-                    }
-                };
-                const Ids nj = numbers(j);
-                Ids nn = numbers(jn);
+                const uint32_t nj = numbers(j);
+                uint32_t nn = numbers(jn);
                 f3 p1, p2, p3;
                 points(j, nj, p1, p2, p3);
                 for (;;) {
@@ -1793,10 +1771,10 @@ __global__ __launch_bounds__(64 * kFaceWaves, face_occupancy(K, NU, NL, PASS)) v
             const uint32_t vn = __builtin_amdgcn_readfirstlane(ch.vn);
             WaveQ<NL> wq;
             wq.load(D, oc);
-            if (vn > 0 && vn <= win_cap(K))
+            if (SPLIT || (vn > 0 && vn <= win_cap(K)))
                 cross_chunk<K, NU, NL, true, REC, SPLIT>(c, f0, nfc, vlo, vn, S, D, oc, wq, ldep[wl], cutq[wl], partials, lane);
             else
-                cross_chunk<K, NU, NL, false, REC, SPLIT>(c, f0, nfc, vlo, vn, S, D, oc, wq, ldep[wl], cutq[wl], partials, lane);
+                cross_chunk<K, NU, NL, false, REC, false>(c, f0, nfc, vlo, vn, S, D, oc, wq, ldep[wl], cutq[wl], partials, lane);
         }
     }
 }
@@ -2502,6 +2480,7 @@ struct sfh_batch_t {
     float4* d_xrecs = nullptr;      // records of the meshes' crossing faces, for steps that read them
     uint32_t* d_done = nullptr;     // per body: chunks k_step finished in this step (zero between steps)
     bool all_faces = false;         // every body has at least one chunk
+    bool all_windows = false;       // every chunk has a vertex window
     bool recs = true;               // the face launch reads the meshes' face records, else their packed faces
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
@@ -2876,7 +2855,10 @@ static constexpr uint64_t kRecordFaces = 2000000;
 // compounds' 324 / 326).
 static constexpr uint32_t kSplitChunks = 12288;
 
-static bool two_pass(const sfh_batch_t* b) { return b->K >= 8 && b->nchunks > kSplitChunks; }
+// A chunk without a window takes its depths from the vertices, which the second
+// pass would load again: such batches take one pass (3,000 shuffled hulls of 5,000
+// faces 176 us a step, 201 in two passes).
+static bool two_pass(const sfh_batch_t* b) { return b->K >= 8 && b->all_windows && b->nchunks > kSplitChunks; }
 
 // (Re)builds the chunks: every body's faces cut into chunks of 64*K
 // consecutive faces, each with its vertex window.
@@ -2884,7 +2866,7 @@ static int batch_build_chunks(sfh_batch_t* b)
 {
     std::vector<Chunk> chunks;
     const uint32_t csize = 64u * b->K;
-    b->all_faces = true;
+    b->all_faces = b->all_windows = true;
     for (uint32_t i = 0; i < b->n; ++i) {
         BodyStatic& s = b->h_static[i];
         b->all_faces = b->all_faces && s.nf > 0;
@@ -2899,6 +2881,7 @@ static int batch_build_chunks(sfh_batch_t* b)
             ch.first = c * csize;
             ch.count = std::min(csize, s.nf - c * csize);
             if (m) chunk_window(m->blkwin, ch.first, ch.count, win_cap(b->K), ch.vlo, ch.vn);
+            b->all_windows = b->all_windows && ch.vn > 0;
             chunks.push_back(ch);
         }
     }

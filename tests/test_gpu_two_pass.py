@@ -3,7 +3,7 @@ twice (more than 12,288 chunks, 8 faces per lane or more, one layer; on two laye
 once): from face records, and from packed faces and vertices where the batch's
 distinct meshes hold more than two million faces.  Meshes of one face, of a row of 64, of
 a chunk with one face more or less, and shuffled ones, whose vertex windows are
-too large to stage.  Every body's row is held to the FP64 oracle with the error
+too large to stage and whose batches take the rows once.  Every body's row is held to the FP64 oracle with the error
 statement of tests/util.py, and does not depend on the launch's shape."""
 from functools import lru_cache
 
