@@ -52,7 +52,8 @@ int sfh_init(int device);
  * vertex_pos points at Vertex::pos of vertex 0; vertex_stride is the byte
  * distance between vertices: sizeof(Vertex) = 24, sizeof(TexturableVertex) =
  * 44, or 12 for packed xyz.  face_ids holds Face::vertexID, 3 per face.  The
- * device copy is packed: 12 B per vertex, 12 B per face. */
+ * device copy is packed: 12 B per vertex, 12 B per face, and 36 B per face of
+ * records and vertex numbers formed from them. */
 int sfh_mesh_create(const void* vertex_pos, size_t vertex_stride, uint32_t nv,
                     const uint32_t* face_ids, uint32_t nf, sfh_mesh* out);
 int sfh_mesh_destroy(sfh_mesh mesh);

@@ -1809,8 +1809,8 @@ __global__ __launch_bounds__(64 * kFaceWaves, face_occupancy(K, NU, NL, PASS)) v
 //      The counter has wrapped to zero for the next step.
 // Measured: a tick of 203 bodies (576 chunks, 60 % overlapped, two wave
 // layers) 39.4 -> 17.9 us, an aerodynamic batch of 300 bodies 16.5 -> 9.4 us,
-// the per-body calls 38 -> 32 us (2,070 faces, submerged) and 52 -> 43 us
-// (12,000 faces, surface), 13 us of which are the caller's Python.  Of the
+// the per-body calls 38 -> 23 us (2,070 faces, submerged) and 52 -> 29 us
+// (12,000 faces, surface), their rows through pinned memory.  Of the
 // tick's kernel 1.0 us are its loads, 2.9 the prologue, 4.3 the depths and the
 // wet faces' terms, 2.9 the sums and up to 2 the cut faces, 2.2 the partials'
 // way through memory, 1.5 the finish: chains of dependent loads and FP64
