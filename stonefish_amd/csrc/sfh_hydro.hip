@@ -2910,8 +2910,12 @@ static int batch_build_chunks(sfh_batch_t* b)
     }
     b->recs = !packed || faces <= kRecordFaces;
     for (BodyStatic& s : b->h_static) s.xrecs = nullptr;
-    if (b->recs && two_pass(b)) {
-        HIPCHK(hipMalloc(&b->d_xrecs, kCrossRecBytes * (faces + 4 * used.size())));
+    if (b->recs && two_pass(b) && hipMalloc(&b->d_xrecs, kCrossRecBytes * (faces + 4 * used.size())) != hipSuccess) {
+        (void)hipGetLastError();
+        b->d_xrecs = nullptr;
+        b->recs = false;   // meshes whose chunks all have a window are packed
+    }
+    if (b->d_xrecs) {
         std::vector<float4*> at(used.size());
         size_t next = 0;   // in float4: each mesh's block starts at a multiple of 16 bytes
         for (size_t i = 0; i < used.size(); ++i) {
