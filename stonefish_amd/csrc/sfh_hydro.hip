@@ -3693,10 +3693,11 @@ extern "C" int sfh_batch_compute_host(sfh_batch b, sfh_ocean o, const double* st
     if (bad != SFH_OK) return bad;
     const size_t ns = (size_t)b->nunits * SFH_STATE_DOUBLES, no = (size_t)b->nunits * SFH_OUT_DOUBLES;
     const size_t bytes = sizeof(double) * std::max<size_t>(1, ns + no);
-    const bool direct = step_fused(b, make_oceank(o), Step::host), staged = direct || bytes <= kHostStaged;
+    bool direct = step_fused(b, make_oceank(o), Step::host), staged = direct || bytes <= kHostStaged;
     if (staged && !b->h_io && hipHostMalloc((void**)&b->h_io, bytes, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
         b->h_io = nullptr;
-        return fail(SFH_ERR_HIP, "pinned staging of %zu bytes failed", bytes);
+        direct = staged = false;   // no pinned memory left: the buffers are copied as they are
     }
     if (!direct && !b->d_io && hipMalloc(&b->d_io, bytes) != hipSuccess) {
         b->d_io = nullptr;
