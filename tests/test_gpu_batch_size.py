@@ -2,11 +2,13 @@
 layer a batch of more than 12,288 chunks takes a crossing chunk's rows twice, from
 records of its faces; a smaller one takes them once, from the vertices.  The
 records hold what the vertices give, so all slots of the rows, the submerged
-volume among them, are the same bits.  Hulls of fine and of coarse faces and a
+volume among them, are the same bits.  So are those of a masked step of the large
+batch, which takes the rows once.  Hulls of fine and of coarse faces and a
 revolved one with slivers at its pole, at every number of faces per lane that has
 both ways."""
 import numpy as np
 import pytest
+import torch
 
 from stonefish_amd import hydro as H
 from stonefish_amd import meshes as M
@@ -44,3 +46,13 @@ def test_rows_do_not_depend_on_the_batch(gpu, K, layers):
     assert (a[:, 21] == 2).sum() > few // 2 and (a[:, 19] > 0).sum() > few // 2
     for name, sl in {**H.OUT_FIELDS, "position": 21}.items():
         assert np.array_equal(a[:, sl], b[:, sl]), (name, np.abs(a[:, sl] - b[:, sl]).max())
+    d_st = torch.from_numpy(st).cuda()
+    mask = torch.zeros(many, dtype=torch.uint8, device="cuda")
+    mask[:few:2] = 1
+    out = torch.full((many, 24), 0.375, dtype=torch.float64, device="cuda")
+    large.compute_masked(go, d_st.data_ptr(), mask.data_ptr(), out.data_ptr())
+    torch.cuda.synchronize()
+    out = out.cpu().numpy()
+    written = b[::2, :20] != 0.0   # slots the step leaves untouched keep the fill there, zero in b
+    assert np.array_equal(out[:few:2, :20][written], b[::2, :20][written])
+    assert np.array_equal(out[:few:2, 20:22], b[::2, 20:22]) and (out[1:few:2] == 0.375).all()
